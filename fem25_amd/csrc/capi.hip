@@ -14,6 +14,7 @@
 
 #include "f25_internal.h"
 #include "kernels.hip"
+#include "affine.hip"
 
 using namespace f25;
 using namespace f25k;
@@ -98,6 +99,14 @@ struct f25_mesh_s {
     double *d_xl = nullptr, *d_zl = nullptr, *d_xd = nullptr, *d_zd = nullptr;
     double *d_shl = nullptr, *d_wq = nullptr, *d_xq = nullptr;
     double *d_t1d = nullptr;    // 1-D tables: val1 (nl*nq1) then der1
+    // parallelogram elements (affine.hip): 1-D table, element records of the
+    // model, a zero value, and the elements (ascending) that run there (with
+    // the PML elements) or at the general quadrature points
+    double *d_taf = nullptr, *d_rec = nullptr;
+    std::vector<char> affine;
+    bool rect = true;   // the parallelograms' sides all lie along x and z
+    int *d_aelem = nullptr, *d_gelem = nullptr;
+    int naff = 0, ngen = 0;
     char *d_cdom = nullptr, *d_cnp = nullptr;
     double *d_rho = nullptr, *d_lam = nullptr, *d_mu = nullptr;
     double *d_blk = nullptr;
@@ -213,6 +222,30 @@ static int check_err(f25_mesh *m) {
     return 0;
 }
 
+// Elements the kernels of affine.hip take: those whose bilinear map is affine
+// in FP64 (x1 - x2 + x3 - x4 zero to the rounding of the differences, as on
+// any structured rectangular or sheared mesh: the twist then changes the
+// Jacobian by less than its own rounding) with det J > 0 as geo_at requires;
+// and the PML elements, which those kernels skip as the others do.  Anything
+// else keeps the reference's quadrature.
+static bool is_affine(const f25_mesh *m, int e) {
+    double x[4], z[4];
+    for (int k = 0; k < 4; ++k) {
+        x[k] = m->xl[m->ieng[4 * e + k] - 1];
+        z[k] = m->zl[m->ieng[4 * e + k] - 1];
+    }
+    double h = 0.0;
+    for (int k = 0; k < 4; ++k) {
+        const int n = (k + 1) % 4;
+        h = std::max(h, std::max(std::fabs(x[n] - x[k]), std::fabs(z[n] - z[k])));
+    }
+    const double bx = (x[0] - x[1]) + (x[2] - x[3]), bz = (z[0] - z[1]) + (z[2] - z[3]);
+    const double tol = 4e-16 * h;
+    const double det = 0.0625 * (((x[1] - x[0]) + (x[2] - x[3])) * ((z[3] - z[0]) + (z[2] - z[1])) -
+                                 ((x[3] - x[0]) + (x[2] - x[1])) * ((z[1] - z[0]) + (z[2] - z[3])));
+    return std::fabs(bx) <= tol && std::fabs(bz) <= tol && det > 2.22e-16;
+}
+
 static int upload_mesh(f25_mesh *m) {
     const f25_mesh_desc &d = m->d;
     hipStream_t s = m->st;
@@ -277,7 +310,25 @@ static int upload_mesh(f25_mesh *m) {
             for (int k = 0; k < 4; ++k) m->fixa[m->ieng[4 * e + k] - 1] = 1;
     TRY(upload(&m->d_fixa, m->fixa.data(), m->fixa.size(), s));
     TRY(dalloc(&m->d_part, (size_t)d.nelem * 12));
-    (void)nen;
+    // elements by kind of quadrature
+    m->affine.assign(d.nelem, 0);
+    std::vector<int> ael, gel;
+    for (int e = 0; e < d.nelem; ++e) {
+        m->affine[e] = m->cdom[e] == 'A' || is_affine(m, e);
+        (m->affine[e] ? ael : gel).push_back(e);
+        if (!m->affine[e] || m->cdom[e] == 'A') continue;
+        const int *a = &m->ieng[4 * e];
+        auto same = [](const std::vector<double> &v, int p, int q) { return v[p - 1] == v[q - 1]; };
+        m->rect = m->rect && same(m->xl, a[0], a[3]) && same(m->xl, a[1], a[2]) && same(m->zl, a[0], a[1]) &&
+                  same(m->zl, a[2], a[3]);
+    }
+    m->naff = (int)ael.size();
+    m->ngen = (int)gel.size();
+    TRY(upload(&m->d_aelem, ael.data(), ael.size(), s));
+    TRY(upload(&m->d_gelem, gel.data(), gel.size(), s));
+    const std::vector<double> taf = af_table(m->tab);
+    TRY(upload(&m->d_taf, taf.data(), taf.size(), s));
+    TRY(dalloc(&m->d_rec, (size_t)d.nelem * AFR));
     HIPCHK(hipStreamSynchronize(s));
     return 0;
 }
@@ -451,6 +502,7 @@ extern "C" int f25_mesh_destroy(f25_mesh *m) {
     if (m->st) (void)hipStreamSynchronize(m->st);
     dfree(m->d_ieng); dfree(m->d_lm); dfree(m->d_first); dfree(m->d_order); dfree(m->d_pml_order); dfree(m->d_err);
     dfree(m->d_xl); dfree(m->d_zl); dfree(m->d_xd); dfree(m->d_zd); dfree(m->d_shl); dfree(m->d_wq); dfree(m->d_t1d);
+    dfree(m->d_taf); dfree(m->d_rec); dfree(m->d_aelem); dfree(m->d_gelem);
     dfree(m->d_xq); dfree(m->d_cdom); dfree(m->d_cnp); dfree(m->d_rho); dfree(m->d_lam); dfree(m->d_mu);
     if (m->ag.exec) (void)hipGraphExecDestroy(m->ag.exec);
     dfree(m->d_vcf); dfree(m->d_dvcf); dfree(m->d_vpad);
@@ -578,6 +630,8 @@ extern "C" int f25_set_model(f25_mesh *m, const double *dens, const double *ecoe
         TRY(dalloc(&m->d_blk_hi, nb));
         TRY(dalloc(&m->d_blk_lo, nb));
     }
+    hipLaunchKernelGGL(k_aff_rec, dim3((m->d.nelem + 255) / 256), dim3(256), 0, m->st, m->d.nelem, m->d_ieng, m->d_xl,
+                       m->d_zl, m->d_rho, m->d_lam, m->d_mu, m->d_cdom, m->d_rec);
     TRY(run_blocks(m, m->d_rho, m->d_lam, m->d_mu, m->d_blk, m->d_blk32, m->d_blk_hi, m->d_blk_lo));
     TRY(vcoef(m, m->d_blk, &m->d_vcf));
     m->have_model = true;
@@ -1570,12 +1624,13 @@ static int grad_threads(int nl) {
     }
 }
 
+// elements at the general quadrature points: elems (n of them), null: all
 template <typename R>
-static int grad_launch(f25_mesh *m, int ntrip, const double *d_om, const double *d_ky, const void *u, const void *l) {
+static int grad_general(f25_mesh *m, const int *elems, int n, int ntrip, const double *d_om, const double *d_ky, const void *u, const void *l) {
     typedef typename CxOf<R>::T C2;
     const int nen = m->tab.nen;
     // every order up to p6 runs the sum-factorised kernel
-    typedef void (*GradSf)(const double *, const double *, const double *, const int *, const double *,
+    typedef void (*GradSf)(const int *, const double *, const double *, const double *, const int *, const double *,
                            const double *, const char *, const int *, int, int64_t, const double *,
                            const double *, const C2 *, const C2 *, double *, int *);
     // trips per pass (GradOcc::T): with two, four workgroups fit per CU at
@@ -1600,18 +1655,50 @@ static int grad_launch(f25_mesh *m, int ntrip, const double *d_om, const double 
                        (grad_ppl<R>(nl) == 2 ? (size_t)2 * nl * q1 * sizeof(double) : 0);
     if (lsf > 64 * 1024)
         HIPCHK(hipFuncSetAttribute((const void *)ksf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lsf));
-    HIPCHK(hipEventRecord(m->ev0, m->st));
-    hipLaunchKernelGGL(ksf, dim3(m->d.nelem), dim3(grad_threads<R>(nl)), lsf, m->st, m->d_t1d, m->d_wq,
+    hipLaunchKernelGGL(ksf, dim3(n), dim3(grad_threads<R>(nl)), lsf, m->st, elems, m->d_t1d, m->d_wq,
                        m->d_xq, m->d_ieng, m->d_xl, m->d_zl, m->d_cdom, m->d_lm, ntrip, (int64_t)m->g.ndof,
                        d_om, d_ky, (const C2 *)u, (const C2 *)l, m->d_part, m->d_err);
+    return 0;
+}
+
+// parallelogram elements: waves of a workgroup by the chunks of triples
+template <int NL>
+static int grad_affine(f25_mesh *m, int ntrip, const double *d_om, const double *d_ky, const double2 *u,
+                       const double2 *l) {
+    typedef AfShape<NL> S;
+    auto kern = m->rect ? k_grad_af<NL, true> : k_grad_af<NL, false>;
+    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_grad));
+    const int nw = std::min(S::NW, (ntrip + S::PW - 1) / S::PW);
+    hipLaunchKernelGGL(kern, dim3(m->naff), dim3(64 * nw), S::lds_grad, m->st, m->d_aelem, m->d_rec, m->d_taf, m->d_lm,
+                       ntrip, (int64_t)m->g.ndof, d_om, d_ky, u, l, m->d_part);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+// The FP64 gradient takes its parallelograms through affine.hip.  The FP32
+// one keeps the general points and its FP32 arithmetic for every element:
+// its results are its rounding, which another arithmetic would change.
+static int grad_launch(f25_mesh *m, int ntrip, const double *d_om, const double *d_ky, const void *u, const void *l,
+                       bool fp32) {
+    HIPCHK(hipEventRecord(m->ev0, m->st));
+    if (fp32) return grad_general<float>(m, nullptr, m->d.nelem, ntrip, d_om, d_ky, u, l);
+    const double2 *ud = (const double2 *)u, *ld = (const double2 *)l;
+    if (m->naff) switch (m->tab.nl) {
+        case 3: TRY(grad_affine<3>(m, ntrip, d_om, d_ky, ud, ld)); break;
+        case 4: TRY(grad_affine<4>(m, ntrip, d_om, d_ky, ud, ld)); break;
+        case 5: TRY(grad_affine<5>(m, ntrip, d_om, d_ky, ud, ld)); break;
+        case 6: TRY(grad_affine<6>(m, ntrip, d_om, d_ky, ud, ld)); break;
+        case 7: TRY(grad_affine<7>(m, ntrip, d_om, d_ky, ud, ld)); break;
+        default: FAIL(F25_ERR_ARG, "unsupported order");
+    }
+    if (m->ngen) TRY(grad_general<double>(m, m->d_gelem, m->ngen, ntrip, d_om, d_ky, u, l));
     return 0;
 }
 
 // fp32: complex64 fields, FP32 interpolation and densities per triple, FP64 sums
 static int grad_core(f25_mesh *m, int ntrip, const double *d_om, const double *d_ky, const void *u,
                      const void *l, double *g, int chain, bool fp32 = false) {
-    if (fp32) TRY(grad_launch<float>(m, ntrip, d_om, d_ky, u, l));
-    else TRY(grad_launch<double>(m, ntrip, d_om, d_ky, u, l));
+    TRY(grad_launch(m, ntrip, d_om, d_ky, u, l, fp32));
     HIPCHK(hipEventRecord(m->ev1, m->st));
     hipLaunchKernelGGL(k_grad_gather, dim3((m->d.nnpg + 255) / 256), dim3(256), 0, m->st, m->d.nnpg,
                        m->ncon_anchor, m->d_mconn, m->d_ieng, m->d_part, m->d_rho, m->d_lam, m->d_mu,

@@ -23,6 +23,11 @@ struct Tables {
 };
 void make_tables(int nord, Tables &t);
 void gll_nodes(int n, double *x, double *w);
+// 1-D table of the kernels for parallelogram elements (affine.hip): the
+// cardinal functions of the nl interpolation points and their derivatives at
+// the nl Gauss-Legendre points, v[q*nl + j] then v'[q*nl + j], followed by
+// w h0, w h1, h0, h1, w at the points, h0 = (1 - s)/2, h1 = (1 + s)/2
+std::vector<double> af_table(const Tables &t);
 
 // Host-side mesh graph (GEN_GRAPH25 numbering, graph25_driver.f90:30-86).
 struct Graph {

@@ -185,6 +185,44 @@ void make_tables(int nord, Tables &t) {
         }
 }
 
+std::vector<double> af_table(const Tables &t) {
+    const int n = t.nl;
+    std::vector<double> o(2 * n * n + 5 * n);
+    for (int q = 0; q < n; ++q) {
+        // root q of P_n by Newton from the usual cosine start, ascending
+        long double x = -std::cos(3.14159265358979323846L * (q + 0.75L) / (n + 0.5L)), dp = 1.0L;
+        for (int it = 0; it < 8; ++it) {
+            long double p0 = 1.0L, p1 = x;
+            for (int k = 2; k <= n; ++k) {
+                const long double p2 = ((2 * k - 1) * x * p1 - (k - 1) * p0) / k;
+                p0 = p1;
+                p1 = p2;
+            }
+            dp = n * (x * p1 - p0) / (x * x - 1.0L);
+            x -= p1 / dp;
+        }
+        const long double w = 2.0L / ((1.0L - x * x) * dp * dp), h0 = 0.5L * (1.0L - x), h1 = 0.5L * (1.0L + x);
+        for (int j = 0; j < n; ++j) {
+            long double v = 1.0L, d = 0.0L;
+            for (int m = 0; m < n; ++m) {
+                if (m == j) continue;
+                const long double f = 1.0L / ((long double)t.xipts[j] - t.xipts[m]);
+                d = (d * (x - t.xipts[m]) + v) * f;   // product rule, factor by factor
+                v *= (x - t.xipts[m]) * f;
+            }
+            o[q * n + j] = (double)v;
+            o[n * n + q * n + j] = (double)d;
+        }
+        double *c = &o[2 * n * n];
+        c[q] = (double)(w * h0);
+        c[n + q] = (double)(w * h1);
+        c[2 * n + q] = (double)h0;
+        c[3 * n + q] = (double)h1;
+        c[4 * n + q] = (double)w;
+    }
+    return o;
+}
+
 // ---------------------------------------------------------------------------
 // Bilinear position of GLL point (xi, eta) in element e (CSF2DND, csf2d.f:135).
 void gll_xz(const f25_mesh_desc &d, int e, double xi, double eta, double &x, double &z) {

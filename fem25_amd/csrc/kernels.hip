@@ -1599,9 +1599,9 @@ struct GradOcc {
 
 template <int NL, int T, typename R = double>
 __global__ __launch_bounds__((GradOcc<NL, R>::NT)) __attribute__((amdgpu_waves_per_eu(GradOcc<NL, R>::WPE))) void k_grad_sf(
-    const double *__restrict__ t1d, const double *__restrict__ wq, const double *__restrict__ xq,
-    const int *__restrict__ ieng, const double *__restrict__ xl, const double *__restrict__ zl,
-    const char *__restrict__ cdom, const int *__restrict__ lm, int ntrip, int64_t ndof,
+    const int *__restrict__ elems, const double *__restrict__ t1d, const double *__restrict__ wq,
+    const double *__restrict__ xq, const int *__restrict__ ieng, const double *__restrict__ xl,
+    const double *__restrict__ zl, const char *__restrict__ cdom, const int *__restrict__ lm, int ntrip, int64_t ndof,
     const double *__restrict__ omega, const double *__restrict__ ky, const typename CxOf<R>::T *__restrict__ u,
     const typename CxOf<R>::T *__restrict__ l, double *__restrict__ part, int *__restrict__ err) {
     typedef typename CxOf<R>::T C2;
@@ -1625,7 +1625,7 @@ __global__ __launch_bounds__((GradOcc<NL, R>::NT)) __attribute__((amdgpu_waves_p
     constexpr bool XL = PPL == 2;
     double2 *si = reinterpret_cast<double2 *>(s1 + 2 * N1 * Q1);
     __shared__ double red[NT / 64][12];
-    const int e = blockIdx.x, tid = threadIdx.x;
+    const int e = elems ? elems[blockIdx.x] : blockIdx.x, tid = threadIdx.x;
     if (cdom[e] == 'A') {   // PML elements are outside the non-PML gradient path
         if (tid < 12) part[(size_t)e * 12 + tid] = 0.0;
         return;

@@ -1,0 +1,102 @@
+"""Parallelogram elements (affine.hip) beside elements of general shape: a
+sheared mesh whose one displaced anchor leaves four elements non-affine, so
+both kinds of kernels write one result.  Batches at the edges of a wave's
+vectors (PW of them) and of a workgroup's four waves, against the oracle."""
+from __future__ import annotations
+
+import functools
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import oracle
+from fem25_amd import configs as cf
+
+TWOPI = 2.0 * np.pi
+
+
+def pw(p: int) -> int:
+    """Complex vectors of one wave: half of the even number of (p + 1)-lane groups in 64."""
+    return (64 // (p + 1)) // 2
+
+
+@functools.lru_cache(maxsize=None)
+def case(p: int, npml: int = 0):
+    nx, nz = (8, 6) if npml else (5, 4)
+    m = cf.structured_mesh(nx, nz, p, width=2e3 * nx, depth=2e3 * nz, npml=npml, nbielak=1 if npml else 0)
+    if not npml:
+        m.xlocs += 0.25 * m.zlocs              # exact in FP64: every element a parallelogram
+    a = (nz // 2) * (nx + 1) + nx // 2
+    m.xlocs[a] += 310.0
+    m.zlocs[a] -= 170.0
+    mod = cf.layered_model(m, seed=11, n_anom=4, amp=0.1)
+    pml = cf.PML(rcoeff=1e-3, kappa=1.0, fcent=0.05) if npml else cf.PML()
+    return m, mod, pml, oracle.graph(m)
+
+
+@functools.lru_cache(maxsize=None)
+def handle(p: int, npml: int = 0):
+    from fem25_amd.api import MeshInfo
+    m, mod, pml, _ = case(p, npml)
+    mi = MeshInfo(m, pml)
+    mi.set_model(mod)
+    return mi
+
+
+def batch(n: int):
+    om, ky, f, py = cf.freq_ky_batch(3, (n + 2) // 3, 0.02, 0.1, 3500.0)
+    return om[:n], ky[:n], f[:n], py[:n]
+
+
+def err(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+def test_mixed_mesh_has_both_kinds():
+    for p in (2, 6):
+        m, *_ = case(p)
+        x, z = m.xlocs[m.ieng - 1], m.zlocs[m.ieng - 1]
+        twist = [np.abs(v[:, 0] - v[:, 1] + v[:, 2] - v[:, 3]) for v in (x, z)]
+        assert np.count_nonzero(twist[0] + twist[1]) == 4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p", [2, 3, 4, 5, 6])
+def test_gradient(p):
+    m, mod, pml, g = case(p)
+    mi = handle(p)
+    n = 4 * pw(p) + 1
+    om, ky, f, py = batch(n)
+    u, lam = cf.seeded_complex(g.ndof, batch=n, seed=1), cf.seeded_complex(g.ndof, batch=n, seed=2)
+    each = [oracle.grad_exact(m, mod, g, f[b], py[b], u[b], lam[b], pml)[1] for b in range(n)]
+    for k in (1, pw(p), pw(p) + 1, n):
+        ref, got = sum(each[:k]), mi.gradient(om[:k], ky[:k], u[:k], lam[:k])
+        for c in range(3):
+            assert err(got[:, c], ref[:, c]) < 1e-12, (k, c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("npml", [0, 2])
+@pytest.mark.parametrize("p", [2, 3, 4, 5, 6])
+def test_product(p, npml):
+    import torch
+    from fem25_amd import _lib
+    m, mod, pml, g = case(p, npml)
+    mi = handle(p, npml)
+    n = 4 * pw(p) + 1
+    om, ky, f, py = batch(n)
+    x = cf.seeded_complex(g.ndof, batch=n, seed=3)
+    probe = sorted({0, pw(p) - 1, pw(p), n - 1})
+    ref = {b: sp.csr_matrix((oracle.asmble_z(m, mod, g, f[b], py[b], pml), g.jcptr - 1, g.irptr - 1),
+                            shape=(g.ndof, g.ndof)) @ x[b] for b in probe}
+    for k in (1, pw(p), pw(p) + 1, n):
+        y = mi.apply_batch(om[:k], ky[:k], x[:k])
+        for b in probe:
+            if b < k:
+                assert err(y[b], ref[b]) < 1e-12, (k, b)
+    x32 = torch.from_numpy(np.ascontiguousarray(x.T)).to(torch.complex64).cuda()
+    y32 = torch.empty_like(x32)
+    mi.apply_batch_dev(om, ky, x32, y32, _lib.F25_APPLY_F32)
+    y32 = y32.cpu().numpy().T
+    assert all(err(y32[b], ref[b]) < 2e-6 for b in probe)

@@ -1,5 +1,5 @@
-// Kernels for parallelogram elements (gfx950): the adjoint gradient by sum
-// factorisation at the NL-point Gauss-Legendre rule.
+// Kernels for parallelogram elements (gfx950): the batched product and the
+// adjoint gradient by sum factorisation at the NL-point Gauss-Legendre rule.
 //
 // An element whose bilinear map is affine has a constant Jacobian, so every
 // integrand of the element operator and of its model derivatives is a
@@ -17,7 +17,12 @@
 // (its w is -Re u_2; the sign goes to k).  A lane owns one eta point of one
 // real problem: its first pass contracts the element's values along eta with
 // the lane's own 1-D values, everything along xi is then lane-local with
-// wave-uniform coefficients.
+// coefficients common to the wave.  In the product those reach the FMAs as
+// DPP operands: the 16 values of a xi point (v_i, v'_i and the weighted hats)
+// lie across each row of 16 lanes, one register pair a point.  (As scalar registers the
+// tables of p6 do not fit: hoisted out of the loops they spilled, 3,700 vector
+// instructions per chunk of the product instead of 1,900; loaded per point
+// each load is waited for.)
 #pragma once
 
 namespace f25k {
@@ -27,12 +32,12 @@ namespace f25k {
 // PML element
 constexpr int AFR = 20;
 
-// 1-D table (af_table on the host): v_j(q) [NL][NL], v'_j(q) [NL][NL], then
-// w h_0, w h_1, h_0, h_1, w at the points (h_0, h_1 the hat functions)
+// offsets in the 1-D table (af_table on the host): rows of 16 values per
+// point, v_j, v'_j, then w h_0 and w h_1 at HW0, HW1 (h_0, h_1 the hat
+// functions); after the rows h_0, h_1, w
 template <int NL>
 struct AfTab {
-    static constexpr int V = 0, D = NL * NL, HW0 = 2 * NL * NL, HW1 = HW0 + NL, H0 = HW1 + NL, H1 = H0 + NL,
-                         W = H1 + NL, SIZE = W + NL;
+    static constexpr int HW0 = 14, HW1 = 15, H0 = 16 * NL, H1 = 17 * NL, W = 18 * NL;
 };
 
 // Lanes of a wave: PP real problems (PW complex vectors) times NL eta points
@@ -42,9 +47,14 @@ struct AfShape {
     static constexpr int NEN = NL * NL, NEE = 3 * NEN;
     static constexpr int PP = (64 / NL) & ~1, PW = PP / 2, LN = PP * NL;
     static constexpr int NW = 4;                             // waves of a workgroup
+    // the product's LDS per wave: element values of PW vectors, the exchange
+    // of one component's sums, the addresses the element's rows are read from
+    // and written to
+    static constexpr int XS = NEE * PW, ES = 2 * NL * 64;
+    static constexpr size_t lds_apply = (size_t)NW * (XS * 16 + ES * 8 + NEE * 16) + 16 * NL * 8;
     // the gradient's LDS per wave: element values of both fields for PW triples
     static constexpr int GS = 2 * NEE * PW;
-    static constexpr size_t lds_grad = (size_t)NW * GS * 16 + 2 * NL * NL * 8;
+    static constexpr size_t lds_grad = (size_t)NW * GS * 16 + 16 * NL * 8;
 };
 
 __global__ void k_aff_rec(int nelem, const int *__restrict__ ieng, const double *__restrict__ xl,
@@ -137,10 +147,32 @@ __device__ __forceinline__ void af_first(const double *a, const double *an, cons
     }
 }
 
-// Value and reference derivatives at xi point q (vq, dq: its 1-D values).
+// acc += (value J of the row of 16 lanes in cq) * op, in program order: the
+// statement order below keeps the live values within the registers, which the
+// compiler's own order of an unrolled point loop does not
+template <int J>
+__device__ __forceinline__ void fb(double &acc, double cq, double op) {
+    asm volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+v"(acc)
+                 : "v"(cq), "v"(op), "i"(J));
+}
+
+// Values and reference derivatives of three components at the xi point of cq.
+template <int NL, int... I>
+__device__ __forceinline__ void af_point(const double (*T1)[NL], const double (*T2)[NL], double cq, double *U, double *Xi,
+                                         double *Et, std::integer_sequence<int, I...>) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) U[c] = Xi[c] = Et[c] = 0.0;
+    ((fb<I>(U[0], cq, T1[0][I]), fb<I>(U[1], cq, T1[1][I]), fb<I>(U[2], cq, T1[2][I]),
+      fb<NL + I>(Xi[0], cq, T1[0][I]), fb<NL + I>(Xi[1], cq, T1[1][I]), fb<NL + I>(Xi[2], cq, T1[2][I]),
+      fb<I>(Et[0], cq, T2[0][I]), fb<I>(Et[1], cq, T2[1][I]), fb<I>(Et[2], cq, T2[2][I])),
+     ...);
+}
+
+// The same for one component with scalar 1-D values (vq, dq: uniform).
 template <int NL>
-__device__ __forceinline__ void af_point(const double *T1, const double *T2, const double *vq, const double *dq,
-                                         double &U, double &Xi, double &Et) {
+__device__ __forceinline__ void af_point_s(const double *T1, const double *T2, const double *vq, const double *dq,
+                                           double &U, double &Xi, double &Et) {
     U = vq[0] * T1[0];
     Xi = dq[0] * T1[0];
     Et = vq[0] * T2[0];
@@ -149,6 +181,236 @@ __device__ __forceinline__ void af_point(const double *T1, const double *T2, con
         U = fma(vq[i], T1[i], U);
         Xi = fma(dq[i], T1[i], Xi);
         Et = fma(vq[i], T2[i], Et);
+    }
+}
+
+// Projection of one component's fluxes at the xi point of cq on the node columns.
+template <int NL, int... I>
+__device__ __forceinline__ void af_project(double *P1, double *P2, double cq, double A, double B, double N,
+                                           std::integer_sequence<int, I...>) {
+    ((fb<I>(P1[I], cq, N), fb<I>(P2[I], cq, B)), ...);
+    (fb<NL + I>(P1[I], cq, A), ...);
+}
+
+// Rows of one node column from its sums at the eta point of cq.
+template <int NL, int... J>
+__device__ __forceinline__ void af_rows(double *Y, double cq, double p1, double p2, std::integer_sequence<int, J...>) {
+    (fb<J>(Y[J], cq, p1), ...);
+    (fb<NL + J>(Y[J], cq, p2), ...);
+}
+
+// ---------------------------------------------------------------------------
+// y_b = S(omega_b, ky_b) x_b over the parallelogram elements of one colour.
+// A wave takes PW pairs of one element at a time and walks the element's
+// chunks of pairs part, part + nsplit, ... of nch; four waves of consecutive
+// numbers form a workgroup and share only the 1-D table.  Per chunk: the
+// first pass from LDS, then per xi point the fields, the fluxes (density and
+// moduli bilinear in the corners) and their projection back along xi; the
+// last contraction, over eta, runs across lanes: one component's sums at a
+// time go through LDS and each lane forms the NL rows of one xi node column.
+// The next chunk's values stream into LDS meanwhile.  A fixed DOF reads the
+// zero value of its LDS slot.  The rows of y a lane adds to are read from and
+// written to addresses kept in LDS: zpad (npair zeros) for a node touched
+// first and for a fixed DOF, sink (npair values) for the stores of a fixed
+// DOF, so that none of them is a branch (they were a quarter of the
+// instructions).  PML elements only store zeros where they touch a node
+// first.  lm, lm_out: the DOFs read and written, as in k_apply_v (below 2^27,
+// so that a slot's DOF and pair pack into one register).
+//
+// Bound by memory at p4 and by FP64 issue and memory together at p6: four
+// colours read x 1.56 (p4) and 1.36 (p6) times and read y back for the nodes
+// they share, 7.3 GB a product at 200x100 p4, 128 pairs (4.2 TB/s without
+// the point loop, where a large copy runs at 4.66).  Measured on MI355X
+// against the block product of k_apply_v: 200x100 p4, 128 pairs 2.25 -> 1.93
+// ms; 160x80 p6, 192 pairs 6.92 -> 4.2; 40x20 p4, one pair 135 -> 68 us.  On
+// the way, at p4 / p6: scalar tables 2.17 / 5.81; loads waited for after the
+// stores 2.13 / 4.84; the three components' rows kept and stored together
+// 2.33 / 5.80; row addresses computed per row 2.05 / 4.75; the rows' values
+// loaded before the point loop 2.05 / 7.1 (registers).
+template <int NL, typename XT, bool RECT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_apply_af(
+        const int *__restrict__ order, int nel, int nsplit, int nch, const double *__restrict__ rec,
+        const double *__restrict__ tab, const int *__restrict__ lm, const int *__restrict__ lm_out,
+        const unsigned long long *__restrict__ first, int npair, const double *__restrict__ omega,
+        const double *__restrict__ ky, const XT *__restrict__ x, XT *__restrict__ y, const XT *__restrict__ zpad,
+        XT *__restrict__ sink) {
+    typedef AfShape<NL> S;
+    typedef AfTab<NL> TB;
+    typedef decltype(XT().x) R;
+    constexpr int NEE = S::NEE, PP = S::PP, PW = S::PW, LN = S::LN, ES = S::ES;
+    constexpr bool DIRECT = sizeof(XT) == 16;     // straight to LDS; float2 is widened through registers
+    constexpr int NG = (S::XS + 63) / 64;
+    extern __shared__ double sm[];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    double2 *sx = reinterpret_cast<double2 *>(sm) + wv * S::XS;
+    double *sb = sm + S::NW * S::XS * 2 + wv * ES;
+    uint64_t *sr = reinterpret_cast<uint64_t *>(sm + S::NW * (S::XS * 2 + ES)) + wv * 2 * NEE;   // read, then written
+    double *st = sm + S::NW * (S::XS * 2 + ES + 2 * NEE);
+    for (int i = threadIdx.x; i < 16 * NL; i += 256) st[i] = tab[i];
+    __syncthreads();
+    const int wx = blockIdx.x * S::NW + wv, ei = wx / nsplit, part = wx % nsplit;
+    if (ei >= nel) return;
+    const int e = order[ei];
+    const double *rc = rec + (size_t)e * AFR;
+    const unsigned long long fmask = first[e];
+    const int *L = lm + (size_t)e * NEE, *LO = lm_out + (size_t)e * NEE;
+    if (rc[17] != 0.0) {
+        for (int ch = part; ch < nch; ch += nsplit)
+            for (int s = lane; s < S::XS; s += 64) {
+                const int d = s / PW, pair = ch * PW + s % PW, dof = LO[d];
+                if (dof >= 0 && pair < npair && ((fmask >> (d / 3)) & 1ull)) y[(size_t)dof * npair + pair] = XT{0, 0};
+            }
+        return;
+    }
+    // gather slot s = lane + 64 r: element value s / PW of pair s % PW.  Every
+    // DOF is loaded before the first is used (one latency, not one per slot)
+    constexpr int NO = (NEE + 63) / 64;
+    int dp[NG], ds[NO];
+#pragma unroll
+    for (int r = 0; r < NG; ++r) dp[r] = L[min((lane + 64 * r) / PW, NEE - 1)];
+#pragma unroll
+    for (int r = 0; r < NO; ++r) ds[r] = LO[min(lane + 64 * r, NEE - 1)];
+#pragma unroll
+    for (int r = 0; r < NG; ++r) {
+        const int s = lane + 64 * r;
+        if (s < S::XS && dp[r] < 0) sx[s] = make_double2(0.0, 0.0);
+        dp[r] = s < S::XS && dp[r] >= 0 ? dp[r] * 16 + s % PW : -1;
+    }
+#pragma unroll
+    for (int r = 0; r < NO; ++r) {
+        const int i = lane + 64 * r;
+        XT *row = ds[r] >= 0 ? y + (size_t)ds[r] * npair : sink;
+        if (i < NEE) {
+            sr[i] = reinterpret_cast<uint64_t>(ds[r] >= 0 && !((fmask >> (i / 3)) & 1ull) ? row : zpad);
+            sr[NEE + i] = reinterpret_cast<uint64_t>(row);
+        }
+    }
+    XT pre[DIRECT ? 1 : NG];
+    auto get = [&](int p0) {
+#pragma unroll
+        for (int r = 0; r < NG; ++r)
+            if (dp[r] >= 0) {
+                const XT *src = x + ((size_t)(dp[r] >> 4) * npair + min(p0 + (dp[r] & 15), npair - 1));
+                if constexpr (DIRECT) dma16(src, sx + 64 * r);
+                else pre[r] = *src;
+            }
+    };
+    lds_wait();
+    get(part * PW);
+    const int le = min(lane, LN - 1), eta = le / PP, pr = (le % PP) >> 1, im = le & 1;
+    const double *stl = st + (lane & 15);   // the lane's values of the table's rows
+    const auto seq = std::make_integer_sequence<int, NL>();
+    auto pairof = [&](int ch) { return min(ch * PW + pr, npair - 1); };
+    double omn = omega[pairof(part)], kyn = ky[pairof(part)];   // of the next chunk, loaded ahead with its values
+    // geometry and the corner values at the lane's eta point, times w det J
+    const double rx = rc[0], sxx = rc[1], rz = rc[2], sz = rc[3];
+    const double h0 = tab[TB::H0 + eta], h1 = tab[TB::H1 + eta], we = tab[TB::W + eta] * rc[4];
+    const double rL = (rc[5] * h0 + rc[8] * h1) * we, rR = (rc[6] * h0 + rc[7] * h1) * we;
+    const double lL = (rc[9] * h0 + rc[12] * h1) * we, lR = (rc[10] * h0 + rc[11] * h1) * we;
+    const double mL = (rc[13] * h0 + rc[16] * h1) * we, mR = (rc[14] * h0 + rc[15] * h1) * we;
+    if constexpr (DIRECT) dma_wait();
+    for (int ch = part; ch < nch; ch += nsplit) {
+        const int pair = ch * PW + pr;
+        const bool live = lane < LN && pair < npair;
+        const double w2 = -omn * omn, kv = im ? -kyn : kyn;
+        if constexpr (!DIRECT) {
+#pragma unroll
+            for (int r = 0; r < NG; ++r)
+                if (dp[r] >= 0) sx[lane + 64 * r] = make_double2((double)pre[r].x, (double)pre[r].y);
+            lds_wait();
+        }
+        double T1[3][NL], T2[3][NL];
+        {
+            double v[NL], d[NL], c0[NL];
+#pragma unroll
+            for (int j = 0; j < NL; ++j) { v[j] = st[eta * 16 + j]; d[j] = (RECT ? sz : 1.0) * st[eta * 16 + NL + j]; }
+            const double *a = reinterpret_cast<const double *>(sx) + 2 * pr;
+            auto at = [&](int c) { return a + c * PW * 2 + (c == 1 ? 1 - im : im); };
+#pragma unroll
+            for (int j = 0; j < NL; ++j) c0[j] = at(0)[j * NL * 3 * PW * 2];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) af_first<NL, 3 * PW * 2>(at(c), at(c < 2 ? c + 1 : 0), v, d, c0, T1[c], T2[c]);
+        }
+        lds_wait();
+        if (ch + nsplit < nch) {
+            get((ch + nsplit) * PW);
+            omn = omega[pairof(ch + nsplit)];
+            kyn = ky[pairof(ch + nsplit)];
+        }
+        const double rL2 = rL * w2, rR2 = rR * w2;
+        double P1[3][NL], P2[3][NL];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int i = 0; i < NL; ++i) P1[c][i] = P2[c][i] = 0.0;
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            const double cq = stl[q * 16];
+            double U[3], Xi[3], Et[3], X[3], Z[3], lq = 0.0, mq = 0.0, rq = 0.0;
+            fb<TB::HW0>(lq, cq, lL); fb<TB::HW0>(mq, cq, mL); fb<TB::HW0>(rq, cq, rL2);
+            fb<TB::HW1>(lq, cq, lR); fb<TB::HW1>(mq, cq, mR); fb<TB::HW1>(rq, cq, rR2);
+            af_point<NL>(T1, T2, cq, U, Xi, Et, seq);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                X[c] = RECT ? rx * Xi[c] : rx * Xi[c] + sxx * Et[c];
+                Z[c] = RECT ? Et[c] : rz * Xi[c] + sz * Et[c];
+            }
+            const double ld = lq * (X[0] + Z[2] + kv * U[1]), m2 = 2.0 * mq;
+            const double FX0 = fma(m2, X[0], ld), FZ2 = fma(m2, Z[2], ld), F13 = mq * (Z[0] + X[2]);
+            const double FX1 = mq * (X[1] - kv * U[0]), FZ1 = mq * (Z[1] - kv * U[2]);
+            const double FX[3] = {FX0, FX1, F13}, FZ[3] = {F13, FZ1, FZ2};
+            const double FN[3] = {rq * U[0] - kv * FX1, fma(kv, ld, fma(kv * kv, m2, rq) * U[1]), rq * U[2] - kv * FZ1};
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const double A = RECT ? rx * FX[c] : rx * FX[c] + rz * FZ[c];
+                const double B = RECT ? sz * FZ[c] : sxx * FX[c] + sz * FZ[c];
+                af_project<NL>(P1[c], P2[c], cq, A, B, FN[c], seq);
+            }
+        }
+        double cr[NL];
+#pragma unroll
+        for (int q = 0; q < NL; ++q) cr[q] = stl[q * 16];
+        // the rows this lane adds to: node column i = eta, rows j; bytes from
+        // a row's address to the lane's value of components 1, 3 and of 2
+        const uint64_t po = (uint64_t)min(pair, npair - 1) * sizeof(XT);
+        const uint64_t oc[2] = {po + im * sizeof(R), po + (1 - im) * sizeof(R)};
+        const uint64_t *se = sr + 3 * eta;
+        R yv[3][NL];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int j = 0; j < NL; ++j) yv[c][j] = *(const __attribute__((address_space(1))) R *)(se[j * NL * 3 + c] + oc[c == 1]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            lds_wait();   // the previous component's sums are read
+#pragma unroll
+            for (int i = 0; i < NL; ++i) {
+                sb[(2 * i) * 64 + lane] = P1[c][i];
+                sb[(2 * i + 1) * 64 + lane] = P2[c][i];
+            }
+            lds_wait();
+            double Y[NL];
+#pragma unroll
+            for (int j = 0; j < NL; ++j) Y[j] = 0.0;
+            const double *b = sb + 2 * eta * 64 + le % PP;
+#pragma unroll
+            for (int q = 0; q < NL; ++q) {
+                const double p1 = b[q * PP], p2 = b[64 + q * PP];
+                af_rows<NL>(Y, cr[q], p1, p2, seq);
+            }
+            if (c == 0) {
+                // every load so far (the rows' values, the next chunk's) is
+                // awaited here, before the first store: a later wait for any
+                // of them would wait for the stores before it too
+                dma_wait();
+#pragma unroll
+                for (int k = 0; k < 3 * NL; ++k) asm volatile("" : "+v"(yv[k / NL][k % NL]));
+            }
+            if (live)
+#pragma unroll
+                for (int j = 0; j < NL; ++j)
+                    *(__attribute__((address_space(1))) R *)(se[NEE + j * NL * 3 + c] + oc[c == 1]) = (R)((double)yv[c][j] + Y[j]);
+        }
     }
 }
 
@@ -169,7 +431,8 @@ __device__ __forceinline__ void af_point(const double *T1, const double *T2, con
 // across vectors (index arithmetic per load) 2.03 ms at p4, one column at a
 // time in the first pass (each waited for its LDS reads) 1.82; the point
 // loop unrolled spills (p6 1.03 ms against 0.56), its 1-D values loaded one
-// point ahead 1.67 ms.
+// point ahead 1.67 ms, or as DPP operands in program order 1.71 (p6 0.65):
+// here the scalar loads of a rolled loop cost less than that order.
 template <int NL, bool RECT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_grad_af(
         const int *__restrict__ elems, const double *__restrict__ rec, const double *__restrict__ tab,
@@ -191,7 +454,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         if (threadIdx.x < 12) part[(size_t)e * 12 + threadIdx.x] = 0.0;
         return;
     }
-    for (int i = threadIdx.x; i < 2 * NL * NL; i += blockDim.x) st[i] = tab[i];
+    for (int i = threadIdx.x; i < 16 * NL; i += blockDim.x) st[i] = tab[i];
     __syncthreads();
     const int nch = (ntrip + PW - 1) / PW;
     typedef AfGather<NEE, 2 * PW> G;
@@ -221,7 +484,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         {
             double v[NL], d[NL];
 #pragma unroll
-            for (int j = 0; j < NL; ++j) { v[j] = st[eta * NL + j]; d[j] = (RECT ? sz : 1.0) * st[NL * NL + eta * NL + j]; }
+            for (int j = 0; j < NL; ++j) { v[j] = st[eta * 16 + j]; d[j] = (RECT ? sz : 1.0) * st[eta * 16 + NL + j]; }
             const double *a = reinterpret_cast<const double *>(sw + tr * NEE);
             auto at = [&](int k) {   // component k % 3 of field k / 3
                 return a + (k / 3) * (2 * PW * NEE) + 2 * (k % 3) + (k % 3 == 1 ? 1 - im : im);
@@ -244,8 +507,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         for (int k = 0; k < 6; ++k) s[k] = 0.0;
 #pragma unroll 1
         for (int q = 0; q < NL; ++q) {
-            const double *vq = tab + TB::V + q * NL, *dq = tab + TB::D + q * NL;
-            const double a0 = tab[TB::HW0 + q], a1 = tab[TB::HW1 + q];
+            const double *vq = tab + 16 * q, *dq = vq + NL;
+            const double a0 = tab[16 * q + TB::HW0], a1 = tab[16 * q + TB::HW1];
             double U[2][3], X0[2], Z2[2], div[2], a12[2], a23[2], a13[2];
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
@@ -253,7 +516,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
                     double Xi, Et;
-                    af_point<NL>(T1[f][c], T2[f][c], vq, dq, U[f][c], Xi, Et);
+                    af_point_s<NL>(T1[f][c], T2[f][c], vq, dq, U[f][c], Xi, Et);
                     X[c] = RECT ? rx * Xi : rx * Xi + sxx * Et;
                     Z[c] = RECT ? Et : rz * Xi + sz * Et;
                 }

@@ -107,6 +107,9 @@ struct f25_mesh_s {
     bool rect = true;   // the parallelograms' sides all lie along x and z
     int *d_aelem = nullptr, *d_gelem = nullptr;
     int naff = 0, ngen = 0;
+    // the same by colour: order splits into aorder and gorder
+    int *d_aorder = nullptr, *d_gorder = nullptr;
+    std::vector<int> acptr, gcptr;
     char *d_cdom = nullptr, *d_cnp = nullptr;
     double *d_rho = nullptr, *d_lam = nullptr, *d_mu = nullptr;
     double *d_blk = nullptr;
@@ -246,6 +249,20 @@ static bool is_affine(const f25_mesh *m, int e) {
     return std::fabs(bx) <= tol && std::fabs(bz) <= tol && det > 2.22e-16;
 }
 
+// a colour order's elements by kind (m->affine), each in colour order
+static void split_order(const f25_mesh *m, const std::vector<int> &order, const std::vector<int> &cptr,
+                        std::vector<int> &ao, std::vector<int> &ap, std::vector<int> &go, std::vector<int> &gp) {
+    ao.clear();
+    go.clear();
+    ap.assign(1, 0);
+    gp.assign(1, 0);
+    for (size_t c = 0; c + 1 < cptr.size(); ++c) {
+        for (int i = cptr[c]; i < cptr[c + 1]; ++i) (m->affine[order[i]] ? ao : go).push_back(order[i]);
+        ap.push_back((int)ao.size());
+        gp.push_back((int)go.size());
+    }
+}
+
 static int upload_mesh(f25_mesh *m) {
     const f25_mesh_desc &d = m->d;
     hipStream_t s = m->st;
@@ -326,6 +343,9 @@ static int upload_mesh(f25_mesh *m) {
     m->ngen = (int)gel.size();
     TRY(upload(&m->d_aelem, ael.data(), ael.size(), s));
     TRY(upload(&m->d_gelem, gel.data(), gel.size(), s));
+    split_order(m, m->order, m->cptr, ael, m->acptr, gel, m->gcptr);
+    TRY(upload(&m->d_aorder, ael.data(), ael.size(), s));
+    TRY(upload(&m->d_gorder, gel.data(), gel.size(), s));
     const std::vector<double> taf = af_table(m->tab);
     TRY(upload(&m->d_taf, taf.data(), taf.size(), s));
     TRY(dalloc(&m->d_rec, (size_t)d.nelem * AFR));
@@ -503,6 +523,7 @@ extern "C" int f25_mesh_destroy(f25_mesh *m) {
     dfree(m->d_ieng); dfree(m->d_lm); dfree(m->d_first); dfree(m->d_order); dfree(m->d_pml_order); dfree(m->d_err);
     dfree(m->d_xl); dfree(m->d_zl); dfree(m->d_xd); dfree(m->d_zd); dfree(m->d_shl); dfree(m->d_wq); dfree(m->d_t1d);
     dfree(m->d_taf); dfree(m->d_rec); dfree(m->d_aelem); dfree(m->d_gelem);
+    dfree(m->d_aorder); dfree(m->d_gorder);
     dfree(m->d_xq); dfree(m->d_cdom); dfree(m->d_cnp); dfree(m->d_rho); dfree(m->d_lam); dfree(m->d_mu);
     if (m->ag.exec) (void)hipGraphExecDestroy(m->ag.exec);
     dfree(m->d_vcf); dfree(m->d_dvcf); dfree(m->d_vpad);
@@ -925,21 +946,16 @@ static size_t apply_v_grid(int n, int npair) {
     return 8 * (((size_t)(n + 7) / 8 * ngrp * wpt + 3) / 4);
 }
 
-// FP64 product (k_apply_v): one launch per element colour
+// FP64 product on element blocks (k_apply_v): the n elements of one colour
 template <int NL, int NRT>
-static int launch_apply_v(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x,
-                          double2 *y, const double *vcf) {
+static int launch_apply_v(f25_mesh *m, const int *order, int n, const double *om, const double *kv, int npair,
+                          const double2 *x, double2 *y, const double *vcf) {
     const double2 *zpad = reinterpret_cast<const double2 *>(m->d_vpad);
     double2 *sink = reinterpret_cast<double2 *>(m->d_vpad) + m->vpad_cap;
-    for (size_t c = 0; c + 1 < m->cptr.size(); ++c) {
-        int n = m->cptr[c + 1] - m->cptr[c];
-        if (!n) continue;
-        const size_t nwg = apply_v_grid<NL, NRT>(n, npair);
-        if (nwg > 0x7fffffff) FAIL(F25_ERR_ARG, "too many pairs for one launch");
-        hipLaunchKernelGGL((k_apply_v<NL, NRT>), dim3((unsigned)nwg), dim3(VShape<NL, NRT>::NT), 0, m->st,
-                           m->d_order + m->cptr[c], n, vcf, m->d_lm, m->d_lm, m->d_first, npair, om, kv, x, y,
-                           zpad, sink);
-    }
+    const size_t nwg = apply_v_grid<NL, NRT>(n, npair);
+    if (nwg > 0x7fffffff) FAIL(F25_ERR_ARG, "too many pairs for one launch");
+    hipLaunchKernelGGL((k_apply_v<NL, NRT>), dim3((unsigned)nwg), dim3(VShape<NL, NRT>::NT), 0, m->st, order, n, vcf,
+                       m->d_lm, m->d_lm, m->d_first, npair, om, kv, x, y, zpad, sink);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1020,11 +1036,10 @@ static int ensure_vpad(f25_mesh *m, int npair) {
     return 0;
 }
 
-// the launches of the FP64 product (ensure_vpad first)
-static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x, double2 *y,
-                      const double *vcf) {
+static int launch_blocks_f64(f25_mesh *m, const int *order, int n, const double *om, const double *kv, int npair,
+                             const double2 *x, double2 *y, const double *vcf) {
     switch (m->tab.nl * 8 + apply_nrt(m)) {
-#define F25_AV(N, T) case N * 8 + T: return launch_apply_v<N, T>(m, om, kv, npair, x, y, vcf);
+#define F25_AV(N, T) case N * 8 + T: return launch_apply_v<N, T>(m, order, n, om, kv, npair, x, y, vcf);
         F25_AV(3, 1) F25_AV(3, 2) F25_AV(4, 1) F25_AV(4, 2) F25_AV(5, 1) F25_AV(5, 2) F25_AV(5, 3)
         F25_AV(6, 2) F25_AV(6, 3) F25_AV(6, 4) F25_AV(7, 2) F25_AV(7, 3) F25_AV(7, 4)
 #undef F25_AV
@@ -1032,10 +1047,67 @@ static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair
     FAIL(F25_ERR_ARG, "unsupported order");
 }
 
+// Product of n parallelogram elements of one colour (k_apply_af).  Waves per
+// element: one per chunk of pairs until the launch has about 16,384 waves
+// (eight per CU, several times over), so that the element's setup is shared
+// by as many chunks as the mesh allows; at least four where there are as
+// many chunks, one workgroup per element.
+template <int NL, typename XT>
+static int launch_apply_af(f25_mesh *m, const int *order, int n, const int *lm_in, const int *lm_out,
+                           const unsigned long long *first, const double *rec, const double *om, const double *kv,
+                           int npair, const XT *x, XT *y) {
+    typedef AfShape<NL> S;
+    auto kern = m->rect ? k_apply_af<NL, XT, true> : k_apply_af<NL, XT, false>;
+    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_apply));
+    const int nch = (npair + S::PW - 1) / S::PW;
+    const int nsplit = std::min(nch, std::max(S::NW, (16384 + n - 1) / n));
+    const int64_t nwg = ((int64_t)n * nsplit + S::NW - 1) / S::NW;
+    if (nwg > 0x7fffffff) FAIL(F25_ERR_ARG, "too many pairs for one launch");
+    hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(256), S::lds_apply, m->st, order, n, nsplit, nch, rec, m->d_taf,
+                       lm_in, lm_out, first, npair, om, kv, x, y, reinterpret_cast<const XT *>(m->d_vpad),
+                       reinterpret_cast<XT *>(m->d_vpad + 2 * (size_t)m->vpad_cap));
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+template <typename XT>
+static int affine_colour(f25_mesh *m, const int *order, int n, const int *lm_in, const int *lm_out,
+                         const unsigned long long *first, const double *rec, const double *om, const double *kv,
+                         int npair, const XT *x, XT *y) {
+    switch (m->tab.nl) {
+#define F25_AF(N) case N: return launch_apply_af<N, XT>(m, order, n, lm_in, lm_out, first, rec, om, kv, npair, x, y);
+        F25_AF(3) F25_AF(4) F25_AF(5) F25_AF(6) F25_AF(7)
+#undef F25_AF
+    }
+    FAIL(F25_ERR_ARG, "unsupported order");
+}
+
+// whether the product's parallelograms run in k_apply_af: it packs a DOF and
+// a pair into one register, and a row-tile count asked for (f25_set_apply_tiles)
+// means the block kernel
+static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt && m->g.ndof < (1 << 27); }
+
+// the launches of the FP64 product (ensure_vpad first), one or two per
+// colour: the parallelograms by rec (null: as blocks too), the others by vcf
+static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x, double2 *y,
+                      const double *rec, const double *vcf) {
+    const bool aff = rec && affine_product(m);
+    for (size_t c = 0; c + 1 < m->cptr.size(); ++c) {
+        const std::vector<int> &gp = aff ? m->gcptr : m->cptr;
+        if (aff && m->acptr[c + 1] > m->acptr[c])
+            TRY(affine_colour(m, m->d_aorder + m->acptr[c], m->acptr[c + 1] - m->acptr[c], m->d_lm, m->d_lm, m->d_first,
+                              rec, om, kv, npair, x, y));
+        if (gp[c + 1] > gp[c])
+            TRY(launch_blocks_f64(m, (aff ? m->d_gorder : m->d_order) + gp[c], gp[c + 1] - gp[c], om, kv, npair, x, y,
+                                  vcf));
+    }
+    return 0;
+}
+
 static int apply_f64(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x, double2 *y,
-                     const double *vcf) {
+                     const double *rec, const double *vcf) {
     TRY(ensure_vpad(m, npair));
-    return launch_f64(m, om, kv, npair, x, y, vcf);
+    return launch_f64(m, om, kv, npair, x, y, rec, vcf);
 }
 
 // ---- elements of the batched product integrated per omega ---------------
@@ -1157,7 +1229,7 @@ static int disp_product(f25_mesh *m, int npair, const double *d_ky, const XT *x,
 
 // F25_APPLY_GRAPH: capture the launches once per argument set, then replay
 static int apply_f64_graph(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x,
-                           double2 *y, const double *vcf) {
+                           double2 *y, const double *rec, const double *vcf) {
     TRY(ensure_vpad(m, npair));
     auto &G = m->ag;
     const auto &P = m->pa;
@@ -1172,7 +1244,7 @@ static int apply_f64_graph(f25_mesh *m, const double *om, const double *kv, int 
         }
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(m->st, hipStreamCaptureModeThreadLocal));
-        int r = m->disp ? disp_product(m, npair, kv, x, y) : launch_f64(m, om, kv, npair, x, y, vcf);
+        int r = m->disp ? disp_product(m, npair, kv, x, y) : launch_f64(m, om, kv, npair, x, y, rec, vcf);
         if (!r && !m->disp) r = pml_launch(m, npair, kv, x, y);
         hipError_t e = hipStreamEndCapture(m->st, &g);
         if (r) {
@@ -1197,7 +1269,7 @@ static int apply_f64_graph(f25_mesh *m, const double *om, const double *kv, int 
 // included (the operator product), null for products on derivative blocks
 // (the PML anchors' parameters are held fixed there).
 static int apply_core(f25_mesh *m, int npair, const double *d_om, const double *d_ky, int mode,
-                      const void *x, void *y, const double *vcf, const double *h_om) {
+                      const void *x, void *y, const double *rec, const double *vcf, const double *h_om) {
     // every DOF is written by the first element touching it: no zero fill
     const bool graph = (mode & F25_APPLY_GRAPH) != 0;
     mode &= ~F25_APPLY_GRAPH;
@@ -1213,9 +1285,9 @@ static int apply_core(f25_mesh *m, int npair, const double *d_om, const double *
         if (mode == F25_APPLY_F32) TRY(disp_product(m, npair, d_ky, (const float2 *)x, (float2 *)y));
         else TRY(disp_product(m, npair, d_ky, (const double2 *)x, (double2 *)y));
     } else if (mode == F25_APPLY_F64 && graph)
-        TRY(apply_f64_graph(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y, vcf));
+        TRY(apply_f64_graph(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y, rec, vcf));
     else if (mode == F25_APPLY_F64) {
-        TRY(apply_f64(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y, vcf));
+        TRY(apply_f64(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y, rec, vcf));
         TRY(pml_launch(m, npair, d_ky, (const double2 *)x, (double2 *)y));
     } else if (mode == F25_APPLY_F32) {
         TRY((dispatch_apply<float, float2, false>(m, d_om, d_ky, npair, (const float2 *)x, (float2 *)y,
@@ -1261,7 +1333,7 @@ extern "C" int f25_apply_batch_dev(f25_mesh *m, int npair, const double *omega, 
     if (!m->have_model) FAIL(F25_ERR_STATE, "f25_set_model has not been called");
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
-    return apply_core(m, npair, m->d_omky, m->d_omky + m->omky_cap, mode, x, y, m->d_vcf, omega);
+    return apply_core(m, npair, m->d_omky, m->d_omky + m->omky_cap, mode, x, y, m->d_rec, m->d_vcf, omega);
 }
 
 extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omega, const double *ky,
@@ -1271,7 +1343,7 @@ extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omeg
     if (!m->have_model) FAIL(F25_ERR_STATE, "f25_set_model has not been called");
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
-    TRY(apply_core(m, npair, m->d_omky, m->d_omky + m->omky_cap, F25_APPLY_F64, u, r, m->d_vcf, omega));
+    TRY(apply_core(m, npair, m->d_omky, m->d_omky + m->omky_cap, F25_APPLY_F64, u, r, m->d_rec, m->d_vcf, omega));
     const int gy = (int)std::min<int64_t>(256, std::max<int64_t>(1, m->g.ndof / 256));
     double *part = nullptr, *sums = nullptr;
     int rc = dalloc(&part, (size_t)gy * npair * 2);
@@ -3081,7 +3153,7 @@ extern "C" int f25_gn_fv(f25_mesh *m, int ntrip, const double *omega, const doub
     r = (e == hipSuccess) ? 0 : F25_ERR_HIP;
     if (!r) r = transpose_dev(m->st, a, b, ntrip, m->g.ndof);
     if (!r) r = vcoef(m, m->d_dblk, &m->d_dvcf);
-    if (!r) r = apply_core(m, ntrip, d_om, d_ky, F25_APPLY_F64, b, a, m->d_dvcf, nullptr);
+    if (!r) r = apply_core(m, ntrip, d_om, d_ky, F25_APPLY_F64, b, a, nullptr, m->d_dvcf, nullptr);
     if (!r) r = transpose_dev(m->st, a, b, m->g.ndof, ntrip);
     if (!r) {
         e = hipMemcpyAsync(out, b, nn * 16, hipMemcpyDeviceToHost, m->st);

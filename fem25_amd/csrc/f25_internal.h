@@ -23,10 +23,11 @@ struct Tables {
 };
 void make_tables(int nord, Tables &t);
 void gll_nodes(int n, double *x, double *w);
-// 1-D table of the kernels for parallelogram elements (affine.hip): the
-// cardinal functions of the nl interpolation points and their derivatives at
-// the nl Gauss-Legendre points, v[q*nl + j] then v'[q*nl + j], followed by
-// w h0, w h1, h0, h1, w at the points, h0 = (1 - s)/2, h1 = (1 + s)/2
+// 1-D table of the kernels for parallelogram elements (affine.hip) at the nl
+// Gauss-Legendre points: for each point q a row of 16 values, the cardinal
+// functions of the interpolation points v_j(q), their derivatives v'_j(q)
+// (2 nl <= 14 values), at 14 and 15 w h0 and w h1; after the rows h0, h1 and
+// w at the points (h0 = (1 - s)/2, h1 = (1 + s)/2)
 std::vector<double> af_table(const Tables &t);
 
 // Host-side mesh graph (GEN_GRAPH25 numbering, graph25_driver.f90:30-86).

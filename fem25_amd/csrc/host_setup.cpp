@@ -187,7 +187,7 @@ void make_tables(int nord, Tables &t) {
 
 std::vector<double> af_table(const Tables &t) {
     const int n = t.nl;
-    std::vector<double> o(2 * n * n + 5 * n);
+    std::vector<double> o(19 * n, 0.0);
     for (int q = 0; q < n; ++q) {
         // root q of P_n by Newton from the usual cosine start, ascending
         long double x = -std::cos(3.14159265358979323846L * (q + 0.75L) / (n + 0.5L)), dp = 1.0L;
@@ -210,15 +210,14 @@ std::vector<double> af_table(const Tables &t) {
                 d = (d * (x - t.xipts[m]) + v) * f;   // product rule, factor by factor
                 v *= (x - t.xipts[m]) * f;
             }
-            o[q * n + j] = (double)v;
-            o[n * n + q * n + j] = (double)d;
+            o[16 * q + j] = (double)v;
+            o[16 * q + n + j] = (double)d;
         }
-        double *c = &o[2 * n * n];
-        c[q] = (double)(w * h0);
-        c[n + q] = (double)(w * h1);
-        c[2 * n + q] = (double)h0;
-        c[3 * n + q] = (double)h1;
-        c[4 * n + q] = (double)w;
+        o[16 * q + 14] = (double)(w * h0);
+        o[16 * q + 15] = (double)(w * h1);
+        o[16 * n + q] = (double)h0;
+        o[17 * n + q] = (double)h1;
+        o[18 * n + q] = (double)w;
     }
     return o;
 }

@@ -888,51 +888,42 @@ extern "C" int f25_asmb_peff(f25_mesh *m, const void *cdist, const void *ue, voi
 }
 
 // ---------------------------------------------------------------------------
+// the FP32 modes' product on element blocks (k_apply): n elements of one colour
 template <int NL, typename BT, typename XT, bool REFINE, int CSEL>
-static int launch_apply_c(f25_mesh *m, const double *om, const double *kv, int npair, const XT *x,
-                          XT *y, const BT *blk, const BT *blk_lo) {
+static int launch_apply_c(f25_mesh *m, const int *order, int n, const double *om, const double *kv, int npair,
+                          const XT *x, XT *y, const BT *blk, const BT *blk_lo) {
     const double *cmx = REFINE ? reinterpret_cast<const double *>(m->d_colmax) : nullptr;
     typedef ApplyLds<NL, BT, REFINE> LD;
     constexpr size_t lds = CSEL < 0 ? LD::bytes : (5 * LD::per_blk + 3 * ApplyShape<NL>::NEN * sizeof(int));
-    static bool attr_set = false;
     auto kern = k_apply<NL, BT, XT, REFINE, CSEL>;
-    if (!attr_set) {
-        HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
-    for (size_t c = 0; c + 1 < m->cptr.size(); ++c) {
-        int n = m->cptr[c + 1] - m->cptr[c];
-        if (!n) continue;
-        hipLaunchKernelGGL(kern, dim3(n), dim3(64 * ApplyLds<NL, BT, REFINE>::NW), lds, m->st,
-                           m->d_order + m->cptr[c], blk, blk_lo,
-                           m->d_lm, m->d_first, npair, om, kv, cmx, x, y);
-    }
+    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, dim3(n), dim3(64 * ApplyLds<NL, BT, REFINE>::NW), lds, m->st, order, blk, blk_lo, m->d_lm,
+                       m->d_first, npair, om, kv, cmx, x, y);
     HIPCHK(hipGetLastError());
     return 0;
 }
 
 template <int NL, typename BT, typename XT, bool REFINE>
-static int launch_apply(f25_mesh *m, const double *om, const double *kv, int npair, const XT *x,
-                        XT *y, const BT *blk, const BT *blk_lo) {
+static int launch_apply(f25_mesh *m, const int *order, int n, const double *om, const double *kv, int npair,
+                        const XT *x, XT *y, const BT *blk, const BT *blk_lo) {
     if constexpr (!ApplyLds<NL, BT, REFINE>::PH) {
-        return launch_apply_c<NL, BT, XT, REFINE, -1>(m, om, kv, npair, x, y, blk, blk_lo);
-    } else {
-        // one output component per pass; the colour order is kept within each pass
-        TRY((launch_apply_c<NL, BT, XT, REFINE, 0>(m, om, kv, npair, x, y, blk, blk_lo)));
-        TRY((launch_apply_c<NL, BT, XT, REFINE, 1>(m, om, kv, npair, x, y, blk, blk_lo)));
-        return launch_apply_c<NL, BT, XT, REFINE, 2>(m, om, kv, npair, x, y, blk, blk_lo);
+        return launch_apply_c<NL, BT, XT, REFINE, -1>(m, order, n, om, kv, npair, x, y, blk, blk_lo);
+    } else {   // one output component per launch
+        TRY((launch_apply_c<NL, BT, XT, REFINE, 0>(m, order, n, om, kv, npair, x, y, blk, blk_lo)));
+        TRY((launch_apply_c<NL, BT, XT, REFINE, 1>(m, order, n, om, kv, npair, x, y, blk, blk_lo)));
+        return launch_apply_c<NL, BT, XT, REFINE, 2>(m, order, n, om, kv, npair, x, y, blk, blk_lo);
     }
 }
 
 template <typename BT, typename XT, bool REFINE>
-static int dispatch_apply(f25_mesh *m, const double *om, const double *kv, int npair, const XT *x,
-                          XT *y, const BT *blk, const BT *blk_lo) {
+static int dispatch_apply(f25_mesh *m, const int *order, int n, const double *om, const double *kv, int npair,
+                          const XT *x, XT *y, const BT *blk, const BT *blk_lo) {
     switch (m->tab.nl) {
-        case 3: return launch_apply<3, BT, XT, REFINE>(m, om, kv, npair, x, y, blk, blk_lo);
-        case 4: return launch_apply<4, BT, XT, REFINE>(m, om, kv, npair, x, y, blk, blk_lo);
-        case 5: return launch_apply<5, BT, XT, REFINE>(m, om, kv, npair, x, y, blk, blk_lo);
-        case 6: return launch_apply<6, BT, XT, REFINE>(m, om, kv, npair, x, y, blk, blk_lo);
-        case 7: return launch_apply<7, BT, XT, REFINE>(m, om, kv, npair, x, y, blk, blk_lo);
+        case 3: return launch_apply<3, BT, XT, REFINE>(m, order, n, om, kv, npair, x, y, blk, blk_lo);
+        case 4: return launch_apply<4, BT, XT, REFINE>(m, order, n, om, kv, npair, x, y, blk, blk_lo);
+        case 5: return launch_apply<5, BT, XT, REFINE>(m, order, n, om, kv, npair, x, y, blk, blk_lo);
+        case 6: return launch_apply<6, BT, XT, REFINE>(m, order, n, om, kv, npair, x, y, blk, blk_lo);
+        case 7: return launch_apply<7, BT, XT, REFINE>(m, order, n, om, kv, npair, x, y, blk, blk_lo);
     }
     FAIL(F25_ERR_ARG, "unsupported order");
 }
@@ -1101,6 +1092,32 @@ static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair
             TRY(launch_blocks_f64(m, (aff ? m->d_gorder : m->d_order) + gp[c], gp[c + 1] - gp[c], om, kv, npair, x, y,
                                   vcf));
     }
+    return 0;
+}
+
+// The FP32 products (ensure_vpad first).  Plain FP32 takes its parallelograms
+// through k_apply_af on complex64 vectors: FP64 arithmetic runs at the rate
+// of FP32 arithmetic without packed instructions, and the vectors are what
+// the kernel moves.  The refined product keeps its blocks for every element.
+static int launch_f32(f25_mesh *m, const double *om, const double *kv, int npair, const float2 *x, float2 *y) {
+    const bool aff = affine_product(m);
+    for (size_t c = 0; c + 1 < m->cptr.size(); ++c) {
+        const std::vector<int> &gp = aff ? m->gcptr : m->cptr;
+        if (aff && m->acptr[c + 1] > m->acptr[c])
+            TRY(affine_colour(m, m->d_aorder + m->acptr[c], m->acptr[c + 1] - m->acptr[c], m->d_lm, m->d_lm, m->d_first,
+                              m->d_rec, om, kv, npair, x, y));
+        if (gp[c + 1] > gp[c])
+            TRY((dispatch_apply<float, float2, false>(m, (aff ? m->d_gorder : m->d_order) + gp[c], gp[c + 1] - gp[c], om,
+                                                      kv, npair, x, y, m->d_blk32, nullptr)));
+    }
+    return 0;
+}
+
+static int launch_refined(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x, double2 *y) {
+    for (size_t c = 0; c + 1 < m->cptr.size(); ++c)
+        if (m->cptr[c + 1] > m->cptr[c])
+            TRY((dispatch_apply<float, double2, true>(m, m->d_order + m->cptr[c], m->cptr[c + 1] - m->cptr[c], om, kv,
+                                                      npair, x, y, m->d_blk_hi, m->d_blk_lo)));
     return 0;
 }
 
@@ -1290,8 +1307,8 @@ static int apply_core(f25_mesh *m, int npair, const double *d_om, const double *
         TRY(apply_f64(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y, rec, vcf));
         TRY(pml_launch(m, npair, d_ky, (const double2 *)x, (double2 *)y));
     } else if (mode == F25_APPLY_F32) {
-        TRY((dispatch_apply<float, float2, false>(m, d_om, d_ky, npair, (const float2 *)x, (float2 *)y,
-                                                  m->d_blk32, nullptr)));
+        TRY(ensure_vpad(m, npair));
+        TRY(launch_f32(m, d_om, d_ky, npair, (const float2 *)x, (float2 *)y));
         TRY(pml_launch(m, npair, d_ky, (const float2 *)x, (float2 *)y));
     } else {
         if (npair > m->colmax_cap) {
@@ -1304,8 +1321,7 @@ static int apply_core(f25_mesh *m, int npair, const double *d_om, const double *
         hipLaunchKernelGGL(k_colmax, dim3((npair + 63) / 64, gy), dim3(256), 0, m->st, (int64_t)m->g.ndof,
                            npair, (const double2 *)x, m->d_colmax);
         HIPCHK(hipGetLastError());
-        TRY((dispatch_apply<float, double2, true>(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y,
-                                                  m->d_blk_hi, m->d_blk_lo)));
+        TRY(launch_refined(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y));
         TRY(pml_launch(m, npair, d_ky, (const double2 *)x, (double2 *)y));
     }
     HIPCHK(hipEventRecord(m->ev1, m->st));

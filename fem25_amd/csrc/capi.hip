@@ -117,7 +117,11 @@ struct f25_mesh_s {
     float *d_blk_hi = nullptr, *d_blk_lo = nullptr;   // fixed-point split (refined mode)
     unsigned long long *d_colmax = nullptr;           // per-pair max |x| (refined mode)
     int colmax_cap = 0;
+    // element blocks and coefficients that hold the current model: built by the
+    // first call that reads them (the parallelograms' products do not)
+    bool blk_ok = false, blk32_ok = false, vcf_ok = false;
     double *d_dblk = nullptr;   // blocks of a model perturbation (GN products)
+    double *d_drec = nullptr;   // element records of a model perturbation
     double *d_vcf = nullptr;    // d_blk in the coefficient layout of the FP64 product (k_apply_v)
     double *d_dvcf = nullptr;   // d_dblk in that layout
     size_t vcf_cap = 0, dvcf_cap = 0;
@@ -181,8 +185,8 @@ struct f25_mesh_s {
     // FILL_UWAVE_QMESH; built on first use
     struct {
         bool built = false, uw = false;
-        std::vector<int> cptr;
-        int *d_order = nullptr;
+        std::vector<int> cptr, acptr, gcptr;     // all, parallelograms, the others
+        int *d_order = nullptr, *d_aorder = nullptr, *d_gorder = nullptr;
         int *d_lm[4] = {};                       // E in, B out, B in, E out
         unsigned long long *d_first0 = nullptr;  // every row adds
         int *d_brows = nullptr;
@@ -522,7 +526,7 @@ extern "C" int f25_mesh_destroy(f25_mesh *m) {
     if (m->st) (void)hipStreamSynchronize(m->st);
     dfree(m->d_ieng); dfree(m->d_lm); dfree(m->d_first); dfree(m->d_order); dfree(m->d_pml_order); dfree(m->d_err);
     dfree(m->d_xl); dfree(m->d_zl); dfree(m->d_xd); dfree(m->d_zd); dfree(m->d_shl); dfree(m->d_wq); dfree(m->d_t1d);
-    dfree(m->d_taf); dfree(m->d_rec); dfree(m->d_aelem); dfree(m->d_gelem);
+    dfree(m->d_taf); dfree(m->d_rec); dfree(m->d_drec); dfree(m->d_aelem); dfree(m->d_gelem);
     dfree(m->d_aorder); dfree(m->d_gorder);
     dfree(m->d_xq); dfree(m->d_cdom); dfree(m->d_cnp); dfree(m->d_rho); dfree(m->d_lam); dfree(m->d_mu);
     if (m->ag.exec) (void)hipGraphExecDestroy(m->ag.exec);
@@ -534,7 +538,7 @@ extern "C" int f25_mesh_destroy(f25_mesh *m) {
     dfree(m->d_mygrad); dfree(m->d_jcsc); dfree(m->d_icsc); dfree(m->d_dab_pos);
     dfree(m->d_ew);
     dfree(m->d_omky);
-    dfree(m->br.d_order); dfree(m->br.d_first0); dfree(m->br.d_brows); dfree(m->br.d_xz); dfree(m->br.d_comp);
+    dfree(m->br.d_order); dfree(m->br.d_aorder); dfree(m->br.d_gorder); dfree(m->br.d_first0); dfree(m->br.d_brows); dfree(m->br.d_xz); dfree(m->br.d_comp);
     dfree(m->br.d_pw);
     for (auto &q : m->br.d_lm) dfree(q);
     if (m->br.exec) (void)hipGraphExecDestroy(m->br.exec);
@@ -622,6 +626,41 @@ static int run_blocks(f25_mesh *m, const double *rho, const double *lam, const d
 
 static int vcoef(f25_mesh *m, const double *blk, double **vcf);
 
+// The element blocks of the current model (with the FP32 copies), and their
+// coefficient layout for k_apply_v, built on the first use after a model
+// change: a line search's products on parallelograms read neither, and the
+// blocks were most of its time (k_blocks and k_vcoef, 1.6 ms of 1.9 per model
+// and 16 products at 120x61 p4).
+static int ensure_blocks(f25_mesh *m, bool fp32) {
+    if (m->blk_ok && (m->blk32_ok || !fp32)) return 0;
+    const size_t nb = (size_t)m->d.nelem * NBLK * m->tab.nen * m->tab.nen;
+    if (!m->d_blk) TRY(dalloc(&m->d_blk, nb));
+    if (fp32) {
+        if (!m->d_blk32) TRY(dalloc(&m->d_blk32, nb));
+        if (!m->d_blk_hi) TRY(dalloc(&m->d_blk_hi, nb));
+        if (!m->d_blk_lo) TRY(dalloc(&m->d_blk_lo, nb));
+    }
+    TRY(run_blocks(m, m->d_rho, m->d_lam, m->d_mu, m->d_blk, fp32 ? m->d_blk32 : nullptr, fp32 ? m->d_blk_hi : nullptr,
+                   fp32 ? m->d_blk_lo : nullptr));
+    m->blk_ok = true;
+    m->blk32_ok = m->blk32_ok || fp32;
+    return 0;
+}
+
+static int ensure_vcf(f25_mesh *m) {
+    if (m->vcf_ok) return 0;
+    TRY(ensure_blocks(m, false));
+    TRY(vcoef(m, m->d_blk, &m->d_vcf));
+    m->vcf_ok = true;
+    return 0;
+}
+
+// records of the elements for affine.hip from a model at the anchors
+static void element_records(f25_mesh *m, const double *rho, const double *lam, const double *mu, double *rec) {
+    hipLaunchKernelGGL(k_aff_rec, dim3((m->d.nelem + 255) / 256), dim3(256), 0, m->st, m->d.nelem, m->d_ieng, m->d_xl,
+                       m->d_zl, rho, lam, mu, m->d_cdom, rec);
+}
+
 extern "C" int f25_set_model(f25_mesh *m, const double *dens, const double *ecoeff) {
     if (!m || !dens || !ecoeff) FAIL(F25_ERR_ARG, "null argument");
     HIPCHK(hipSetDevice(m->dev));
@@ -644,17 +683,15 @@ extern "C" int f25_set_model(f25_mesh *m, const double *dens, const double *ecoe
     HIPCHK(hipMemcpyAsync(m->d_rho, m->rho.data(), n * 8, hipMemcpyHostToDevice, m->st));
     HIPCHK(hipMemcpyAsync(m->d_lam, m->lam.data(), n * 8, hipMemcpyHostToDevice, m->st));
     HIPCHK(hipMemcpyAsync(m->d_mu, m->mu.data(), n * 8, hipMemcpyHostToDevice, m->st));
-    const size_t nb = (size_t)m->d.nelem * NBLK * m->tab.nen * m->tab.nen;
-    if (!m->d_blk) {
-        TRY(dalloc(&m->d_blk, nb));
-        TRY(dalloc(&m->d_blk32, nb));
-        TRY(dalloc(&m->d_blk_hi, nb));
-        TRY(dalloc(&m->d_blk_lo, nb));
+    element_records(m, m->d_rho, m->d_lam, m->d_mu, m->d_rec);
+    if (m->ngen) {
+        const int64_t np = (int64_t)m->ngen * m->tab.nq;
+        hipLaunchKernelGGL(k_jac_check, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, m->st, m->ngen, m->d_gelem,
+                           m->tab.nq1, m->d_xq, m->d_ieng, m->d_xl, m->d_zl, m->d_err);
     }
-    hipLaunchKernelGGL(k_aff_rec, dim3((m->d.nelem + 255) / 256), dim3(256), 0, m->st, m->d.nelem, m->d_ieng, m->d_xl,
-                       m->d_zl, m->d_rho, m->d_lam, m->d_mu, m->d_cdom, m->d_rec);
-    TRY(run_blocks(m, m->d_rho, m->d_lam, m->d_mu, m->d_blk, m->d_blk32, m->d_blk_hi, m->d_blk_lo));
-    TRY(vcoef(m, m->d_blk, &m->d_vcf));
+    HIPCHK(hipGetLastError());
+    TRY(check_err(m));
+    m->blk_ok = m->blk32_ok = m->vcf_ok = false;
     m->have_model = true;
     m->basis_ok = false;
     m->pa.valid = false;
@@ -736,6 +773,7 @@ static int ensure_basis(f25_mesh *m) {
     TRY(ensure_csr(m));
     TRY(ensure_kinds(m));
     if (m->basis_ok) return 0;
+    TRY(ensure_blocks(m, false));
     const int ndof = m->g.ndof;
     const size_t nz = m->g.irptr[ndof];
     if (!m->d_v0) {
@@ -1005,13 +1043,8 @@ extern "C" int f25_set_apply_tiles(f25_mesh *m, int nrt) {
         m->ag.exec = nullptr;
         m->br.exec = nullptr;
     }
-    const int old = m->apply_nrt;
     m->apply_nrt = nrt;
-    if (m->have_model && apply_nrt(m) != (old ? old : apply_nrt_default(m->tab.nl))) {
-        const int r = vcoef(m, m->d_blk, &m->d_vcf);
-        if (r) return r;
-        HIPCHK(hipStreamSynchronize(m->st));
-    }
+    m->vcf_ok = false;   // the layout depends on the row tiles
     return 0;
 }
 
@@ -1078,7 +1111,17 @@ static int affine_colour(f25_mesh *m, const int *order, int n, const int *lm_in,
 // means the block kernel
 static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt && m->g.ndof < (1 << 27); }
 
-// the launches of the FP64 product (ensure_vpad first), one or two per
+// what the product's launches read: zero rows and sink, and the element
+// blocks of the elements that are not parallelograms
+static int product_ready(f25_mesh *m, int npair, int mode) {
+    TRY(ensure_vpad(m, npair));
+    if (m->disp) return 0;   // every element per omega
+    if (mode == F25_APPLY_F32_REFINED) return ensure_blocks(m, true);
+    if (affine_product(m) && !m->ngen) return 0;
+    return mode == F25_APPLY_F32 ? ensure_blocks(m, true) : ensure_vcf(m);
+}
+
+// the launches of the FP64 product (product_ready first), one or two per
 // colour: the parallelograms by rec (null: as blocks too), the others by vcf
 static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x, double2 *y,
                       const double *rec, const double *vcf) {
@@ -1095,7 +1138,7 @@ static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair
     return 0;
 }
 
-// The FP32 products (ensure_vpad first).  Plain FP32 takes its parallelograms
+// The FP32 products (product_ready first).  Plain FP32 takes its parallelograms
 // through k_apply_af on complex64 vectors: FP64 arithmetic runs at the rate
 // of FP32 arithmetic without packed instructions, and the vectors are what
 // the kernel moves.  The refined product keeps its blocks for every element.
@@ -1119,12 +1162,6 @@ static int launch_refined(f25_mesh *m, const double *om, const double *kv, int n
             TRY((dispatch_apply<float, double2, true>(m, m->d_order + m->cptr[c], m->cptr[c + 1] - m->cptr[c], om, kv,
                                                       npair, x, y, m->d_blk_hi, m->d_blk_lo)));
     return 0;
-}
-
-static int apply_f64(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x, double2 *y,
-                     const double *rec, const double *vcf) {
-    TRY(ensure_vpad(m, npair));
-    return launch_f64(m, om, kv, npair, x, y, rec, vcf);
 }
 
 // ---- elements of the batched product integrated per omega ---------------
@@ -1247,7 +1284,6 @@ static int disp_product(f25_mesh *m, int npair, const double *d_ky, const XT *x,
 // F25_APPLY_GRAPH: capture the launches once per argument set, then replay
 static int apply_f64_graph(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x,
                            double2 *y, const double *rec, const double *vcf) {
-    TRY(ensure_vpad(m, npair));
     auto &G = m->ag;
     const auto &P = m->pa;
     const int nom = (int)P.om.size();
@@ -1304,10 +1340,9 @@ static int apply_core(f25_mesh *m, int npair, const double *d_om, const double *
     } else if (mode == F25_APPLY_F64 && graph)
         TRY(apply_f64_graph(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y, rec, vcf));
     else if (mode == F25_APPLY_F64) {
-        TRY(apply_f64(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y, rec, vcf));
+        TRY(launch_f64(m, d_om, d_ky, npair, (const double2 *)x, (double2 *)y, rec, vcf));
         TRY(pml_launch(m, npair, d_ky, (const double2 *)x, (double2 *)y));
     } else if (mode == F25_APPLY_F32) {
-        TRY(ensure_vpad(m, npair));
         TRY(launch_f32(m, d_om, d_ky, npair, (const float2 *)x, (float2 *)y));
         TRY(pml_launch(m, npair, d_ky, (const float2 *)x, (float2 *)y));
     } else {
@@ -1349,6 +1384,7 @@ extern "C" int f25_apply_batch_dev(f25_mesh *m, int npair, const double *omega, 
     if (!m->have_model) FAIL(F25_ERR_STATE, "f25_set_model has not been called");
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
+    TRY(product_ready(m, npair, mode & ~F25_APPLY_GRAPH));
     return apply_core(m, npair, m->d_omky, m->d_omky + m->omky_cap, mode, x, y, m->d_rec, m->d_vcf, omega);
 }
 
@@ -1359,6 +1395,7 @@ extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omeg
     if (!m->have_model) FAIL(F25_ERR_STATE, "f25_set_model has not been called");
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
+    TRY(product_ready(m, npair, F25_APPLY_F64));
     TRY(apply_core(m, npair, m->d_omky, m->d_omky + m->omky_cap, F25_APPLY_F64, u, r, m->d_rec, m->d_vcf, omega));
     const int gy = (int)std::min<int64_t>(256, std::max<int64_t>(1, m->g.ndof / 256));
     double *part = nullptr, *sums = nullptr;
@@ -1434,7 +1471,11 @@ static int bielak_prepare(f25_mesh *m) {
     std::vector<int> brows;
     for (int d = 0; d < m->g.ndof; ++d)
         if (isb[d]) brows.push_back(d);
+    std::vector<int> ao, go;
+    split_order(m, ord, ptr, ao, B.acptr, go, B.gcptr);
     TRY(upload(&B.d_order, ord.data(), ord.size(), m->st));
+    TRY(upload(&B.d_aorder, ao.data(), ao.size(), m->st));
+    TRY(upload(&B.d_gorder, go.data(), go.size(), m->st));
     for (int k = 0; k < 4; ++k) TRY(upload(&B.d_lm[k], lmv[k].data(), lmv[k].size(), m->st));
     TRY(dalloc(&B.d_first0, (size_t)nelem));
     fill_async(B.d_first0, (size_t)nelem, 0ull, m->st);
@@ -1447,28 +1488,23 @@ static int bielak_prepare(f25_mesh *m) {
 }
 
 template <int NL, int NRT>
-static int launch_ring(f25_mesh *m, int pass, const double *om, const double *kv, int npair, const double2 *x,
-                       double2 *y) {
+static int launch_ring(f25_mesh *m, int pass, const int *order, int n, const double *om, const double *kv, int npair,
+                       const double2 *x, double2 *y) {
     auto &B = m->br;
     const double2 *zpad = reinterpret_cast<const double2 *>(m->d_vpad);
     double2 *sink = reinterpret_cast<double2 *>(m->d_vpad) + m->vpad_cap;
-    for (size_t c = 0; c + 1 < B.cptr.size(); ++c) {
-        const int n = B.cptr[c + 1] - B.cptr[c];
-        if (!n) continue;
-        const size_t nwg = apply_v_grid<NL, NRT>(n, npair);
-        if (nwg > 0x7fffffff) FAIL(F25_ERR_ARG, "too many pairs for one launch");
-        hipLaunchKernelGGL((k_apply_v<NL, NRT>), dim3((unsigned)nwg), dim3(VShape<NL, NRT>::NT), 0, m->st,
-                           B.d_order + B.cptr[c], n, m->d_vcf, B.d_lm[2 * pass], B.d_lm[2 * pass + 1], B.d_first0,
-                           npair, om, kv, x, y, zpad, sink);
-    }
+    const size_t nwg = apply_v_grid<NL, NRT>(n, npair);
+    if (nwg > 0x7fffffff) FAIL(F25_ERR_ARG, "too many pairs for one launch");
+    hipLaunchKernelGGL((k_apply_v<NL, NRT>), dim3((unsigned)nwg), dim3(VShape<NL, NRT>::NT), 0, m->st, order, n,
+                       m->d_vcf, B.d_lm[2 * pass], B.d_lm[2 * pass + 1], B.d_first0, npair, om, kv, x, y, zpad, sink);
     HIPCHK(hipGetLastError());
     return 0;
 }
 
-static int ring_pass(f25_mesh *m, int pass, const double *om, const double *kv, int npair, const double2 *x,
-                     double2 *y) {
+static int ring_blocks(f25_mesh *m, int pass, const int *order, int n, const double *om, const double *kv, int npair,
+                       const double2 *x, double2 *y) {
     switch (m->tab.nl * 8 + apply_nrt(m)) {
-#define F25_RV(N, T) case N * 8 + T: return launch_ring<N, T>(m, pass, om, kv, npair, x, y);
+#define F25_RV(N, T) case N * 8 + T: return launch_ring<N, T>(m, pass, order, n, om, kv, npair, x, y);
         F25_RV(3, 1) F25_RV(3, 2) F25_RV(4, 1) F25_RV(4, 2) F25_RV(5, 1) F25_RV(5, 2) F25_RV(5, 3)
         F25_RV(6, 2) F25_RV(6, 3) F25_RV(6, 4) F25_RV(7, 2) F25_RV(7, 3) F25_RV(7, 4)
 #undef F25_RV
@@ -1476,7 +1512,29 @@ static int ring_pass(f25_mesh *m, int pass, const double *om, const double *kv, 
     FAIL(F25_ERR_ARG, "unsupported order");
 }
 
-// the effective force's launches (bielak_prepare and ensure_vpad first):
+static int ring_pass(f25_mesh *m, int pass, const double *om, const double *kv, int npair, const double2 *x,
+                     double2 *y) {
+    auto &B = m->br;
+    const bool aff = affine_product(m);
+    for (size_t c = 0; c + 1 < B.cptr.size(); ++c) {
+        const std::vector<int> &gp = aff ? B.gcptr : B.cptr;
+        if (aff && B.acptr[c + 1] > B.acptr[c])
+            TRY(affine_colour(m, B.d_aorder + B.acptr[c], B.acptr[c + 1] - B.acptr[c], B.d_lm[2 * pass],
+                              B.d_lm[2 * pass + 1], B.d_first0, m->d_rec, om, kv, npair, x, y));
+        if (gp[c + 1] > gp[c])
+            TRY(ring_blocks(m, pass, (aff ? B.d_gorder : B.d_order) + gp[c], gp[c + 1] - gp[c], om, kv, npair, x, y));
+    }
+    return 0;
+}
+
+// what the ring's launches read (bielak_prepare first)
+static int ring_ready(f25_mesh *m, int npair) {
+    TRY(ensure_vpad(m, npair));
+    const std::vector<int> &gp = affine_product(m) ? m->br.gcptr : m->br.cptr;
+    return gp.back() ? ensure_vcf(m) : 0;
+}
+
+// the effective force's launches (bielak_prepare and ring_ready first):
 // zero fill, pass 0, 'B' rows negated, pass 1; no host synchronisation
 static int peff_launches(f25_mesh *m, int npair, const double *om, const double *kv, const double2 *u,
                          double2 *y) {
@@ -1505,7 +1563,7 @@ extern "C" int f25_peff_batch_dev(f25_mesh *m, int npair, const double *omega, c
     HIPCHK(hipSetDevice(m->dev));
     TRY(bielak_prepare(m));
     TRY(stage_omky(m, npair, omega, ky));
-    TRY(ensure_vpad(m, npair));
+    TRY(ring_ready(m, npair));
     const double *om = m->d_omky, *kv = m->d_omky + m->omky_cap;
     HIPCHK(hipEventRecord(m->ev0, m->st));
     TRY(peff_launches(m, npair, om, kv, (const double2 *)ue_dev, (double2 *)peff_dev));
@@ -1625,7 +1683,7 @@ extern "C" int f25_bielak_rhs_dev(f25_mesh *m, int npair, const double *omega, c
         B.exec = nullptr;
     }
     TRY(stage_omky(m, npair, omega, ky));
-    TRY(ensure_vpad(m, npair));
+    TRY(ring_ready(m, npair));
     TRY(uwave_params(m, npair, kappax, kappaz, baz, aoi));
     const double *om = m->d_omky, *kv = m->d_omky + m->omky_cap;
     // staging buffers may have moved since the capture
@@ -3153,9 +3211,18 @@ extern "C" int f25_gn_fv(f25_mesh *m, int ntrip, const double *omega, const doub
     TRY(upload(&d_r, dr.data(), n, m->st));
     TRY(upload(&d_l, dl.data(), n, m->st));
     TRY(upload(&d_m, dm.data(), n, m->st));
-    const size_t nb = (size_t)m->d.nelem * NBLK * m->tab.nen * m->tab.nen;
-    if (!m->d_dblk) TRY(dalloc(&m->d_dblk, nb));
-    int r = run_blocks(m, d_r, d_l, d_m, m->d_dblk, nullptr, nullptr, nullptr);
+    // the perturbation's records, and its blocks for elements of general shape
+    const bool aff = affine_product(m), blocks = !aff || m->ngen;
+    int r = 0;
+    if (aff) {
+        if (!m->d_drec) r = dalloc(&m->d_drec, (size_t)m->d.nelem * AFR);
+        if (!r) element_records(m, d_r, d_l, d_m, m->d_drec);
+    }
+    if (!r && blocks) {
+        if (!m->d_dblk) r = dalloc(&m->d_dblk, (size_t)m->d.nelem * NBLK * m->tab.nen * m->tab.nen);
+        if (!r) r = run_blocks(m, d_r, d_l, d_m, m->d_dblk, nullptr, nullptr, nullptr);
+    }
+    if (!r && hipStreamSynchronize(m->st) != hipSuccess) r = F25_ERR_HIP;
     dfree(d_r); dfree(d_l); dfree(d_m);
     if (r) return r;
     const size_t nn = (size_t)m->g.ndof * ntrip;
@@ -3168,8 +3235,9 @@ extern "C" int f25_gn_fv(f25_mesh *m, int ntrip, const double *omega, const doub
     hipError_t e = hipMemcpyAsync(a, u, nn * 16, hipMemcpyHostToDevice, m->st);
     r = (e == hipSuccess) ? 0 : F25_ERR_HIP;
     if (!r) r = transpose_dev(m->st, a, b, ntrip, m->g.ndof);
-    if (!r) r = vcoef(m, m->d_dblk, &m->d_dvcf);
-    if (!r) r = apply_core(m, ntrip, d_om, d_ky, F25_APPLY_F64, b, a, nullptr, m->d_dvcf, nullptr);
+    if (!r && blocks) r = vcoef(m, m->d_dblk, &m->d_dvcf);
+    if (!r) r = ensure_vpad(m, ntrip);
+    if (!r) r = apply_core(m, ntrip, d_om, d_ky, F25_APPLY_F64, b, a, aff ? m->d_drec : nullptr, m->d_dvcf, nullptr);
     if (!r) r = transpose_dev(m->st, a, b, m->g.ndof, ntrip);
     if (!r) {
         e = hipMemcpyAsync(out, b, nn * 16, hipMemcpyDeviceToHost, m->st);

@@ -56,6 +56,18 @@ __device__ inline int geo_at(double xi, double eta, const int *ie, const double 
 }
 
 // ---------------------------------------------------------------------------
+// Jacobian check of n elements (elems) at their quadrature points: err = 2
+// where it is undefined or negative.
+__global__ void k_jac_check(int n, const int *__restrict__ elems, int nq1, const double *__restrict__ xq,
+                            const int *__restrict__ ieng, const double *__restrict__ xl,
+                            const double *__restrict__ zl, int *__restrict__ err) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int nq = nq1 * nq1, k = (int)(i / nq), q = (int)(i % nq);
+    if (k >= n) return;
+    Geo g;
+    if (geo_at(xq[q % nq1], xq[q / nq1], ieng + 4 * elems[k], xl, zl, g)) *err = 2;
+}
+
 // Element blocks.  One workgroup per element; every thread owns up to PPT
 // (a, b) node pairs and accumulates the nine blocks over quadrature points
 // staged in LDS chunk by chunk.

@@ -99,8 +99,9 @@ int f25_mesh_sizes(f25_mesh *m, int64_t sizes[6]);
  * NULL): IEN(NEN,NELEM), LM(3,NEN,NELEM), IRPTR(NDOF+1), JCPTR(NZ), CNP(NDOF). */
 int f25_mesh_graph(f25_mesh *m, int *ien, int *lm, int *irptr, int *jcptr, char *cnp);
 /* DENS(NNPG) kg/m^3 and ECOEFF(NNPG,2) = (lambda, mu) Pa.  Recomputes the
- * element blocks on the device; a call with the model already set returns
- * at once (so drop-in shims may call it before every product). */
+ * element records on the device (the element blocks are rebuilt by the first
+ * call that reads them); a call with the model already set returns at once
+ * (so drop-in shims may call it before every product). */
 int f25_set_model(f25_mesh *m, const double *dens, const double *ecoeff);
 
 /* Quality factors QP(NNPG), QS(NNPG) at the anchors and the reference

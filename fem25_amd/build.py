@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libfem25hip.so")
 SRCS = [os.path.join(HERE, "csrc", f) for f in ("host_setup.cpp", "capi.hip")]
-DEPS = SRCS + [os.path.join(HERE, "csrc", f) for f in ("kernels.hip", "affine.hip", "f25_internal.h")] + [
+DEPS = SRCS + [os.path.join(HERE, "csrc", f) for f in ("kernels.hip", "affine.hip", "pml.hip", "f25_internal.h")] + [
     os.path.join(ROOT, "include", "fem25hip.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -15,6 +15,7 @@
 #include "f25_internal.h"
 #include "kernels.hip"
 #include "affine.hip"
+#include "pml.hip"
 
 using namespace f25;
 using namespace f25k;
@@ -151,6 +152,9 @@ struct f25_mesh_s {
         int *d_grp = nullptr, *d_gpair = nullptr;
         int grp_cap = 0, gpair_cap = 0, ngrp = 0;
     } pa;
+    // CSR positions of the values of the elements integrated per call
+    // (k_pml_pos): the PML elements', and every element's (dispersive medium)
+    int *d_pos[2] = {};
     int apply_nrt = 0;          // row tiles of k_apply_v (0: the order's default)
     double *d_vpad = nullptr;   // k_apply_v: vpad_cap zero double2, then vpad_cap double2 of store sink
     int vpad_cap = 0;
@@ -542,6 +546,7 @@ extern "C" int f25_mesh_destroy(f25_mesh *m) {
     dfree(m->br.d_pw);
     for (auto &q : m->br.d_lm) dfree(q);
     if (m->br.exec) (void)hipGraphExecDestroy(m->br.exec);
+    dfree(m->d_pos[0]); dfree(m->d_pos[1]);
     dfree(m->pa.d_mats); dfree(m->pa.d_om); dfree(m->pa.d_grp); dfree(m->pa.d_gpair);
     if (m->blas) (void)rocblas_destroy_handle(m->blas);
     if (m->ev0) (void)hipEventDestroy(m->ev0);
@@ -806,10 +811,46 @@ static int ensure_basis(f25_mesh *m) {
     return 0;
 }
 
+// CSR positions for the elements integrated per call, built once per mesh
+// (and again for every element when a medium first is dispersive)
+static int ensure_pml_pos(f25_mesh *m) {
+    const int k = m->disp ? 1 : 0;
+    const size_t n = m->disp ? m->order.size() : m->pml_order.size(), nee = 3 * m->tab.nen;
+    if (m->d_pos[k] || !n) return 0;
+    int *d = nullptr;
+    TRY(dalloc(&d, n * nee * nee));
+    hipLaunchKernelGGL(k_pml_pos, dim3((unsigned)n), dim3(256), 0, m->st, (int)nee, m->disp ? m->d_order : m->d_pml_order,
+                       m->d_lm, m->d_irptr, m->d_jcptr, d, m->d_err);
+    const hipError_t e = hipGetLastError();
+    const int r = e == hipSuccess ? check_err(m) : F25_ERR_HIP;
+    if (r) {
+        if (e != hipSuccess) g_err = hipGetErrorString(e);
+        dfree(d);
+        return r;
+    }
+    m->d_pos[k] = d;
+    return 0;
+}
+
+// the elements order[o .. o + n) of one colour, added into out
+template <int NL, typename CT>
+static int pml_add(f25_mesh *m, int o, int n, const PmlPar &p, CT *out) {
+    typedef PmlSf<NL> S;
+    auto kern = k_pml_sf<NL, false, CT>;
+    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
+    hipLaunchKernelGGL(kern, dim3(n, 6), dim3(S::NT), S::lds, m->st, o, 1, (m->disp ? m->d_order : m->d_pml_order) + o,
+                       (const double *)nullptr, m->d_t1d, m->d_wq, m->d_xq, m->d_ieng, m->d_xl, m->d_zl, m->d_xd,
+                       m->d_zd, m->d_cdom, m->d_rho, m->d_lam, m->d_mu, m->disp ? m->d_qp : nullptr,
+                       m->disp ? m->d_qs : nullptr, p, m->d_lm, m->d_irptr, m->d_pos[m->disp ? 1 : 0], out, m->d_err);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 template <typename CT>
 static int asmble_impl(f25_mesh *m, char cftype, double freq, double py, CT *out) {
     const double omega = 6.2831853071795862 * freq, kv = omega * py;
     const int ndof = m->g.ndof;
+    TRY(ensure_pml_pos(m));
     HIPCHK(hipEventRecord(m->ev0, m->st));
     // dispersive media: every element is integrated per call (KMDAMP/CMDAMP);
     // otherwise the frequency-independent basis gives the non-PML part
@@ -821,7 +862,6 @@ static int asmble_impl(f25_mesh *m, char cftype, double freq, double py, CT *out
                            (int64_t)m->g.irptr[ndof], m->d_cbase, m->d_kind, m->d_v0, m->d_v1, m->d_v2, omega, kv,
                            out);
     const std::vector<int> &cp = disp ? m->cptr : m->pml_cptr;
-    const int *ord = disp ? m->d_order : m->d_pml_order;
     if (disp || !m->pml_order.empty()) {
         PmlPar p;
         p.omega = omega;
@@ -832,16 +872,17 @@ static int asmble_impl(f25_mesh *m, char cftype, double freq, double py, CT *out
         p.rcoeff = pp[0]; p.dmax = pp[1]; p.kappa = pp[2]; p.fcent = pp[3];
         p.freq = freq;
         p.freq0 = m->freq0;
-        const int nen = m->tab.nen;
-        size_t lds = (8 * 9 + 3 * 8 * nen) * sizeof(double);
         for (size_t c = 0; c + 1 < cp.size(); ++c) {
-            int n = cp[c + 1] - cp[c];
+            const int n = cp[c + 1] - cp[c];
             if (!n) continue;
-            hipLaunchKernelGGL((k_pml<CT>), dim3(n), dim3(256), lds, m->st, nen, m->tab.nq1, n,
-                               ord + cp[c], m->d_shl, m->d_wq, m->d_xq, m->d_ieng,
-                               m->d_xl, m->d_zl, m->d_xd, m->d_zd, m->d_cdom, m->d_rho, m->d_lam, m->d_mu,
-                               disp ? m->d_qp : nullptr, disp ? m->d_qs : nullptr, m->d_lm,
-                               m->d_irptr, m->d_jcptr, p, out, m->d_err);
+            switch (m->tab.nl) {
+                case 3: TRY((pml_add<3, CT>(m, cp[c], n, p, out))); break;
+                case 4: TRY((pml_add<4, CT>(m, cp[c], n, p, out))); break;
+                case 5: TRY((pml_add<5, CT>(m, cp[c], n, p, out))); break;
+                case 6: TRY((pml_add<6, CT>(m, cp[c], n, p, out))); break;
+                case 7: TRY((pml_add<7, CT>(m, cp[c], n, p, out))); break;
+                default: FAIL(F25_ERR_ARG, "unsupported order");
+            }
         }
     }
     HIPCHK(hipEventRecord(m->ev1, m->st));

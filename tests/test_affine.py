@@ -100,3 +100,23 @@ def test_product(p, npml):
     mi.apply_batch_dev(om, ky, x32, y32, _lib.F25_APPLY_F32)
     y32 = y32.cpu().numpy().T
     assert all(err(y32[b], ref[b]) < 2e-6 for b in probe)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("disp", [False, True])
+@pytest.mark.parametrize("p", [2, 3, 4, 5, 6])
+def test_assembled_with_elements_per_omega(p, disp):
+    """PML elements, and in a dispersive medium every element, integrated per
+    call, some of general shape (both geometries of the element matrices)."""
+    from fem25_amd.api import MeshInfo
+    m, mod, pml, g = case(p, 2)
+    if disp:
+        mod = cf.with_attenuation(mod, 120.0, 60.0, 1.0)
+    mi = MeshInfo(m, pml)
+    mi.set_model(mod)
+    for f, py in ((0.05, 0.0), (0.08, 9e-5)):
+        ref = oracle.asmble_z(m, mod, g, f, py, pml)
+        assert err(mi.asmble(b"B", f, py, complex128=True), ref) < 1e-13
+        got = mi.asmble(b"B", f, py)
+        assert np.max(np.abs(got - ref)) < 1e-6 * np.max(np.abs(ref))
+    mi.close()

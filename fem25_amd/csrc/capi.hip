@@ -113,6 +113,7 @@ struct f25_mesh_s {
     std::vector<int> acptr, gcptr;
     char *d_cdom = nullptr, *d_cnp = nullptr;
     double *d_rho = nullptr, *d_lam = nullptr, *d_mu = nullptr;
+    double2 *d_vps = nullptr;   // (Vp, Vs) at the anchors
     double *d_blk = nullptr;
     float *d_blk32 = nullptr;                          // fl32 of the blocks (FP32 mode)
     float *d_blk_hi = nullptr, *d_blk_lo = nullptr;   // fixed-point split (refined mode)
@@ -532,7 +533,7 @@ extern "C" int f25_mesh_destroy(f25_mesh *m) {
     dfree(m->d_xl); dfree(m->d_zl); dfree(m->d_xd); dfree(m->d_zd); dfree(m->d_shl); dfree(m->d_wq); dfree(m->d_t1d);
     dfree(m->d_taf); dfree(m->d_rec); dfree(m->d_drec); dfree(m->d_aelem); dfree(m->d_gelem);
     dfree(m->d_aorder); dfree(m->d_gorder);
-    dfree(m->d_xq); dfree(m->d_cdom); dfree(m->d_cnp); dfree(m->d_rho); dfree(m->d_lam); dfree(m->d_mu);
+    dfree(m->d_xq); dfree(m->d_cdom); dfree(m->d_cnp); dfree(m->d_rho); dfree(m->d_lam); dfree(m->d_mu); dfree(m->d_vps);
     if (m->ag.exec) (void)hipGraphExecDestroy(m->ag.exec);
     dfree(m->d_vcf); dfree(m->d_dvcf); dfree(m->d_vpad);
     dfree(m->d_blk); dfree(m->d_blk32); dfree(m->d_blk_hi); dfree(m->d_blk_lo); dfree(m->d_colmax); dfree(m->d_dblk); dfree(m->d_irptr);
@@ -684,11 +685,13 @@ extern "C" int f25_set_model(f25_mesh *m, const double *dens, const double *ecoe
         TRY(dalloc(&m->d_rho, n));
         TRY(dalloc(&m->d_lam, n));
         TRY(dalloc(&m->d_mu, n));
+        TRY(dalloc(&m->d_vps, n));
     }
     HIPCHK(hipMemcpyAsync(m->d_rho, m->rho.data(), n * 8, hipMemcpyHostToDevice, m->st));
     HIPCHK(hipMemcpyAsync(m->d_lam, m->lam.data(), n * 8, hipMemcpyHostToDevice, m->st));
     HIPCHK(hipMemcpyAsync(m->d_mu, m->mu.data(), n * 8, hipMemcpyHostToDevice, m->st));
     element_records(m, m->d_rho, m->d_lam, m->d_mu, m->d_rec);
+    hipLaunchKernelGGL(k_anchor_vel, dim3((n + 255) / 256), dim3(256), 0, m->st, n, m->d_rho, m->d_lam, m->d_mu, m->d_vps);
     if (m->ngen) {
         const int64_t np = (int64_t)m->ngen * m->tab.nq;
         hipLaunchKernelGGL(k_jac_check, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, m->st, m->ngen, m->d_gelem,
@@ -840,7 +843,7 @@ static int pml_add(f25_mesh *m, int o, int n, const PmlPar &p, CT *out) {
     HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
     hipLaunchKernelGGL(kern, dim3(n, 6), dim3(S::NT), S::lds, m->st, o, 1, (m->disp ? m->d_order : m->d_pml_order) + o,
                        (const double *)nullptr, m->d_t1d, m->d_wq, m->d_xq, m->d_ieng, m->d_xl, m->d_zl, m->d_xd,
-                       m->d_zd, m->d_cdom, m->d_rho, m->d_lam, m->d_mu, m->disp ? m->d_qp : nullptr,
+                       m->d_zd, m->d_cdom, m->d_rho, m->d_lam, m->d_mu, m->d_vps, m->disp ? m->d_qp : nullptr,
                        m->disp ? m->d_qs : nullptr, p, m->d_lm, m->d_irptr, m->d_pos[m->disp ? 1 : 0], out, m->d_err);
     HIPCHK(hipGetLastError());
     return 0;
@@ -929,10 +932,10 @@ extern "C" int f25_csr_apply_dev(f25_mesh *m, int precision, const void *s, cons
     const int ndof = m->g.ndof;
     HIPCHK(hipEventRecord(m->ev0, m->st));
     if (precision == F25_C128)
-        hipLaunchKernelGGL((k_spmv<double2, double>), dim3((ndof + 3) / 4), dim3(256), 0, m->st, ndof,
+        hipLaunchKernelGGL(k_spmv<double2>, dim3((ndof + 15) / 16), dim3(256), 0, m->st, ndof,
                            m->d_irptr, m->d_jcptr, (const double2 *)s, (const double2 *)x, (double2 *)y);
     else if (precision == F25_C64)
-        hipLaunchKernelGGL((k_spmv<float2, float>), dim3((ndof + 3) / 4), dim3(256), 0, m->st, ndof,
+        hipLaunchKernelGGL(k_spmv<float2>, dim3((ndof + 15) / 16), dim3(256), 0, m->st, ndof,
                            m->d_irptr, m->d_jcptr, (const float2 *)s, (const float2 *)x, (float2 *)y);
     else
         FAIL(F25_ERR_ARG, "bad precision");

@@ -24,9 +24,10 @@ enum { PB_11 = 0, PB_22, PB_33, PB_13, PB_12, PB_23, PB_M, PB_L2, NPB };
 template <int NL>
 struct PmlSf {
     static constexpr int N1 = NL, Q1 = 2 * NL + 3, Q = Q1 * Q1, NEN = NL * NL, NEE = 3 * NEN;
-    static constexpr int NT = NL <= 5 ? 128 : (NL == 6 ? 256 : 384);   // N1^3 threads in the last stage
+    // threads: the Q points and the N1^3 items of the last stage in one or two rounds
+    static constexpr int NT = NL <= 4 ? 128 : (NL == 5 ? 192 : (NL == 6 ? 256 : 384));
     static constexpr int NG = N1 * N1 * Q1;
-    static constexpr size_t lds = (size_t)(4 * Q + 4 * NG) * sizeof(double2) + 2 * N1 * Q1 * sizeof(double);
+    static constexpr size_t lds = (size_t)(4 * Q + 4 * NG) * sizeof(double2) + (2 * N1 * Q1 + NEE) * sizeof(double);
 };
 
 // Moduli L, M, density R (all times the quadrature weight and det J), stretch
@@ -37,7 +38,7 @@ __device__ inline PmlPoint pml_at(int e, int ix, int iz, const double *__restric
                                   const double *__restrict__ zl, const double *__restrict__ xd,
                                   const double *__restrict__ zd, bool pml, const double *__restrict__ rho,
                                   const double *__restrict__ lam, const double *__restrict__ mu,
-                                  const double *__restrict__ qp, const double *__restrict__ qs, const PmlPar &par,
+                                  const double2 *__restrict__ vps, const double *__restrict__ qp, const double *__restrict__ qs, const PmlPar &par,
                                   int *__restrict__ err) {
     const int *ie = ieng + 4 * e;
     Geo g;
@@ -58,9 +59,10 @@ __device__ inline PmlPoint pml_at(int e, int ix, int iz, const double *__restric
             xdep += g.sf[k] * xd[gi];
             zdep += g.sf[k] * zd[gi];
         }
-        vel += g.sf[k] * sqrt((lam[gi] + 2.0 * mu[gi]) / rho[gi]);
+        const double2 v = vps[gi];
+        vel += g.sf[k] * v.x;
         if (qp) {
-            vsv += g.sf[k] * sqrt(mu[gi] / rho[gi]);
+            vsv += g.sf[k] * v.y;
             qpv += g.sf[k] * qp[gi];
             qsv += g.sf[k] * qs[gi];
         }
@@ -123,6 +125,13 @@ __device__ inline void pml_coef(int kb, const PmlPoint &p, double k, double w2, 
     }
 }
 
+// (Vp, Vs) at the anchors, the velocities pml_at interpolates
+__global__ void k_anchor_vel(int n, const double *__restrict__ rho, const double *__restrict__ lam,
+                             const double *__restrict__ mu, double2 *__restrict__ vps) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) vps[i] = make_double2(sqrt((lam[i] + 2.0 * mu[i]) / rho[i]), sqrt(mu[i] / rho[i]));
+}
+
 // Positions of the element rows' and columns' values in CSR order, relative
 // to the row's start, -1 where a DOF is fixed: pos[slot][row][col].  Built
 // once per list of elements; a pair missing from the pattern sets err = 3.
@@ -150,9 +159,13 @@ __global__ void k_pml_pos(int nee, const int *__restrict__ order, const int *__r
 // elements share a value).
 //
 // Bound by latency: a few hundred workgroups a colour, each a chain of four
-// short stages.  Measured on MI355X against the direct sums, one workgroup
-// per element, geometry per node and a search of the pattern per value:
-// PML_FIGURES
+// short stages; the values it adds to are loaded before the last one.
+// Measured on MI355X per colour against the direct sums (one workgroup per
+// element, geometry per node, a search of the pattern per value): 198 PML
+// elements at p4, COMPLEX*8, 445 -> 63 -> about 30 us; 528 dispersive
+// elements at p4, COMPLEX*16, 825 -> 136 -> about 65 us (the second step:
+// velocities per anchor, loads ahead of the sums, loops over the points not
+// unrolled, 122 registers instead of 432).
 template <int NL, bool SPLIT, typename CT>
 __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
         int slot0, int nom, const int *__restrict__ order, const double *__restrict__ omf,
@@ -160,7 +173,7 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
         const int *__restrict__ ieng, const double *__restrict__ xl, const double *__restrict__ zl,
         const double *__restrict__ xd, const double *__restrict__ zd, const char *__restrict__ cdom,
         const double *__restrict__ rho, const double *__restrict__ lam, const double *__restrict__ mu,
-        const double *__restrict__ qp, const double *__restrict__ qs, PmlPar par, const int *__restrict__ lm,
+        const double2 *__restrict__ vps, const double *__restrict__ qp, const double *__restrict__ qs, PmlPar par, const int *__restrict__ lm,
         const int64_t *__restrict__ irptr, const int *__restrict__ pos, CT *__restrict__ out, int *__restrict__ err) {
     typedef PmlSf<NL> S;
     constexpr int N1 = S::N1, Q1 = S::Q1, Q = S::Q, NEN = S::NEN, NEE = S::NEE, NT = S::NT, NG = S::NG;
@@ -168,6 +181,7 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
     double2 *sC = reinterpret_cast<double2 *>(sm);   // [4][Q]
     double2 *sG = sC + 4 * Q;                        // [4][eta][ai][bi]
     double *sv = reinterpret_cast<double *>(sG + 4 * NG), *sd = sv + N1 * Q1;   // v, v' [q][i]
+    int64_t *sr = reinterpret_cast<int64_t *>(sd + N1 * Q1);                     // the rows' starts in CSR order
     const int e = order[blockIdx.x], kb = blockIdx.y, tid = threadIdx.x;
     if constexpr (SPLIT) {
         par.omega = omf[blockIdx.z];
@@ -178,10 +192,15 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
         sv[i] = t1d[(i % N1) * Q1 + i / N1];
         sd[i] = t1d[(N1 + i % N1) * Q1 + i / N1];
     }
+    if constexpr (!SPLIT)
+        for (int i = tid; i < NEE; i += NT) {
+            const int d = lm[(size_t)e * NEE + i];
+            sr[i] = d >= 0 ? irptr[d] : 0;
+        }
     const bool pml = cdom[e] == 'A';
     for (int q = tid; q < Q; q += NT) {
         double2 c[4];
-        pml_coef(kb, pml_at(e, q % Q1, q / Q1, wq, xq, ieng, xl, zl, xd, zd, pml, rho, lam, mu, qp, qs, par, err),
+        pml_coef(kb, pml_at(e, q % Q1, q / Q1, wq, xq, ieng, xl, zl, xd, zd, pml, rho, lam, mu, vps, qp, qs, par, err),
                  par.kv, par.omega * par.omega, c);
 #pragma unroll
         for (int k = 0; k < 4; ++k) sC[k * Q + q] = c[k];
@@ -196,6 +215,7 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
         for (int k = 0; k < 4; ++k) g[k] = make_double2(0.0, 0.0);
         const double2 *C = sC + qe * Q1;
         if (kb <= PB_33) {
+#pragma unroll 2
             for (int x = 0; x < Q1; ++x) {
                 const double va = sv[x * N1 + ai], vb = sv[x * N1 + bi], da = sd[x * N1 + ai], db = sd[x * N1 + bi];
                 cfma(g[0], da * db, C[x]);
@@ -205,6 +225,7 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
                 cfma(g[3], va * vb, C[2 * Q + x]);
             }
         } else if (kb == PB_13) {
+#pragma unroll 2
             for (int x = 0; x < Q1; ++x) {
                 const double va = sv[x * N1 + ai], vb = sv[x * N1 + bi], da = sd[x * N1 + ai], db = sd[x * N1 + bi];
                 cfma(g[0], da * db, C[x]);
@@ -213,6 +234,7 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
                 cfma(g[3], va * vb, C[3 * Q + x]);
             }
         } else if (kb <= PB_23) {
+#pragma unroll 2
             for (int x = 0; x < Q1; ++x) {
                 const double va = sv[x * N1 + ai], vb = sv[x * N1 + bi], da = sd[x * N1 + ai], db = sd[x * N1 + bi];
                 cfma(g[0], da * vb, C[x]);
@@ -232,9 +254,35 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
     const int cj = kb == PB_11 ? 0 : (kb == PB_22 || kb == PB_12 ? 1 : 2);
     for (int it = tid; it < N1 * N1 * N1; it += NT) {
         const int bi = it % N1, ai = (it / N1) % N1, aj = it / (N1 * N1), a = aj * N1 + ai;
+        const int ra = 3 * a + ci;
+        // the values this thread adds to, loaded before the sums (for a fixed
+        // row or column the element's first value of the row start: not stored)
+        [[maybe_unused]] CT *po[N1], *pt[N1];
+        [[maybe_unused]] CT vo[N1], vt[N1];
+        [[maybe_unused]] bool ok[N1];
+        if constexpr (!SPLIT) {
+            const int *P = pos + (size_t)(slot0 + blockIdx.x) * NEE * NEE;
+            int p[N1], t[N1];
+#pragma unroll
+            for (int j = 0; j < N1; ++j) {
+                const int cb = 3 * (j * N1 + bi) + cj;
+                p[j] = P[ra * NEE + cb];
+                t[j] = P[cb * NEE + ra];
+            }
+#pragma unroll
+            for (int j = 0; j < N1; ++j) {
+                const int cb = 3 * (j * N1 + bi) + cj;
+                ok[j] = p[j] >= 0;
+                po[j] = out + sr[ra] + (ok[j] ? p[j] : 0);
+                pt[j] = out + sr[cb] + (ok[j] ? t[j] : 0);
+                vo[j] = *po[j];
+                if (ci != cj) vt[j] = *pt[j];
+            }
+        }
         double2 s[N1];
 #pragma unroll
         for (int j = 0; j < N1; ++j) s[j] = make_double2(0.0, 0.0);
+#pragma unroll 1
         for (int y = 0; y < Q1; ++y) {
             const double2 *g = sG + (y * N1 + ai) * N1 + bi;
             const double va = sv[y * N1 + aj], da = sd[y * N1 + aj];
@@ -252,21 +300,17 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
 #pragma unroll
             for (int j = 0; j < N1; ++j) o[j * N1] = CT{s[j].x, s[j].y};
         } else {
-            const int *L = lm + (size_t)e * NEE, *P = pos + (size_t)(slot0 + blockIdx.x) * NEE * NEE;
-            const int ra = 3 * a + ci;
             const double sg = kb == PB_13 ? 1.0 : -1.0;
 #pragma unroll
             for (int j = 0; j < N1; ++j) {
-                const int cb = 3 * (j * N1 + bi) + cj;
-                const int p = P[ra * NEE + cb];
-                if (p < 0) continue;
-                CT &o = out[irptr[L[ra]] + p];
-                o.x += s[j].x;
-                o.y += s[j].y;
+                if (!ok[j]) continue;
+                vo[j].x += s[j].x;
+                vo[j].y += s[j].y;
+                *po[j] = vo[j];
                 if (ci == cj) continue;
-                CT &t = out[irptr[L[cb]] + P[cb * NEE + ra]];
-                t.x += sg * s[j].x;
-                t.y += sg * s[j].y;
+                vt[j].x += sg * s[j].x;
+                vt[j].y += sg * s[j].y;
+                *pt[j] = vt[j];
             }
         }
     }

@@ -107,7 +107,9 @@ def test_product(p, npml):
 @pytest.mark.parametrize("p", [2, 3, 4, 5, 6])
 def test_assembled_with_elements_per_omega(p, disp):
     """PML elements, and in a dispersive medium every element, integrated per
-    call, some of general shape (both geometries of the element matrices)."""
+    call, some of general shape (both geometries of the element matrices); and
+    the assembled operator's product in both types."""
+    import torch
     from fem25_amd.api import MeshInfo
     m, mod, pml, g = case(p, 2)
     if disp:
@@ -119,4 +121,11 @@ def test_assembled_with_elements_per_omega(p, disp):
         assert err(mi.asmble(b"B", f, py, complex128=True), ref) < 1e-13
         got = mi.asmble(b"B", f, py)
         assert np.max(np.abs(got - ref)) < 1e-6 * np.max(np.abs(ref))
+        x = cf.seeded_complex(g.ndof, seed=5)
+        want = sp.csr_matrix((ref, g.jcptr - 1, g.irptr - 1), shape=(g.ndof, g.ndof)) @ x
+        for dt, tol in ((torch.complex128, 1e-13), (torch.complex64, 1e-6)):
+            s, xd = (torch.from_numpy(np.ascontiguousarray(a)).to(dt).cuda() for a in (ref, x))
+            y = torch.empty_like(xd)
+            mi.csr_apply_dev(s, xd, y)
+            assert err(y.cpu().numpy(), want) < tol
     mi.close()

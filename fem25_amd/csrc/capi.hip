@@ -139,13 +139,13 @@ struct f25_mesh_s {
         bool disp = false;
     } ag;
     // PML elements in the batched product: per distinct omega of the batch
-    // their element matrices by power of ky (k_pml_split), applied after the
+    // their element blocks by power of ky (k_pml_sf), applied after the
     // element-block product by k_apply_pml over groups of pairs of one omega
     struct {
         std::vector<double> om;            // distinct omegas the matrices hold
         bool valid = false;                // cleared when the model or the medium changes
         bool disp = false;                 // the matrices cover every element (dispersive medium)
-        double2 *d_mats = nullptr;         // [slot][omega][3][NEE][NEE]
+        double2 *d_mats = nullptr;         // [slot][omega][NPB][NEN][NEN]
         size_t mats_cap = 0;
         double *d_om = nullptr;
         int om_cap = 0;
@@ -841,7 +841,7 @@ static int pml_add(f25_mesh *m, int o, int n, const PmlPar &p, CT *out) {
     typedef PmlSf<NL> S;
     auto kern = k_pml_sf<NL, false, CT>;
     HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
-    hipLaunchKernelGGL(kern, dim3(n, 6), dim3(S::NT), S::lds, m->st, o, 1, (m->disp ? m->d_order : m->d_pml_order) + o,
+    hipLaunchKernelGGL(kern, dim3(n, 6), dim3(S::NT), S::lds, m->st, o, 1, 0, (m->disp ? m->d_order : m->d_pml_order) + o,
                        (const double *)nullptr, m->d_t1d, m->d_wq, m->d_xq, m->d_ieng, m->d_xl, m->d_zl, m->d_xd,
                        m->d_zd, m->d_cdom, m->d_rho, m->d_lam, m->d_mu, m->d_vps, m->disp ? m->d_qp : nullptr,
                        m->disp ? m->d_qs : nullptr, p, m->d_lm, m->d_irptr, m->d_pos[m->disp ? 1 : 0], out, m->d_err);
@@ -1216,8 +1216,24 @@ static const std::vector<int> &omega_cptr(const f25_mesh *m) { return m->disp ? 
 static const int *omega_order(const f25_mesh *m) { return m->disp ? m->d_order : m->d_pml_order; }
 static size_t omega_nelem(const f25_mesh *m) { return m->disp ? m->order.size() : m->pml_order.size(); }
 
+// the blocks by power of ky of every element held per omega, for nom omegas
+template <int NL>
+static int pml_split(f25_mesh *m, int nom, const PmlPar &p) {
+    typedef PmlSf<NL> S;
+    auto kern = k_pml_sf<NL, true, double2>;
+    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
+    for (int f = 0; f < nom; f += 65535)   // the grid's limit in z
+        hipLaunchKernelGGL(kern, dim3((unsigned)omega_nelem(m), NPB, std::min(nom - f, 65535)), dim3(S::NT), S::lds, m->st,
+                           0, nom, f, omega_order(m), m->pa.d_om, m->d_t1d, m->d_wq, m->d_xq, m->d_ieng, m->d_xl, m->d_zl,
+                           m->d_xd, m->d_zd, m->d_cdom, m->d_rho, m->d_lam, m->d_mu, m->d_vps,
+                           m->disp ? m->d_qp : nullptr, m->disp ? m->d_qs : nullptr, p, m->d_lm, (const int64_t *)nullptr,
+                           (const int *)nullptr, m->pa.d_mats, m->d_err);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 // Distinct omegas of the batch (first-appearance order), the pairs of each
-// in groups of at most 16, and the element matrices for those omegas
+// in groups of at most PML_GP, and the element matrices for those omegas
 // (rebuilt when the omegas, the model or the medium change).  No-op without
 // such elements.  h_om: the batch's omegas on the host.
 static int pml_prepare(f25_mesh *m, int npair, const double *h_om) {
@@ -1238,10 +1254,10 @@ static int pml_prepare(f25_mesh *m, int npair, const double *h_om) {
         const int first = (int)P.gpair.size();
         for (int b = 0; b < npair; ++b)
             if (fi[b] == (int)f) P.gpair.push_back(b);
-        for (int g0 = first; g0 < (int)P.gpair.size(); g0 += 16) {
+        for (int g0 = first; g0 < (int)P.gpair.size(); g0 += PML_GP) {
             P.grp.push_back((int)f);
             P.grp.push_back(g0);
-            P.grp.push_back(std::min(16, (int)P.gpair.size() - g0));
+            P.grp.push_back(std::min(PML_GP, (int)P.gpair.size() - g0));
         }
     }
     P.ngrp = (int)P.grp.size() / 3;
@@ -1260,8 +1276,8 @@ static int pml_prepare(f25_mesh *m, int npair, const double *h_om) {
     HIPCHK(hipMemcpyAsync(P.d_grp, P.grp.data(), P.grp.size() * sizeof(int), hipMemcpyHostToDevice, m->st));
     HIPCHK(hipMemcpyAsync(P.d_gpair, P.gpair.data(), P.gpair.size() * sizeof(int), hipMemcpyHostToDevice, m->st));
     if (P.valid && P.disp == m->disp && uo == P.om) return 0;
-    const int nen = m->tab.nen, nee = 3 * nen, nom = (int)uo.size();
-    const size_t nm = omega_nelem(m) * (size_t)nom * 3 * nee * nee;
+    const int nen = m->tab.nen, nom = (int)uo.size();
+    const size_t nm = omega_nelem(m) * (size_t)nom * NPB * nen * nen;
     if (nm > P.mats_cap) {
         dfree(P.d_mats);
         P.mats_cap = 0;
@@ -1280,17 +1296,14 @@ static int pml_prepare(f25_mesh *m, int npair, const double *h_om) {
     p.zwidth = m->d.zwidth;
     p.rcoeff = m->d.pml[0]; p.dmax = m->d.pml[1]; p.kappa = m->d.pml[2]; p.fcent = m->d.pml[3];
     p.freq0 = m->freq0;
-    const size_t lds = (8 * 9 + 3 * 8 * nen) * sizeof(double);
-    const std::vector<int> &cp = omega_cptr(m);
-    for (size_t c = 0; c + 1 < cp.size(); ++c) {
-        const int n = cp[c + 1] - cp[c];
-        if (!n) continue;
-        hipLaunchKernelGGL(k_pml_split, dim3(n, nom), dim3(256), lds, m->st, nen, m->tab.nq1, cp[c], nom,
-                           omega_order(m) + cp[c], P.d_om, m->d_shl, m->d_wq, m->d_xq, m->d_ieng, m->d_xl, m->d_zl,
-                           m->d_xd, m->d_zd, m->d_cdom, m->d_rho, m->d_lam, m->d_mu, m->disp ? m->d_qp : nullptr,
-                           m->disp ? m->d_qs : nullptr, p, P.d_mats, m->d_err);
+    switch (m->tab.nl) {
+        case 3: TRY(pml_split<3>(m, nom, p)); break;
+        case 4: TRY(pml_split<4>(m, nom, p)); break;
+        case 5: TRY(pml_split<5>(m, nom, p)); break;
+        case 6: TRY(pml_split<6>(m, nom, p)); break;
+        case 7: TRY(pml_split<7>(m, nom, p)); break;
+        default: FAIL(F25_ERR_ARG, "unsupported order");
     }
-    HIPCHK(hipGetLastError());
     TRY(check_err(m));
     P.om = uo;
     P.disp = m->disp;
@@ -1300,21 +1313,36 @@ static int pml_prepare(f25_mesh *m, int npair, const double *h_om) {
 
 // y += S_e x over the elements held per omega, colour by colour (after the
 // product, or after a zero fill of y in a dispersive medium)
-template <typename XT>
-static int pml_launch(f25_mesh *m, int npair, const double *d_ky, const XT *x, XT *y) {
+template <int NL, typename XT>
+static int pml_launch_t(f25_mesh *m, int npair, const double *d_ky, const XT *x, XT *y) {
+    typedef PmlApply<NL> S;
     auto &P = m->pa;
-    if (!P.ngrp) return 0;
-    const int nen = m->tab.nen, nom = (int)P.om.size();
-    const size_t lds = (size_t)3 * nen * 16 * sizeof(double2);
+    auto kern = k_apply_pml<NL, XT>;
+    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
     const std::vector<int> &cp = omega_cptr(m);
     for (size_t c = 0; c + 1 < cp.size(); ++c) {
         const int n = cp[c + 1] - cp[c];
         if (!n) continue;
-        hipLaunchKernelGGL(k_apply_pml<XT>, dim3(n, P.ngrp), dim3(256), lds, m->st, nen, cp[c], nom,
-                           omega_order(m) + cp[c], m->d_lm, P.d_grp, P.d_gpair, npair, d_ky, P.d_mats, x, y);
+        for (int g = 0; g < P.ngrp; g += 65535)   // the grid's limit in y
+            hipLaunchKernelGGL(kern, dim3(n, std::min(P.ngrp - g, 65535)), dim3(S::NT), S::lds, m->st, cp[c],
+                               (int)P.om.size(), omega_order(m) + cp[c], m->d_lm, P.d_grp + 3 * (size_t)g, P.d_gpair,
+                               npair, d_ky, P.d_mats, x, y);
     }
     HIPCHK(hipGetLastError());
     return 0;
+}
+
+template <typename XT>
+static int pml_launch(f25_mesh *m, int npair, const double *d_ky, const XT *x, XT *y) {
+    if (!m->pa.ngrp) return 0;
+    switch (m->tab.nl) {
+        case 3: return pml_launch_t<3>(m, npair, d_ky, x, y);
+        case 4: return pml_launch_t<4>(m, npair, d_ky, x, y);
+        case 5: return pml_launch_t<5>(m, npair, d_ky, x, y);
+        case 6: return pml_launch_t<6>(m, npair, d_ky, x, y);
+        case 7: return pml_launch_t<7>(m, npair, d_ky, x, y);
+    }
+    FAIL(F25_ERR_ARG, "unsupported order");
 }
 
 // The whole operator product in a dispersive medium: y = 0, then every

@@ -1,7 +1,15 @@
-// Element matrices integrated per omega (gfx950): PML elements and, in a
-// dispersive medium, every element (CM25ISOQ, KMDAMP, CMDAMP; the moduli and
-// the stretch as described in kernels.hip), by sum factorisation at the
-// reference's 2 p + 5 points per direction.
+// Element matrices integrated per omega (gfx950), by sum factorisation at the
+// reference's 2 p + 5 points per direction:
+//  * PML elements ('A', CM25ISOQ estiff25.f:168-334 with CJACCQ's stretch,
+//    cjac.f:399-581)
+//  * with quality factors (qp != null) every element in the density-
+//    normalised dispersive form: KMDAMP (estiff25.f:511-752) and, for 'A'
+//    elements, CMDAMP (estiff25.f:756-961), velocities from VCMPLX.
+// Both are the KM25ISOQ bilinear forms with complex coefficients at each
+// quadrature point: lambda -> L, mu -> M, rho -> R, derivatives stretched by
+// 1/e_x, 1/e_z (ZDAMPFN) inside PML elements:
+//   standard:   L = w lambda, M = w mu, R = w rho
+//   dispersive: L = w (Vp~^2 - 2 Vs~^2), M = w Vs~^2, R = w.
 //
 // Every component block of the element matrix is a sum over the points of
 // coefficient C(q) times a product of two basis functions or reference
@@ -153,7 +161,7 @@ __global__ void k_pml_pos(int nee, const int *__restrict__ order, const int *__r
 }
 
 // One block of one element.  SPLIT: the blocks by power of ky of omega
-// omf[blockIdx.z], mats[slot][omega][block][a][b] (block 0..3 without ky and
+// omf[f0 + blockIdx.z], mats[slot][omega][block][a][b] (block 0..3 without ky and
 // with the -omega^2 mass, 4 and 5 per ky, 6 and 7 per ky^2).  Otherwise the
 // operator at par, added into CSR order (one launch per colour: no two of its
 // elements share a value).
@@ -168,7 +176,7 @@ __global__ void k_pml_pos(int nee, const int *__restrict__ order, const int *__r
 // unrolled, 122 registers instead of 432).
 template <int NL, bool SPLIT, typename CT>
 __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
-        int slot0, int nom, const int *__restrict__ order, const double *__restrict__ omf,
+        int slot0, int nom, int f0, const int *__restrict__ order, const double *__restrict__ omf,
         const double *__restrict__ t1d, const double *__restrict__ wq, const double *__restrict__ xq,
         const int *__restrict__ ieng, const double *__restrict__ xl, const double *__restrict__ zl,
         const double *__restrict__ xd, const double *__restrict__ zd, const char *__restrict__ cdom,
@@ -184,7 +192,7 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
     int64_t *sr = reinterpret_cast<int64_t *>(sd + N1 * Q1);                     // the rows' starts in CSR order
     const int e = order[blockIdx.x], kb = blockIdx.y, tid = threadIdx.x;
     if constexpr (SPLIT) {
-        par.omega = omf[blockIdx.z];
+        par.omega = omf[f0 + blockIdx.z];
         par.freq = par.omega / (2.0 * M_PI);
         par.kv = kb == PB_12 || kb == PB_23 ? 1.0 : 0.0;
     }
@@ -296,7 +304,7 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
             }
         }
         if constexpr (SPLIT) {
-            CT *o = out + ((((size_t)(slot0 + blockIdx.x) * nom + blockIdx.z) * NPB + kb) * NEN + a) * NEN + bi;
+            CT *o = out + ((((size_t)(slot0 + blockIdx.x) * nom + f0 + blockIdx.z) * NPB + kb) * NEN + a) * NEN + bi;
 #pragma unroll
             for (int j = 0; j < N1; ++j) o[j * N1] = CT{s[j].x, s[j].y};
         } else {
@@ -314,6 +322,162 @@ __global__ __launch_bounds__((PmlSf<NL>::NT)) void k_pml_sf(
             }
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// y_b += S_e(omega_b, ky_b) x_b over the elements of one colour whose blocks
+// k_pml_sf<SPLIT> holds, after the element product has written y (it stores
+// zero rows for PML elements; for a dispersive medium y is zero-filled
+// first).  Workgroup (element, group of up to PML_GP pairs of one omega), a
+// wave per output component and tile of 16 rows: FP64 MFMA over the element's
+// nodes, four at a time, columns eight pairs' real and imaginary parts.  A
+// complex block A acts on a pair's columns as Re A (re, im) + Im A (-im, re);
+// its ky or ky^2 goes to the column, so one read of a tile serves every pair
+// of the omega.  Per component: the diagonal block, its ky^2 part and the two
+// couplings; transposed blocks are read transposed.  grp[3 g + 0..2] = (omega
+// index, first slot in gpair, count).  Arithmetic in FP64 for every vector
+// type.
+//
+// Bound by latency, then memory: eight blocks an element and omega (80 KB at
+// p4) are read once, 330 MB a colour with x and y (70 us at the rate of a
+// copy).  Measured on MI355X, 198 elements of one colour at p4, 240 pairs of
+// 10 omegas: nine blocks for each power of ky, read per 16 pairs, on the
+// vector ALUs 696 us; this form 217 us, and 165 us with the gather's, the
+// tiles' and the rows' loads issued together (four waves per SIMD: at 130
+// registers one workgroup of six waves fits a CU instead of two).
+constexpr int PML_GP = 32;   // pairs of a group
+
+template <int NL>
+struct PmlApply {
+    static constexpr int NEN = NL * NL, NEE = 3 * NEN, MT = (NEN + 15) / 16, KS = (NEN + 3) / 4, KN = 4 * KS;
+    static constexpr int NT = 64 * 3 * MT;
+    static constexpr size_t lds = (size_t)3 * KN * PML_GP * sizeof(double2);
+};
+
+template <int NL, typename XT>
+__global__ __launch_bounds__((PmlApply<NL>::NT)) __attribute__((amdgpu_waves_per_eu(4))) void k_apply_pml(int slot0, int nom, const int *__restrict__ order,
+                                                                  const int *__restrict__ lm, const int *__restrict__ grp,
+                                                                  const int *__restrict__ gpair, int npair,
+                                                                  const double *__restrict__ ky,
+                                                                  const double2 *__restrict__ mats,
+                                                                  const XT *__restrict__ x, XT *__restrict__ y) {
+    typedef PmlApply<NL> S;
+    typedef MfmaTraits<double> MF;
+    typedef decltype(XT().x) R;
+    constexpr int NEN = S::NEN, NEE = S::NEE, MT = S::MT, KS = S::KS, KN = S::KN, GP = PML_GP;
+    extern __shared__ double2 xs[];   // [component][node][pair], zero past the last node and pair
+    const int e = order[blockIdx.x], g = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), ci = wv / MT, mt = wv % MT;
+    const int f = grp[3 * g], first = grp[3 * g + 1], cnt = grp[3 * g + 2];
+    const int *L = lm + (size_t)e * NEE;
+    // a thread gathers pair tid % GP of rows tid / GP + k NT / GP: its loads
+    // are issued together
+    constexpr int RS = S::NT / GP, NR = (3 * KN + RS - 1) / RS;
+    {
+        const int p = tid % GP, r0 = tid / GP;
+        const size_t pair = gpair[first + min(p, cnt - 1)];
+        int d[NR];
+        XT t[NR];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) d[k] = L[min(r0 + k * RS, NEE - 1)];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) t[k] = x[(size_t)max(d[k], 0) * npair + pair];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const int r = r0 + k * RS;
+            const bool in = r < NEE && d[k] >= 0 && p < cnt;
+            if (r < 3 * KN)
+                xs[((r % 3) * KN + r / 3) * GP + p] =
+                    in ? make_double2((double)t[k].x, (double)t[k].y) : make_double2(0.0, 0.0);
+        }
+    }
+    // this wave's four blocks: (block, transposed, input component)
+    const int t3 = ci == 1 ? PB_12 : PB_13, c3 = ci == 0 ? 2 : 0;      // 13 x3 | -12^T k x1 | 13^T x1
+    const int t4 = ci == 0 ? PB_12 : PB_23, c4 = ci == 1 ? 2 : 1;      // 12 k x2 | 23 k x3 | -23^T k x2
+    const int tb[4] = {ci, ci == 1 ? PB_L2 : PB_M, t3, t4}, ic[4] = {ci, ci, c3, c4};
+    const bool tr[4] = {false, false, ci != 0, ci == 2};
+    const double2 *mb = mats + ((size_t)(slot0 + blockIdx.x) * nom + f) * NPB * NEN * NEN;
+    const int m = mt * 16 + (lane & 15), kg = lane >> 4, col = lane & 15, part = col & 1;
+    const double2 *ab[4];
+    int sb[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int mc = min(m, NEN - 1);
+        ab[t] = mb + (size_t)tb[t] * NEN * NEN + (tr[t] ? mc : mc * NEN);
+        sb[t] = tr[t] ? NEN : 1;
+    }
+    const int nch = (cnt + 7) / 8;
+    // column factors of the couplings, of the ky^2 block, per chunk of pairs
+    constexpr int NC = GP / 8;
+    double f2[NC], f3[NC], f4[NC];
+#pragma unroll
+    for (int h = 0; h < NC; ++h) {
+        const int p = h * 8 + (col >> 1);
+        const double k = p < cnt ? ky[gpair[first + p]] : 0.0;
+        f2[h] = k * k;
+        f3[h] = ci == 1 ? -k : 1.0;
+        f4[h] = ci == 2 ? -k : k;
+    }
+    typedef typename MF::v4 V4;
+    V4 acc[NC];
+#pragma unroll
+    for (int h = 0; h < NC; ++h) acc[h] = V4{0.0, 0.0, 0.0, 0.0};
+    // rows of y this lane adds to, and the blocks' tiles of the first four nodes
+    int dr[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int a = mt * 16 + MF::row(kg, i), d = L[3 * min(a, NEN - 1) + ci];
+        dr[i] = a < NEN ? d : -1;
+    }
+    double2 A[4], An[4];
+    auto load = [&](int s, double2 *v) {
+        const int bc = min(4 * s + kg, NEN - 1);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[t] = ab[t][bc * sb[t]];
+    };
+    load(0, An);
+    __syncthreads();
+#pragma unroll 2
+    for (int s = 0; s < KS; ++s) {
+        const int b = 4 * s + kg;
+        const bool in = b < NEN && m < NEN;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) A[t] = in ? An[t] : make_double2(0.0, 0.0);
+        load(min(s + 1, KS - 1), An);   // the next tiles while these multiply
+#pragma unroll
+        for (int h = 0; h < NC; ++h) {
+            if (h >= nch) break;
+            const int o = b * GP + h * 8 + (col >> 1);
+            const double2 v0 = xs[ic[0] * KN * GP + o], v3 = xs[ic[2] * KN * GP + o], v4 = xs[ic[3] * KN * GP + o];
+            // (re, im) and (-im, re) of the column's part
+            const double b0 = part ? v0.y : v0.x, d0 = part ? v0.x : -v0.y;
+            const double b3 = f3[h] * (part ? v3.y : v3.x), d3 = f3[h] * (part ? v3.x : -v3.y);
+            const double b4 = f4[h] * (part ? v4.y : v4.x), d4 = f4[h] * (part ? v4.x : -v4.y);
+            acc[h] = MF::mma(A[0].x, b0, acc[h]);
+            acc[h] = MF::mma(A[0].y, d0, acc[h]);
+            acc[h] = MF::mma(A[1].x, f2[h] * b0, acc[h]);
+            acc[h] = MF::mma(A[1].y, f2[h] * d0, acc[h]);
+            acc[h] = MF::mma(A[2].x, b3, acc[h]);
+            acc[h] = MF::mma(A[2].y, d3, acc[h]);
+            acc[h] = MF::mma(A[3].x, b4, acc[h]);
+            acc[h] = MF::mma(A[3].y, d4, acc[h]);
+        }
+    }
+    R *yp = reinterpret_cast<R *>(y) + part;
+    R yv[NC][4];
+    size_t po[NC];
+#pragma unroll
+    for (int h = 0; h < NC; ++h) {
+        po[h] = gpair[first + min(h * 8 + (col >> 1), cnt - 1)];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) yv[h][i] = yp[((size_t)max(dr[i], 0) * npair + po[h]) * 2];
+    }
+#pragma unroll
+    for (int h = 0; h < NC; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (dr[i] >= 0 && h * 8 + (col >> 1) < cnt)
+                yp[((size_t)dr[i] * npair + po[h]) * 2] = (R)((double)yv[h][i] + acc[h][i]);
 }
 
 }  // namespace f25k

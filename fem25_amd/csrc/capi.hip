@@ -180,6 +180,10 @@ struct f25_mesh_s {
     int *d_mygrad = nullptr, *d_jcsc = nullptr, *d_icsc = nullptr;
     int *d_dab_pos = nullptr;   // [column][row of its last element]: position in ICSC_FDIST, -1 fixed
     double *d_ew = nullptr;
+    // GNMFREE's tables, J p and partial sums, grown on demand (at most kGnKeep
+    // bytes are kept after a call)
+    unsigned char *d_gn = nullptr;
+    size_t gn_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // (omega, ky) staging, grown on demand
     double *d_omky = nullptr;
@@ -543,6 +547,7 @@ extern "C" int f25_mesh_destroy(f25_mesh *m) {
     dfree(m->d_mygrad); dfree(m->d_jcsc); dfree(m->d_icsc); dfree(m->d_dab_pos);
     dfree(m->d_ew);
     dfree(m->d_omky);
+    dfree(m->d_gn);
     dfree(m->br.d_order); dfree(m->br.d_aorder); dfree(m->br.d_gorder); dfree(m->br.d_first0); dfree(m->br.d_brows); dfree(m->br.d_xz); dfree(m->br.d_comp);
     dfree(m->br.d_pw);
     for (auto &q : m->br.d_lm) dfree(q);
@@ -2951,41 +2956,88 @@ static void launch_gn_jp(hipStream_t st, int nnpgl, int njac, int64_t pt, const 
     int nch, cch;
     gn_jp_chunks(nnpgl, nch, cch);
     hipLaunchKernelGGL(k_gn_jp, dim3(nch, njac), dim3(256), 0, st, nnpgl, cch, pt, dn, djo, dpo, dmy, jac, p, part);
-    const int nb = (int)std::min<int64_t>((pt + 255) / 256, 4096);
+    const int nb = (int)std::min<int64_t>((pt + 63) / 64, 4096);
     hipLaunchKernelGGL(k_gn_jsum, dim3(std::max(nb, 1)), dim3(256), 0, st, nch, pt, part, jp);
 }
 
+static size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
+
+// GNMFREE's scratch for njac Jacobians of pt observations in all and nch
+// column chunks: nobs | joff | poff | alpha | J p (pt) | partials (nch * pt)
+struct GnScratch {
+    size_t joff, poff, alpha, jp, part, bytes;
+    GnScratch(int njac, int64_t pt, int nch) {
+        joff = align256(sizeof(int) * (size_t)njac);
+        poff = align256(joff + sizeof(int64_t) * (size_t)njac);
+        alpha = align256(poff + sizeof(int64_t) * (size_t)njac);
+        jp = align256(alpha + sizeof(double) * (size_t)njac);
+        part = align256(jp + sizeof(double2) * (size_t)pt);
+        bytes = part + sizeof(double2) * (size_t)nch * (size_t)pt;
+    }
+};
+
+// the contraction on a scratch of at least GnScratch::bytes at base; the
+// tables go up in one copy (they lie one after the other)
+static int gnmfree_run(f25_mesh *m, int njac, const int *nobs, const double *alpha, const float2 *jac, const double *p,
+                       double *z, const std::vector<int64_t> &joff, const std::vector<int64_t> &poff, int64_t pt,
+                       const GnScratch &S, unsigned char *base) {
+    const int n = m->inv.nnpgl;
+    std::vector<unsigned char> h(S.jp);
+    std::memcpy(h.data(), nobs, sizeof(int) * (size_t)njac);
+    std::memcpy(h.data() + S.joff, joff.data(), sizeof(int64_t) * (size_t)njac);
+    std::memcpy(h.data() + S.poff, poff.data(), sizeof(int64_t) * (size_t)njac);
+    std::memcpy(h.data() + S.alpha, alpha, sizeof(double) * (size_t)njac);
+    HIPCHK(hipMemcpyAsync(base, h.data(), S.jp, hipMemcpyHostToDevice, m->st));
+    const int *dn = reinterpret_cast<const int *>(base);
+    const int64_t *djo = reinterpret_cast<const int64_t *>(base + S.joff), *dpo = reinterpret_cast<const int64_t *>(base + S.poff);
+    const double *da = reinterpret_cast<const double *>(base + S.alpha);
+    double2 *djp = reinterpret_cast<double2 *>(base + S.jp), *dpart = reinterpret_cast<double2 *>(base + S.part);
+    (void)hipEventRecord(m->ev0, m->st);
+    launch_gn_jp(m->st, n, njac, pt, dn, djo, dpo, m->d_mygrad, jac, p, dpart, djp);
+    // per Jacobian and column where those sums fit the space of J p's partial
+    // sums, which are done with (they do from about 32 observations a Jacobian
+    // up to 16,384 columns), else a wave per column over all Jacobians: no more
+    // scratch either way, and the same choice in both entry points
+    if (sizeof(double) * (size_t)njac * (size_t)n <= S.bytes - S.part) {
+        double *zp = reinterpret_cast<double *>(dpart);
+        hipLaunchKernelGGL(k_gn_zpart, dim3((n + GZ_C - 1) / GZ_C, njac), dim3(256), 0, m->st, n, dn, djo, dpo, jac, djp, zp);
+        hipLaunchKernelGGL(k_gn_zsum, dim3((n + 255) / 256), dim3(256), 0, m->st, n, njac, da, m->d_mygrad, zp, z);
+    } else {
+        hipLaunchKernelGGL(k_gn_z, dim3((n + 3) / 4), dim3(256), 0, m->st, n, njac, dn, djo, dpo, da, m->d_mygrad, jac, djp,
+                           z);
+    }
+    (void)hipEventRecord(m->ev1, m->st);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(m->st);
+    if (e != hipSuccess) FAIL(F25_ERR_HIP, hipGetErrorString(e));
+    float ms = 0.f;
+    if (hipEventElapsedTime(&ms, m->ev0, m->ev1) == hipSuccess) record_ms("gnmfree", ms);
+    return 0;
+}
+
+// Scratch a handle keeps between f25_gnmfree_dev calls: allocating and freeing
+// it took 0.4 of 2.4 ms at 120 Jacobians of 20..120 receivers (110 MB)
+static constexpr size_t kGnKeep = size_t(1) << 30;
+
 static int gnmfree_core(f25_mesh *m, int njac, const int *nobs, const double *alpha, const float2 *jac,
                         const double *p, double *z) {
-    const int n = m->inv.nnpgl;
     std::vector<int64_t> joff, poff;
     int64_t jt, pt;
-    TRY(gn_offsets(njac, nobs, n, joff, poff, jt, pt));
-    int *dn = nullptr;
-    int64_t *djo = nullptr, *dpo = nullptr;
-    double *da = nullptr;
-    double2 *djp = nullptr, *dpart = nullptr;
+    TRY(gn_offsets(njac, nobs, m->inv.nnpgl, joff, poff, jt, pt));
     int nch, cch;
-    gn_jp_chunks(n, nch, cch);
-    int r = upload(&dn, nobs, (size_t)njac, m->st);
-    if (!r) r = upload(&djo, joff.data(), (size_t)njac, m->st);
-    if (!r) r = upload(&dpo, poff.data(), (size_t)njac, m->st);
-    if (!r) r = upload(&da, alpha, (size_t)njac, m->st);
-    if (!r) r = dalloc(&djp, (size_t)std::max<int64_t>(pt, 1));
-    if (!r) r = dalloc(&dpart, (size_t)nch * std::max<int64_t>(pt, 1));
-    if (!r) {
-        (void)hipEventRecord(m->ev0, m->st);
-        launch_gn_jp(m->st, n, njac, pt, dn, djo, dpo, m->d_mygrad, jac, p, dpart, djp);
-        hipLaunchKernelGGL(k_gn_z, dim3((n + 3) / 4), dim3(256), 0, m->st, n, njac, dn, djo, dpo, da,
-                           m->d_mygrad, jac, djp, z);
-        (void)hipEventRecord(m->ev1, m->st);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(m->st);
-        if (e != hipSuccess) { g_err = hipGetErrorString(e); r = F25_ERR_HIP; }
-        float ms = 0.f;
-        if (!r && hipEventElapsedTime(&ms, m->ev0, m->ev1) == hipSuccess) record_ms("gnmfree", ms);
+    gn_jp_chunks(m->inv.nnpgl, nch, cch);
+    const GnScratch S(njac, std::max<int64_t>(pt, 1), nch);
+    if (S.bytes > m->gn_cap) {
+        dfree(m->d_gn);
+        m->gn_cap = 0;
+        TRY(dalloc(&m->d_gn, S.bytes));
+        m->gn_cap = S.bytes;
     }
-    dfree(dn); dfree(djo); dfree(dpo); dfree(da); dfree(djp); dfree(dpart);
+    const int r = gnmfree_run(m, njac, nobs, alpha, jac, p, z, joff, poff, pt, S, m->d_gn);
+    if (m->gn_cap > kGnKeep) {
+        dfree(m->d_gn);
+        m->gn_cap = 0;
+    }
     return r;
 }
 
@@ -3191,8 +3243,6 @@ static int scratch_on(int dev, unsigned char **out) {
     return 0;
 }
 
-static size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
-
 extern "C" int f25_gnmfree_dev_noalloc(f25_mesh *m, int njac, const int *nobs, const double *alpha,
                                        const void *jac, const double *p, double *z) {
     if (!m || njac <= 0 || njac > 65535 || !nobs || !alpha || !jac || !p || !z) FAIL(F25_ERR_ARG, "invalid arguments");
@@ -3200,40 +3250,16 @@ extern "C" int f25_gnmfree_dev_noalloc(f25_mesh *m, int njac, const int *nobs, c
     HIPCHK(hipSetDevice(m->dev));
     unsigned char *base = nullptr;
     TRY(scratch_on(m->dev, &base));
-    const int n = m->inv.nnpgl;
     std::vector<int64_t> joff, poff;
     int64_t jt, pt;
-    TRY(gn_offsets(njac, nobs, n, joff, poff, jt, pt));
+    TRY(gn_offsets(njac, nobs, m->inv.nnpgl, joff, poff, jt, pt));
     int nch, cch;
-    gn_jp_chunks(n, nch, cch);
-    // scratch layout: nobs | joff | poff | alpha | JP (pt) | partials (nch * pt)
-    const size_t o_nobs = 0, o_joff = align256(o_nobs + sizeof(int) * njac),
-                 o_poff = align256(o_joff + sizeof(int64_t) * njac),
-                 o_alpha = align256(o_poff + sizeof(int64_t) * njac),
-                 o_jp = align256(o_alpha + sizeof(double) * njac), o_part = align256(o_jp + sizeof(double2) * pt),
-                 need = o_part + sizeof(double2) * (size_t)nch * pt;
-    if (need > kScratchBytes)
+    gn_jp_chunks(m->inv.nnpgl, nch, cch);
+    const GnScratch S(njac, pt, nch);
+    if (S.bytes > kScratchBytes)
         FAIL(F25_ERR_ARG, "batch too large for the 32 MiB scratch: sum(nobs) * (chunks + 1) * 16 bytes "
                           "exceeds it; split the Jacobians over calls (z accumulates)");
-    int *dn = reinterpret_cast<int *>(base + o_nobs);
-    int64_t *djo = reinterpret_cast<int64_t *>(base + o_joff), *dpo = reinterpret_cast<int64_t *>(base + o_poff);
-    double *da = reinterpret_cast<double *>(base + o_alpha);
-    double2 *djp = reinterpret_cast<double2 *>(base + o_jp), *dpart = reinterpret_cast<double2 *>(base + o_part);
-    HIPCHK(hipMemcpyAsync(dn, nobs, sizeof(int) * njac, hipMemcpyHostToDevice, m->st));
-    HIPCHK(hipMemcpyAsync(djo, joff.data(), sizeof(int64_t) * njac, hipMemcpyHostToDevice, m->st));
-    HIPCHK(hipMemcpyAsync(dpo, poff.data(), sizeof(int64_t) * njac, hipMemcpyHostToDevice, m->st));
-    HIPCHK(hipMemcpyAsync(da, alpha, sizeof(double) * njac, hipMemcpyHostToDevice, m->st));
-    (void)hipEventRecord(m->ev0, m->st);
-    launch_gn_jp(m->st, n, njac, pt, dn, djo, dpo, m->d_mygrad, (const float2 *)jac, p, dpart, djp);
-    hipLaunchKernelGGL(k_gn_z, dim3((n + 3) / 4), dim3(256), 0, m->st, n, njac, dn, djo, dpo, da, m->d_mygrad,
-                       (const float2 *)jac, djp, z);
-    (void)hipEventRecord(m->ev1, m->st);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(m->st);
-    if (e != hipSuccess) FAIL(F25_ERR_HIP, hipGetErrorString(e));
-    float ms = 0.f;
-    if (hipEventElapsedTime(&ms, m->ev0, m->ev1) == hipSuccess) record_ms("gnmfree", ms);
-    return 0;
+    return gnmfree_run(m, njac, nobs, alpha, (const float2 *)jac, p, z, joff, poff, pt, S, base);
 }
 
 extern "C" int f25_gnmfree(f25_mesh *m, int njac, const int *nobs, const double *alpha, const void *jac,

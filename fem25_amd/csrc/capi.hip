@@ -188,6 +188,7 @@ struct f25_mesh_s {
     // (omega, ky) staging, grown on demand
     double *d_omky = nullptr;
     int omky_cap = 0;
+    std::vector<double> h_omky;
     // Bielak sources in the batch: the ring of elements holding both 'B' and
     // 'E' DOFs, by colour, with DOF maps selecting the input and output
     // classes of ASMB_PEFF's two terms, and the DOF positions of
@@ -1444,14 +1445,18 @@ static int apply_core(f25_mesh *m, int npair, const double *d_om, const double *
     return 0;
 }
 
+// omega and ky of a batch on the device, one after the other, in one copy (two
+// took a tenth of a one-pair product): omega at d_omky, ky at d_omky + n
 static int stage_omky(f25_mesh *m, int n, const double *omega, const double *ky) {
     if (n > m->omky_cap) {
         dfree(m->d_omky);
+        m->omky_cap = 0;
         TRY(dalloc(&m->d_omky, 2 * (size_t)n));
         m->omky_cap = n;
     }
-    HIPCHK(hipMemcpyAsync(m->d_omky, omega, n * sizeof(double), hipMemcpyHostToDevice, m->st));
-    HIPCHK(hipMemcpyAsync(m->d_omky + m->omky_cap, ky, n * sizeof(double), hipMemcpyHostToDevice, m->st));
+    m->h_omky.assign(omega, omega + n);
+    m->h_omky.insert(m->h_omky.end(), ky, ky + n);
+    HIPCHK(hipMemcpyAsync(m->d_omky, m->h_omky.data(), 2 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, m->st));
     return 0;
 }
 
@@ -1462,7 +1467,7 @@ extern "C" int f25_apply_batch_dev(f25_mesh *m, int npair, const double *omega, 
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
     TRY(product_ready(m, npair, mode & ~F25_APPLY_GRAPH));
-    return apply_core(m, npair, m->d_omky, m->d_omky + m->omky_cap, mode, x, y, m->d_rec, m->d_vcf, omega);
+    return apply_core(m, npair, m->d_omky, m->d_omky + npair, mode, x, y, m->d_rec, m->d_vcf, omega);
 }
 
 extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omega, const double *ky,
@@ -1473,7 +1478,7 @@ extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omeg
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
     TRY(product_ready(m, npair, F25_APPLY_F64));
-    TRY(apply_core(m, npair, m->d_omky, m->d_omky + m->omky_cap, F25_APPLY_F64, u, r, m->d_rec, m->d_vcf, omega));
+    TRY(apply_core(m, npair, m->d_omky, m->d_omky + npair, F25_APPLY_F64, u, r, m->d_rec, m->d_vcf, omega));
     const int gy = (int)std::min<int64_t>(256, std::max<int64_t>(1, m->g.ndof / 256));
     double *part = nullptr, *sums = nullptr;
     int rc = dalloc(&part, (size_t)gy * npair * 2);
@@ -1641,7 +1646,7 @@ extern "C" int f25_peff_batch_dev(f25_mesh *m, int npair, const double *omega, c
     TRY(bielak_prepare(m));
     TRY(stage_omky(m, npair, omega, ky));
     TRY(ring_ready(m, npair));
-    const double *om = m->d_omky, *kv = m->d_omky + m->omky_cap;
+    const double *om = m->d_omky, *kv = m->d_omky + npair;
     HIPCHK(hipEventRecord(m->ev0, m->st));
     TRY(peff_launches(m, npair, om, kv, (const double2 *)ue_dev, (double2 *)peff_dev));
     HIPCHK(hipEventRecord(m->ev1, m->st));
@@ -1762,7 +1767,7 @@ extern "C" int f25_bielak_rhs_dev(f25_mesh *m, int npair, const double *omega, c
     TRY(stage_omky(m, npair, omega, ky));
     TRY(ring_ready(m, npair));
     TRY(uwave_params(m, npair, kappax, kappaz, baz, aoi));
-    const double *om = m->d_omky, *kv = m->d_omky + m->omky_cap;
+    const double *om = m->d_omky, *kv = m->d_omky + npair;
     // staging buffers may have moved since the capture
     if (B.exec && (B.om != om || B.pw != B.d_pw || B.pad != m->d_vpad || B.vcf != m->d_vcf)) {
         HIPCHK(hipStreamSynchronize(m->st));
@@ -1941,7 +1946,7 @@ extern "C" int f25_gradient_dev(f25_mesh *m, int ntrip, const double *omega, con
     if (!m->have_model) FAIL(F25_ERR_STATE, "f25_set_model has not been called");
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, ntrip, omega, ky));
-    return grad_core(m, ntrip, m->d_omky, m->d_omky + m->omky_cap, u, lam, g, 1);
+    return grad_core(m, ntrip, m->d_omky, m->d_omky + ntrip, u, lam, g, 1);
 }
 
 extern "C" int f25_gradient32_dev(f25_mesh *m, int ntrip, const double *omega, const double *ky,
@@ -1951,7 +1956,7 @@ extern "C" int f25_gradient32_dev(f25_mesh *m, int ntrip, const double *omega, c
     if (!m->have_model) FAIL(F25_ERR_STATE, "f25_set_model has not been called");
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, ntrip, omega, ky));
-    return grad_core(m, ntrip, m->d_omky, m->d_omky + m->omky_cap, u, lam, g, 1, true);
+    return grad_core(m, ntrip, m->d_omky, m->d_omky + ntrip, u, lam, g, 1, true);
 }
 
 static int grad_host(f25_mesh *m, int ntrip, const double *omega, const double *ky, const void *u,

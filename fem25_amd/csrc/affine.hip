@@ -53,8 +53,10 @@ struct AfShape {
     static constexpr int XS = NEE * PW, ES = 2 * NL * 64;
     static constexpr size_t lds_apply = (size_t)NW * (XS * 16 + ES * 8 + NEE * 16) + 16 * NL * 8;
     // the gradient's LDS per wave: element values of both fields for PW triples
-    static constexpr int GS = 2 * NEE * PW;
-    static constexpr size_t lds_grad = (size_t)NW * GS * 16 + 16 * NL * 8;
+    // (VS values a vector: not a multiple of 256 bytes, or the triples' reads
+    // meet in one bank)
+    static constexpr int VS = NEE % 16 ? NEE : NEE + 1, GS = 2 * VS * PW;
+    static constexpr size_t lds_grad(int nw) { return (size_t)nw * GS * 16 + 16 * NL * 8; }
 };
 
 __global__ void k_aff_rec(int nelem, const int *__restrict__ ieng, const double *__restrict__ xl,
@@ -88,11 +90,11 @@ __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" :
 __device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // Gathers one element's values of the wave's V vectors into its LDS region,
-// [vector][NEE] values of 16 bytes: lane i takes element values i, i + 64, ...
+// [vector][VS] values of 16 bytes: lane i takes element values i, i + 64, ...
 // of each vector, so a load is a wave-uniform base (the vector) and a lane
 // offset (the DOF) kept over the whole batch.  Fixed DOFs are not loaded:
 // their values are set to zero once (zero).
-template <int NEE, int V>
+template <int NEE, int V, int VS>
 struct AfGather {
     static constexpr int K = (NEE + 63) / 64;
     int off[K];   // DOF of the lane's element value, -1: none
@@ -104,17 +106,20 @@ struct AfGather {
 #pragma unroll
         for (int k = 0; k < K; ++k)
             if (lane + 64 * k < NEE && off[k] < 0)
-                for (int v = 0; v < V; ++v) dst[v * NEE + lane + 64 * k] = make_double2(0.0, 0.0);
+                for (int v = 0; v < V; ++v) dst[v * VS + lane + 64 * k] = make_double2(0.0, 0.0);
         lds_wait();
     }
-    // base(v): the vector's values by DOF
+    // base(v): the vector's values by DOF, null for a vector that is not there
     template <typename F>
     __device__ __forceinline__ void get(double2 *dst, F base) {
 #pragma unroll
-        for (int k = 0; k < K; ++k)
-            if (off[k] >= 0)
+        for (int v = 0; v < V; ++v) {
+            const double2 *b = base(v);
+            if (b)
 #pragma unroll
-                for (int v = 0; v < V; ++v) dma16(base(v) + off[k], dst + v * NEE + 64 * k);
+                for (int k = 0; k < K; ++k)
+                    if (off[k] >= 0) dma16(b + off[k], dst + v * VS + 64 * k);
+        }
     }
 };
 
@@ -432,7 +437,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // time in the first pass (each waited for its LDS reads) 1.82; the point
 // loop unrolled spills (p6 1.03 ms against 0.56), its 1-D values loaded one
 // point ahead 1.67 ms, or as DPP operands in program order 1.71 (p6 0.65):
-// here the scalar loads of a rolled loop cost less than that order.
+// here the scalar loads of a rolled loop cost less than that order.  LDS and
+// loads follow the triples there are: one triple at 120x60, p4 149 -> 97 us,
+// p6 191 -> 118; vectors a multiple of 256 bytes apart (p3) met in one bank:
+// 128 triples at 120x60 738 -> 392 us.
 template <int NL, bool RECT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_grad_af(
         const int *__restrict__ elems, const double *__restrict__ rec, const double *__restrict__ tab,
@@ -447,7 +455,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nw = blockDim.x >> 6;
     double2 *sw = reinterpret_cast<double2 *>(sm) + wv * S::GS;
-    double *st = sm + S::NW * S::GS * 2;
+    double *st = sm + nw * S::GS * 2;
     const int e = elems[blockIdx.x];
     const double *rc = rec + (size_t)e * AFR;
     if (rc[17] != 0.0) {   // PML elements are outside the gradient
@@ -457,14 +465,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     for (int i = threadIdx.x; i < 16 * NL; i += blockDim.x) st[i] = tab[i];
     __syncthreads();
     const int nch = (ntrip + PW - 1) / PW;
-    typedef AfGather<NEE, 2 * PW> G;
+    typedef AfGather<NEE, 2 * PW, S::VS> G;
     G ga;
     ga.init(lane, lm + (size_t)e * NEE);
     ga.zero(lane, sw);
     // vectors 0 .. PW - 1: u of the chunk's triples, then l
     auto base = [&](int t0) {
         return [=](int v) -> const double2 * {
-            return (v >= PW ? l : u) + (size_t)min(t0 + v % PW, ntrip - 1) * ndof;
+            return t0 + v % PW < ntrip ? (v >= PW ? l : u) + (size_t)(t0 + v % PW) * ndof : nullptr;
         };
     };
     if (wv < nch) ga.get(sw, base(wv * PW));
@@ -485,9 +493,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             double v[NL], d[NL];
 #pragma unroll
             for (int j = 0; j < NL; ++j) { v[j] = st[eta * 16 + j]; d[j] = (RECT ? sz : 1.0) * st[eta * 16 + NL + j]; }
-            const double *a = reinterpret_cast<const double *>(sw + tr * NEE);
+            const double *a = reinterpret_cast<const double *>(sw + tr * S::VS);
             auto at = [&](int k) {   // component k % 3 of field k / 3
-                return a + (k / 3) * (2 * PW * NEE) + 2 * (k % 3) + (k % 3 == 1 ? 1 - im : im);
+                return a + (k / 3) * (2 * PW * S::VS) + 2 * (k % 3) + (k % 3 == 1 ? 1 - im : im);
             };
             double x[NL];
 #pragma unroll

@@ -1895,9 +1895,10 @@ static int grad_affine(f25_mesh *m, int ntrip, const double *d_om, const double 
                        const double2 *l) {
     typedef AfShape<NL> S;
     auto kern = m->rect ? k_grad_af<NL, true> : k_grad_af<NL, false>;
-    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_grad));
+    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)S::lds_grad(S::NW)));
     const int nw = std::min(S::NW, (ntrip + S::PW - 1) / S::PW);
-    hipLaunchKernelGGL(kern, dim3(m->naff), dim3(64 * nw), S::lds_grad, m->st, m->d_aelem, m->d_rec, m->d_taf, m->d_lm,
+    hipLaunchKernelGGL(kern, dim3(m->naff), dim3(64 * nw), S::lds_grad(nw), m->st, m->d_aelem, m->d_rec, m->d_taf, m->d_lm,
                        ntrip, (int64_t)m->g.ndof, d_om, d_ky, u, l, m->d_part);
     HIPCHK(hipGetLastError());
     return 0;

@@ -1161,14 +1161,36 @@ static int affine_colour(f25_mesh *m, const int *order, int n, const int *lm_in,
 // means the block kernel
 static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt && m->g.ndof < (1 << 27); }
 
+// Whether a batch of the operator product takes them there (mode F64 or F32).
+// FP64 arithmetic runs at the rate of FP32 arithmetic without packed
+// instructions, so k_apply_af beats the blocks in both modes (FP32: their
+// matrix units) where the blocks are large (200x100 elements, 45 pairs, FP32:
+// p4 0.93 -> 0.72 ms, p5 2.24 -> 1.10, p6 4.42 -> 2.01) or the batch is too
+// small to fill the chip with a workgroup or a few waves per element (FP32,
+// 40x20, 320 pairs: p2 178 -> 104 us, p3 212 -> 145; 200x100, 8 pairs: 108 ->
+// 85, 133 -> 112).  Blocks of p2 (and of p3 in FP32) cost little and lose less
+// on large batches: FP32, blocks / k_apply_af: 97x61, 45 pairs p3 141 / 163,
+// 128 pairs p2 193 / 221, p3 254 / 360, 200x100, 128 pairs 519 / 570, 695 /
+// 966; FP64 p2, 97x61: 45 pairs 117 / 123, 128 pairs 228 / 250.  The line lies
+// between 256,000 and 266,000 products of one element and one pair.
+static bool affine_batch(const f25_mesh *m, int npair, int mode) {
+    const int nl = mode == F25_APPLY_F32 ? 5 : 4;
+    return affine_product(m) && (m->tab.nl >= nl || (int64_t)m->d.nelem * npair < (1 << 18));
+}
+
 // what the product's launches read: zero rows and sink, and the element
 // blocks of the elements that are not parallelograms
 static int product_ready(f25_mesh *m, int npair, int mode) {
     TRY(ensure_vpad(m, npair));
     if (m->disp) return 0;   // every element per omega
     if (mode == F25_APPLY_F32_REFINED) return ensure_blocks(m, true);
-    if (affine_product(m) && !m->ngen) return 0;
+    if (affine_batch(m, npair, mode) && !m->ngen) return 0;
     return mode == F25_APPLY_F32 ? ensure_blocks(m, true) : ensure_vcf(m);
+}
+
+// the records launch_f64 takes for the operator product
+static const double *product_rec(const f25_mesh *m, int npair) {
+    return affine_batch(m, npair, F25_APPLY_F64) ? m->d_rec : nullptr;
 }
 
 // the launches of the FP64 product (product_ready first), one or two per
@@ -1188,12 +1210,10 @@ static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair
     return 0;
 }
 
-// The FP32 products (product_ready first).  Plain FP32 takes its parallelograms
-// through k_apply_af on complex64 vectors: FP64 arithmetic runs at the rate
-// of FP32 arithmetic without packed instructions, and the vectors are what
-// the kernel moves.  The refined product keeps its blocks for every element.
+// The FP32 products (product_ready first).  The refined product keeps its
+// blocks for every element.
 static int launch_f32(f25_mesh *m, const double *om, const double *kv, int npair, const float2 *x, float2 *y) {
-    const bool aff = affine_product(m);
+    const bool aff = affine_batch(m, npair, F25_APPLY_F32);
     for (size_t c = 0; c + 1 < m->cptr.size(); ++c) {
         const std::vector<int> &gp = aff ? m->gcptr : m->cptr;
         if (aff && m->acptr[c + 1] > m->acptr[c])
@@ -1467,7 +1487,7 @@ extern "C" int f25_apply_batch_dev(f25_mesh *m, int npair, const double *omega, 
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
     TRY(product_ready(m, npair, mode & ~F25_APPLY_GRAPH));
-    return apply_core(m, npair, m->d_omky, m->d_omky + npair, mode, x, y, m->d_rec, m->d_vcf, omega);
+    return apply_core(m, npair, m->d_omky, m->d_omky + npair, mode, x, y, product_rec(m, npair), m->d_vcf, omega);
 }
 
 extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omega, const double *ky,
@@ -1478,7 +1498,8 @@ extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omeg
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
     TRY(product_ready(m, npair, F25_APPLY_F64));
-    TRY(apply_core(m, npair, m->d_omky, m->d_omky + npair, F25_APPLY_F64, u, r, m->d_rec, m->d_vcf, omega));
+    TRY(apply_core(m, npair, m->d_omky, m->d_omky + npair, F25_APPLY_F64, u, r, product_rec(m, npair), m->d_vcf,
+                   omega));
     const int gy = (int)std::min<int64_t>(256, std::max<int64_t>(1, m->g.ndof / 256));
     double *part = nullptr, *sums = nullptr;
     int rc = dalloc(&part, (size_t)gy * npair * 2);

@@ -103,6 +103,35 @@ def test_product(p, npml):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("p", [2, 3, 4])
+def test_product_both_sides_of_the_batch_rule(p):
+    """2,048 parallelograms: below 2^18 products the element-wise kernel, from
+    there on blocks at p2 (and at p3 in FP32).  The same pairs either way,
+    within the rounding of each kind."""
+    import torch
+    from fem25_amd import _lib
+    from fem25_amd.api import MeshInfo
+    m = cf.structured_mesh(64, 32, p, width=64e3, depth=32e3)
+    mi = MeshInfo(m)
+    mi.set_model(cf.layered_model(m, seed=11, n_anom=4, amp=0.1))
+    om, ky, _, _ = cf.freq_ky_batch(8, 16, 0.02, 0.1, 3500.0)
+    x = torch.randn(mi.ndof, 128, dtype=torch.complex128, device="cuda",
+                    generator=torch.Generator(device="cuda").manual_seed(5))
+    y = {}
+    for n in (127, 128):
+        xn = x[:, :n].contiguous()
+        for mode, xx in ((_lib.F25_APPLY_F64, xn), (_lib.F25_APPLY_F32, xn.to(torch.complex64))):
+            out = torch.empty_like(xx)
+            mi.apply_batch_dev(om[:n], ky[:n], xx, out, mode)
+            y[n, mode] = out.to(torch.complex128)
+    for (n, mode), v in y.items():
+        ref = y[127, _lib.F25_APPLY_F64]
+        e = torch.linalg.norm(v[:, :127] - ref, dim=0) / torch.linalg.norm(ref, dim=0)
+        assert float(e.max()) < (1e-12 if mode == _lib.F25_APPLY_F64 else 2e-6), (n, mode)
+    mi.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("disp", [False, True])
 @pytest.mark.parametrize("p", [2, 3, 4, 5, 6])
 def test_assembled_with_elements_per_omega(p, disp):

@@ -79,11 +79,15 @@ __global__ void k_aff_rec(int nelem, const int *__restrict__ ieng, const double 
     o[18] = o[19] = 0.0;
 }
 
-// 16 bytes per lane from global memory straight into LDS (l: the wave's base,
-// lane i's value lands at l + 16 i); complete after dma_wait.
+// 16 or 4 bytes per lane from global memory straight into LDS (l: the wave's
+// base, lane i's value lands at l + 16 i or l + 4 i); complete after dma_wait.
 __device__ __forceinline__ void dma16(const void *g, void *l) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)g,
                                      (__attribute__((address_space(3))) void *)l, 16, 0, 0);
+}
+__device__ __forceinline__ void dma4(const void *g, void *l) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)g,
+                                     (__attribute__((address_space(3))) void *)l, 4, 0, 0);
 }
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // the wave's own LDS accesses so far are complete, and stay before what follows
@@ -127,13 +131,13 @@ struct AfGather {
 // with v'_j; a: LDS, node (j, i) at a[(j NL + i) * STEP].  x holds column 0 on
 // entry and column 0 of the next component (an) on return: each column is
 // read while the one before it is summed.
-template <int NL, int STEP>
-__device__ __forceinline__ void af_first(const double *a, const double *an, const double *v, const double *d,
+template <int NL, int STEP, typename R>
+__device__ __forceinline__ void af_first(const R *a, const R *an, const double *v, const double *d,
                                          double *x, double *T1, double *T2) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
         double n[NL];
-        const double *p = i + 1 < NL ? a + (i + 1) * STEP : an;
+        const R *p = i + 1 < NL ? a + (i + 1) * STEP : an;
 #pragma unroll
         for (int j = 0; j < NL; ++j) n[j] = p[j * NL * STEP];
         double t1 = v[0] * x[0], t2 = d[0] * x[0];
@@ -231,7 +235,10 @@ __device__ __forceinline__ void af_rows(double *Y, double cq, double p1, double 
 // the way, at p4 / p6: scalar tables 2.17 / 5.81; loads waited for after the
 // stores 2.13 / 4.84; the three components' rows kept and stored together
 // 2.33 / 5.80; row addresses computed per row 2.05 / 4.75; the rows' values
-// loaded before the point loop 2.05 / 7.1 (registers).
+// loaded before the point loop 2.05 / 7.1 (registers).  complex64 vectors
+// through registers into LDS, widened on the way, instead of two pieces a
+// value straight into it: 120x60 p6 spills, 128 pairs 2.03 ms against 1.60
+// (p4, p5 within 2%).
 template <int NL, typename XT, bool RECT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_apply_af(
         const int *__restrict__ order, int nel, int nsplit, int nch, const double *__restrict__ rec,
@@ -243,11 +250,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     typedef AfTab<NL> TB;
     typedef decltype(XT().x) R;
     constexpr int NEE = S::NEE, PP = S::PP, PW = S::PW, LN = S::LN, ES = S::ES;
-    constexpr bool DIRECT = sizeof(XT) == 16;     // straight to LDS; float2 is widened through registers
-    constexpr int NG = (S::XS + 63) / 64;
+    // complex128 values lie whole in LDS, complex64 as real parts, then
+    // imaginary parts (two pieces of 4 bytes; widened as they are read)
+    constexpr bool WIDE = sizeof(XT) == 16;
+    constexpr int NG = (S::XS + 63) / 64, STEP = WIDE ? 2 : 1, IM = WIDE ? 1 : S::XS;
     extern __shared__ double sm[];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     double2 *sx = reinterpret_cast<double2 *>(sm) + wv * S::XS;
+    R *sv = reinterpret_cast<R *>(sx);
     double *sb = sm + S::NW * S::XS * 2 + wv * ES;
     uint64_t *sr = reinterpret_cast<uint64_t *>(sm + S::NW * (S::XS * 2 + ES)) + wv * 2 * NEE;   // read, then written
     double *st = sm + S::NW * (S::XS * 2 + ES + 2 * NEE);
@@ -278,7 +288,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
     for (int r = 0; r < NG; ++r) {
         const int s = lane + 64 * r;
-        if (s < S::XS && dp[r] < 0) sx[s] = make_double2(0.0, 0.0);
+        if (s < S::XS && dp[r] < 0) sv[s * STEP] = sv[s * STEP + IM] = 0;
         dp[r] = s < S::XS && dp[r] >= 0 ? dp[r] * 16 + s % PW : -1;
     }
 #pragma unroll
@@ -290,14 +300,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             sr[NEE + i] = reinterpret_cast<uint64_t>(row);
         }
     }
-    XT pre[DIRECT ? 1 : NG];
     auto get = [&](int p0) {
 #pragma unroll
         for (int r = 0; r < NG; ++r)
             if (dp[r] >= 0) {
                 const XT *src = x + ((size_t)(dp[r] >> 4) * npair + min(p0 + (dp[r] & 15), npair - 1));
-                if constexpr (DIRECT) dma16(src, sx + 64 * r);
-                else pre[r] = *src;
+                if constexpr (WIDE) dma16(src, sx + 64 * r);
+                else {
+                    dma4(src, sv + 64 * r);
+                    dma4(reinterpret_cast<const R *>(src) + 1, sv + IM + 64 * r);
+                }
             }
     };
     lds_wait();
@@ -313,28 +325,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const double rL = (rc[5] * h0 + rc[8] * h1) * we, rR = (rc[6] * h0 + rc[7] * h1) * we;
     const double lL = (rc[9] * h0 + rc[12] * h1) * we, lR = (rc[10] * h0 + rc[11] * h1) * we;
     const double mL = (rc[13] * h0 + rc[16] * h1) * we, mR = (rc[14] * h0 + rc[15] * h1) * we;
-    if constexpr (DIRECT) dma_wait();
+    dma_wait();
     for (int ch = part; ch < nch; ch += nsplit) {
         const int pair = ch * PW + pr;
         const bool live = lane < LN && pair < npair;
         const double w2 = -omn * omn, kv = im ? -kyn : kyn;
-        if constexpr (!DIRECT) {
-#pragma unroll
-            for (int r = 0; r < NG; ++r)
-                if (dp[r] >= 0) sx[lane + 64 * r] = make_double2((double)pre[r].x, (double)pre[r].y);
-            lds_wait();
-        }
         double T1[3][NL], T2[3][NL];
         {
             double v[NL], d[NL], c0[NL];
 #pragma unroll
             for (int j = 0; j < NL; ++j) { v[j] = st[eta * 16 + j]; d[j] = (RECT ? sz : 1.0) * st[eta * 16 + NL + j]; }
-            const double *a = reinterpret_cast<const double *>(sx) + 2 * pr;
-            auto at = [&](int c) { return a + c * PW * 2 + (c == 1 ? 1 - im : im); };
+            const R *a = sv + STEP * pr;
+            auto at = [&](int c) { return a + c * PW * STEP + (c == 1 ? 1 - im : im) * IM; };
 #pragma unroll
-            for (int j = 0; j < NL; ++j) c0[j] = at(0)[j * NL * 3 * PW * 2];
+            for (int j = 0; j < NL; ++j) c0[j] = at(0)[j * NL * 3 * PW * STEP];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) af_first<NL, 3 * PW * 2>(at(c), at(c < 2 ? c + 1 : 0), v, d, c0, T1[c], T2[c]);
+            for (int c = 0; c < 3; ++c) af_first<NL, 3 * PW * STEP>(at(c), at(c < 2 ? c + 1 : 0), v, d, c0, T1[c], T2[c]);
         }
         lds_wait();
         if (ch + nsplit < nch) {

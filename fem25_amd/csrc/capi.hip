@@ -1164,8 +1164,8 @@ static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt 
 // Whether a batch of the operator product takes them there (mode F64 or F32).
 // FP64 arithmetic runs at the rate of FP32 arithmetic without packed
 // instructions, so k_apply_af beats the blocks in both modes (FP32: their
-// matrix units) where the blocks are large (200x100 elements, 45 pairs, FP32:
-// p4 0.93 -> 0.72 ms, p5 2.24 -> 1.10, p6 4.42 -> 2.01) or the batch is too
+// matrix units) where the blocks are large (45 pairs, FP32: 200x100 p4 920 ->
+// 700 us, 97x61 p5 696 -> 403, 120x60 p6 1765 -> 746) or the batch is too
 // small to fill the chip with a workgroup or a few waves per element (FP32,
 // 40x20, 320 pairs: p2 178 -> 104 us, p3 212 -> 145; 200x100, 8 pairs: 108 ->
 // 85, 133 -> 112).  Blocks of p2 (and of p3 in FP32) cost little and lose less

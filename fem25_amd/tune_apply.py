@@ -7,7 +7,8 @@ on the GPU and reports the fastest.
 Every candidate runs on the same mesh, model and vectors; the time is the
 library's HIP-event figure for the product's launches (one per element
 colour).  The results of the candidates are compared with each other (they
-differ only in the order of floating-point sums).  The per-order defaults
+differ only in the order of floating-point sums), and all run the product on
+element blocks (row tiles asked for switch sum factorisation off).  The per-order defaults
 compiled into the library (apply_nrt_default in csrc/capi.hip) come from
 this script; f25_set_apply_tiles selects another candidate at run time.
 One JSON line per (order, candidate), then one per order with the fastest.

@@ -185,10 +185,12 @@ int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omega, const do
 int f25_apply_batch(f25_mesh *m, int npair, const double *omega, const double *ky, int mode,
                     const void *x, void *y);
 /* Tuning hook of the FP64 product (no counterpart in the reference, which
- * has no batched product): number of row tiles per output component, 0 =
- * the order's default.  Compiled candidates: p2, p3: 1, 2; p4: 1..3; p5,
- * p6: 2..4.  Rewrites the product's coefficient layout when the model is
- * set.  fem25_amd/tune_apply.py times the candidates. */
+ * has no batched product): number of row tiles per output component of the
+ * product on element blocks, 0 = the order's default (and parallelograms by
+ * sum factorisation).  Compiled candidates: p2, p3: 1, 2; p4: 1..3; p5, p6:
+ * 2..4.  Any other value than 0 sends every element through its blocks; their
+ * coefficient layout is written by the next product.
+ * fem25_amd/tune_apply.py times the candidates. */
 int f25_set_apply_tiles(f25_mesh *m, int nrt);
 
 /* ---- gradient ------------------------------------------------------------ */

@@ -31,10 +31,9 @@ def _p(a, t):
 
 def build(ref: bool = True) -> None:
     subprocess.run(["make", "-s", "liboracle.so"], cwd=_HERE, check=True)
-    if ref and os.path.isdir(os.environ.get("FEM25_REFERENCE", "/root/reference")):
-        subprocess.run(["make", "-s", "-j8", "ref",
-                        "REF=" + os.environ.get("FEM25_REFERENCE", "/root/reference")],
-                       cwd=_HERE, check=True)
+    src = os.environ.get("FEM25_REFERENCE", "/root/reference")
+    if ref and os.path.exists(os.path.join(src, "fwd_struc.h")):   # the sources, not an empty folder
+        subprocess.run(["make", "-s", "-j8", "ref", "REF=" + src], cwd=_HERE, check=True)
 
 
 def lib():

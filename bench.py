@@ -114,11 +114,13 @@ def main() -> int:
     k_ms = float(np.mean(kern_ms))
     # launches per step: one per element colour
     ncol = mi.ncolour
-    flops = 60.0 * nen * nen * mesh.nelem * npair          # useful block flops per step
-    bytes_alg = 2 * ndof * npair * 16 + 9 * nen * nen * 8 * mesh.nelem
-    achieved = flops / (k_ms * 1e-3)
+    flops = product_flops(mesh.nord + 1) * mesh.nelem * npair
+    # x read once, y written once, one record and one DOF map per element
+    bytes_alg = 2 * ndof * npair * 16 + (160 + 12 * nen) * mesh.nelem
+    rates = {"fp64": flops / (k_ms * 1e-3), "hbm": bytes_alg / (k_ms * 1e-3)}
+    bound = max(("hbm", PEAK_HBM), ("fp64", PEAK_FP64), key=lambda b: rates[b[0]] / b[1])[0]
     log(f"FP64 product: {ms_step:.3f} ms/step, kernels {k_ms:.3f} ms, {gdofs:.2f} Gdof/s, "
-        f"{achieved / 1e12:.2f} TFLOP/s")
+        f"{rates['fp64'] / 1e12:.2f} TFLOP/s, {rates['hbm'] / 1e9:.0f} GB/s of algorithmic bytes")
 
     if args.copy_calib:
         yc = torch.empty_like(x)
@@ -151,12 +153,13 @@ def main() -> int:
                                f"{shape['nfreq']} freq x {shape['nky']} ky = {npair} K(omega,ky) "
                                f"products per step",
                    "nelem": mesh.nelem, "nord": mesh.nord, "ndof": ndof, "npair": npair},
-        "roofline": {"bound": "mfma", "achieved": round(achieved / 1e12, 3), "peak": PEAK_FP64 / 1e12,
-                     "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP64, 4), "traffic": traffic,
-                     "traffic_source": traffic_src,
-                     "kernel": f"k_apply_v<{mesh.nord + 1}>",
-                     "compute": "FP64 FMA on the vector ALUs; on gfx950 their peak equals the FP64 "
-                                "MFMA peak (78.6 TFLOP/s)",
+        "roofline": {**roof(bound, rates[bound], "GB/s" if bound == "hbm" else "TFLOP/s"),
+                     "traffic": traffic, "traffic_source": traffic_src,
+                     "kernel": f"k_apply_af<{mesh.nord + 1}>",
+                     "compute": "sum factorisation at the (p + 1)-point Gauss rule, FP64 FMA on the "
+                                "vector ALUs (their peak equals the FP64 MFMA peak on gfx950)",
+                     "fp64_frac": round(rates["fp64"] / PEAK_FP64, 4),
+                     "hbm_frac": round(rates["hbm"] / PEAK_HBM, 4),
                      "launch_avg_ms": round(k_ms / ncol, 4),
                      "algorithmic_flops_per_launch": flops / ncol,
                      "algorithmic_bytes_per_launch": bytes_alg / ncol,
@@ -169,6 +172,22 @@ def main() -> int:
     print(json.dumps(out), flush=True)
     mi.close()
     return 0
+
+
+def product_flops(n1):
+    """Flops per (element, pair) of the sum-factorised product (n1 = p + 1):
+    two real problems, each with the 1-D pass along eta (12 n1^3), the fields
+    and their projection along xi (36 n1^3), the last pass along eta
+    (12 n1^3) and about 60 per point for the fluxes."""
+    return 120.0 * n1 * n1 * (n1 + 1)
+
+
+def gradient_flops(n1):
+    """Flops per (element, triple) of the gradient at the (p + 1)-point rule:
+    two real problems of two fields, each with the 1-D pass along eta
+    (12 n1^3), the fields along xi (18 n1^3) and about 25 per point for their
+    derivatives, and about 60 per point for the densities."""
+    return 120.0 * n1 ** 3 + 220.0 * n1 * n1
 
 
 def roof(bound, achieved, unit):
@@ -200,7 +219,7 @@ def extras(mi, mesh, model, L, torch, x, y, omega, ky, freq, py, npair, gdofs, g
     from fem25_amd import _lib
     ndof, nen, nq = mi.ndof, mi.nen, mi.nq1 * mi.nq1
     out = {}
-    # accuracy of the MFMA product against the assembled CSR operator (FP64)
+    # accuracy of the product against the assembled CSR operator (FP64)
     b = npair - 1
     s = torch.empty(mi.nz, dtype=torch.complex128, device="cuda")
     mi.asmble_dev(b"B", float(freq[b]), float(py[b]), s)
@@ -240,8 +259,9 @@ def extras(mi, mesh, model, L, torch, x, y, omega, ky, freq, py, npair, gdofs, g
                      "median_rel_err_vs_fp64": float(np.median(per)),
                      "rel_err_per_pair": [float(f"{v:.3e}") for v in per],
                      "kernel_ms": round(k_ms, 3),
-                     "roofline": roof("fp32_mfma", 60.0 * nen * nen * mesh.nelem * npair * (4 if "ref" in name else 1)
-                                      / (k_ms * 1e-3), "TFLOP/s")}
+                     "roofline": roof("fp32_mfma", 240.0 * nen * nen * mesh.nelem * npair / (k_ms * 1e-3), "TFLOP/s")
+                     if "ref" in name else
+                     roof("fp64", product_flops(mesh.nord + 1) * mesh.nelem * npair / (k_ms * 1e-3), "TFLOP/s")}
     del x32, y32, yr
     kern = {}
     # assembled FP64 operator: one pass over the CSR basis (HBM)
@@ -264,16 +284,16 @@ def extras(mi, mesh, model, L, torch, x, y, omega, ky, freq, py, npair, gdofs, g
     lam = torch.randn(npair, ndof, dtype=torch.complex128, device="cuda")
     gg = torch.zeros(mesh.nnpg, 3, dtype=torch.float64, device="cuda")
     k_ms, wall = timed(lambda: mi.gradient_dev(omega, ky, u, lam, gg), L, b"grad", 2)
-    # flops per (element, triple), sum factorised: two 1-D passes per field
-    # and component, 4 (12 N1^2 Q1 + 18 N1 Q1^2), plus ~150 per quadrature point
     n1, q1 = mesh.nord + 1, 2 * mesh.nord + 5
-    per = 4.0 * (12 * n1 * n1 * q1 + 18 * n1 * q1 * q1)
-    gfl = (per + 150.0 * nq) * mesh.nelem * npair
+    gfl = gradient_flops(n1) * mesh.nelem * npair
     kern["gradient"] = {"kernel_ms": round(k_ms, 3), "gradients_per_s": round(npair / (wall * 1e-3), 1),
                         "roofline": roof("fp64", gfl / (k_ms * 1e-3), "TFLOP/s")}
     out["gradients_per_s"] = kern["gradient"]["gradients_per_s"]
     # the FP32 gradient (complex64 fields, FP32 densities, FP64 sums) and its
     # error per field against the FP64 gradient
+    # (at the 2 p + 5 point rule; flops per (element, triple): two 1-D passes
+    # per field and component, 4 (12 N1^2 Q1 + 18 N1 Q1^2), plus ~150 per point)
+    gfl32 = (4.0 * (12 * n1 * n1 * q1 + 18 * n1 * q1 * q1) + 150.0 * nq) * mesh.nelem * npair
     u32, l32 = u.to(torch.complex64), lam.to(torch.complex64)
     g64 = torch.zeros_like(gg)
     g32 = torch.zeros_like(gg)
@@ -285,7 +305,7 @@ def extras(mi, mesh, model, L, torch, x, y, omega, ky, freq, py, npair, gdofs, g
             for p, nm in enumerate(("vp", "vs", "rho"))}
     kern["gradient_fp32"] = {"kernel_ms": round(k32, 3), "gradients_per_s": round(npair / (wall32 * 1e-3), 1),
                              "rel_err_vs_fp64_per_field": ferr,
-                             "roofline": roof("fp64", gfl / (k32 * 1e-3), "TFLOP/s")}
+                             "roofline": roof("fp64", gfl32 / (k32 * 1e-3), "TFLOP/s")}
     del u32, l32, g64, g32
     # pseudo-Hessian diagonal (host arrays, 8 wavefields)
     nt = 8
@@ -508,13 +528,13 @@ def cfmat_host(mi, inv, freq, py, wave):
 
 # rocprofv3 FETCH_SIZE / WRITE_SIZE summaries of the product, per workload
 TRAFFIC_PROFILES = {
-    "c2": "k_apply_v_f64_p4_200x100_128pairs.md",
-    "c5p6": "k_apply_v_f64_p6_400x200_192pairs.md",
+    "c2": "k_apply_af_f64_p4_200x100_128pairs.md",
+    "c5p6": "k_apply_af_f64_p6_400x200_192pairs.md",
 }
 
 
 def profiled_traffic(config: str):
-    """HBM bytes per k_apply_v launch from the committed rocprofv3 FETCH_SIZE /
+    """HBM bytes per k_apply_af launch from the committed rocprofv3 FETCH_SIZE /
     WRITE_SIZE summary of this workload (None when there is none)."""
     name = TRAFFIC_PROFILES.get(config)
     if name is None:

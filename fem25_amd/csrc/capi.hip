@@ -1121,11 +1121,7 @@ static int launch_blocks_f64(f25_mesh *m, const int *order, int n, const double 
     FAIL(F25_ERR_ARG, "unsupported order");
 }
 
-// Product of n parallelogram elements of one colour (k_apply_af).  Waves per
-// element: one per chunk of pairs until the launch has about 16,384 waves
-// (eight per CU, several times over), so that the element's setup is shared
-// by as many chunks as the mesh allows; at least four where there are as
-// many chunks, one workgroup per element.
+// Product of n parallelogram elements of one colour (k_apply_af).
 template <int NL, typename XT>
 static int launch_apply_af(f25_mesh *m, const int *order, int n, const int *lm_in, const int *lm_out,
                            const unsigned long long *first, const double *rec, const double *om, const double *kv,
@@ -1134,7 +1130,14 @@ static int launch_apply_af(f25_mesh *m, const int *order, int n, const int *lm_i
     auto kern = m->rect ? k_apply_af<NL, XT, true> : k_apply_af<NL, XT, false>;
     HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_apply));
     const int nch = (npair + S::PW - 1) / S::PW;
-    const int nsplit = std::min(nch, std::max(S::NW, (16384 + n - 1) / n));
+    // waves of an element: a multiple of a workgroup's, so that those share the
+    // lines of neighbouring chunks, and about 8,192 waves a launch, four times
+    // what the chip holds, as each wave starts with the element's addresses;
+    // one per chunk where there are fewer.
+    // (At least 16,384 waves, any count: 97x61, 75 pairs, p5 FP32 593 -> 521
+    // us, p4 500 -> 433, p3 304 -> 266; 48 sizes of p3..p6 1.026 times faster
+    // in the mean, 60x40, 75 pairs, p4 FP32 196 -> 212.)
+    const int nsplit = std::min(nch, S::NW * std::max(1, (8192 / n + S::NW / 2) / S::NW));
     const int64_t nwg = ((int64_t)n * nsplit + S::NW - 1) / S::NW;
     if (nwg > 0x7fffffff) FAIL(F25_ERR_ARG, "too many pairs for one launch");
     hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(256), S::lds_apply, m->st, order, n, nsplit, nch, rec, m->d_taf,
@@ -1165,7 +1168,7 @@ static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt 
 // FP64 arithmetic runs at the rate of FP32 arithmetic without packed
 // instructions, so k_apply_af beats the blocks in both modes (FP32: their
 // matrix units) where the blocks are large (45 pairs, FP32: 200x100 p4 920 ->
-// 700 us, 97x61 p5 696 -> 403, 120x60 p6 1765 -> 746) or the batch is too
+// 700 us, 97x61 p5 696 -> 380, 120x60 p6 1765 -> 669) or the batch is too
 // small to fill the chip with a workgroup or a few waves per element (FP32,
 // 40x20, 320 pairs: p2 178 -> 104 us, p3 212 -> 145; 200x100, 8 pairs: 108 ->
 // 85, 133 -> 112).  Blocks of p2 (and of p3 in FP32) cost little and lose less

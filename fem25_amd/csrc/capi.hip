@@ -108,6 +108,7 @@ struct f25_mesh_s {
     bool rect = true;   // the parallelograms' sides all lie along x and z
     int *d_aelem = nullptr, *d_gelem = nullptr;
     int naff = 0, ngen = 0;
+    int nin = 0, npar = 0;   // elements outside the PML, parallelograms among them
     // the same by colour: order splits into aorder and gorder
     int *d_aorder = nullptr, *d_gorder = nullptr;
     std::vector<int> acptr, gcptr;
@@ -195,8 +196,9 @@ struct f25_mesh_s {
     // FILL_UWAVE_QMESH; built on first use
     struct {
         bool built = false, uw = false;
-        std::vector<int> cptr, acptr, gcptr;     // all, parallelograms, the others
-        int *d_order = nullptr, *d_aorder = nullptr, *d_gorder = nullptr;
+        std::vector<int> cptr;
+        int *d_order = nullptr;
+        bool affine = false;                     // all of them parallelograms
         int *d_lm[4] = {};                       // E in, B out, B in, E out
         unsigned long long *d_first0 = nullptr;  // every row adds
         int *d_brows = nullptr;
@@ -355,6 +357,8 @@ static int upload_mesh(f25_mesh *m) {
     }
     m->naff = (int)ael.size();
     m->ngen = (int)gel.size();
+    m->nin = (int)(m->order.size() - m->pml_order.size());
+    m->npar = m->nin - m->ngen;
     TRY(upload(&m->d_aelem, ael.data(), ael.size(), s));
     TRY(upload(&m->d_gelem, gel.data(), gel.size(), s));
     split_order(m, m->order, m->cptr, ael, m->acptr, gel, m->gcptr);
@@ -549,7 +553,7 @@ extern "C" int f25_mesh_destroy(f25_mesh *m) {
     dfree(m->d_ew);
     dfree(m->d_omky);
     dfree(m->d_gn);
-    dfree(m->br.d_order); dfree(m->br.d_aorder); dfree(m->br.d_gorder); dfree(m->br.d_first0); dfree(m->br.d_brows); dfree(m->br.d_xz); dfree(m->br.d_comp);
+    dfree(m->br.d_order); dfree(m->br.d_first0); dfree(m->br.d_brows); dfree(m->br.d_xz); dfree(m->br.d_comp);
     dfree(m->br.d_pw);
     for (auto &q : m->br.d_lm) dfree(q);
     if (m->br.exec) (void)hipGraphExecDestroy(m->br.exec);
@@ -1159,9 +1163,9 @@ static int affine_colour(f25_mesh *m, const int *order, int n, const int *lm_in,
     FAIL(F25_ERR_ARG, "unsupported order");
 }
 
-// whether the product's parallelograms run in k_apply_af: it packs a DOF and
-// a pair into one register, and a row-tile count asked for (f25_set_apply_tiles)
-// means the block kernel
+// whether k_apply_af can take the product's parallelograms: it packs a DOF
+// and a pair into one register, and a row-tile count asked for
+// (f25_set_apply_tiles) means the block kernel
 static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt && m->g.ndof < (1 << 27); }
 
 // Whether a batch of the operator product takes them there (mode F64 or F32).
@@ -1177,8 +1181,7 @@ static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt 
 // 966; FP64 p2, 97x61: 45 pairs 117 / 123, 128 pairs 228 / 250.  The line lies
 // between 256,000 and 266,000 products of one element and one pair.
 static bool affine_batch(const f25_mesh *m, int npair, int mode) {
-    const int nl = mode == F25_APPLY_F32 ? 5 : 4;
-    return affine_product(m) && (m->tab.nl >= nl || (int64_t)m->d.nelem * npair < (1 << 18));
+    return affine_product(m) && sum_factorised(m->tab.nord, m->nin, m->npar, npair, mode == F25_APPLY_F32);
 }
 
 // what the product's launches read: zero rows and sink, and the element
@@ -1200,7 +1203,7 @@ static const double *product_rec(const f25_mesh *m, int npair) {
 // colour: the parallelograms by rec (null: as blocks too), the others by vcf
 static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair, const double2 *x, double2 *y,
                       const double *rec, const double *vcf) {
-    const bool aff = rec && affine_product(m);
+    const bool aff = rec != nullptr;
     for (size_t c = 0; c + 1 < m->cptr.size(); ++c) {
         const std::vector<int> &gp = aff ? m->gcptr : m->cptr;
         if (aff && m->acptr[c + 1] > m->acptr[c])
@@ -1577,11 +1580,8 @@ static int bielak_prepare(f25_mesh *m) {
     std::vector<int> brows;
     for (int d = 0; d < m->g.ndof; ++d)
         if (isb[d]) brows.push_back(d);
-    std::vector<int> ao, go;
-    split_order(m, ord, ptr, ao, B.acptr, go, B.gcptr);
+    B.affine = std::all_of(ring.begin(), ring.end(), [&](int e) { return m->affine[e] != 0; });
     TRY(upload(&B.d_order, ord.data(), ord.size(), m->st));
-    TRY(upload(&B.d_aorder, ao.data(), ao.size(), m->st));
-    TRY(upload(&B.d_gorder, go.data(), go.size(), m->st));
     for (int k = 0; k < 4; ++k) TRY(upload(&B.d_lm[k], lmv[k].data(), lmv[k].size(), m->st));
     TRY(dalloc(&B.d_first0, (size_t)nelem));
     fill_async(B.d_first0, (size_t)nelem, 0ull, m->st);
@@ -1618,17 +1618,21 @@ static int ring_blocks(f25_mesh *m, int pass, const int *order, int n, const dou
     FAIL(F25_ERR_ARG, "unsupported order");
 }
 
+// The ring's elements are too few for a launch of each kind per colour to pay
+// (sum_factorised): on blocks unless all are parallelograms.
+static bool ring_affine(const f25_mesh *m) { return affine_product(m) && m->br.affine; }
+
 static int ring_pass(f25_mesh *m, int pass, const double *om, const double *kv, int npair, const double2 *x,
                      double2 *y) {
     auto &B = m->br;
-    const bool aff = affine_product(m);
     for (size_t c = 0; c + 1 < B.cptr.size(); ++c) {
-        const std::vector<int> &gp = aff ? B.gcptr : B.cptr;
-        if (aff && B.acptr[c + 1] > B.acptr[c])
-            TRY(affine_colour(m, B.d_aorder + B.acptr[c], B.acptr[c + 1] - B.acptr[c], B.d_lm[2 * pass],
-                              B.d_lm[2 * pass + 1], B.d_first0, m->d_rec, om, kv, npair, x, y));
-        if (gp[c + 1] > gp[c])
-            TRY(ring_blocks(m, pass, (aff ? B.d_gorder : B.d_order) + gp[c], gp[c + 1] - gp[c], om, kv, npair, x, y));
+        const int n = B.cptr[c + 1] - B.cptr[c], *order = B.d_order + B.cptr[c];
+        if (!n) continue;
+        if (ring_affine(m))
+            TRY(affine_colour(m, order, n, B.d_lm[2 * pass], B.d_lm[2 * pass + 1], B.d_first0, m->d_rec, om, kv, npair, x,
+                              y));
+        else
+            TRY(ring_blocks(m, pass, order, n, om, kv, npair, x, y));
     }
     return 0;
 }
@@ -1636,8 +1640,7 @@ static int ring_pass(f25_mesh *m, int pass, const double *om, const double *kv, 
 // what the ring's launches read (bielak_prepare first)
 static int ring_ready(f25_mesh *m, int npair) {
     TRY(ensure_vpad(m, npair));
-    const std::vector<int> &gp = affine_product(m) ? m->br.gcptr : m->br.cptr;
-    return gp.back() ? ensure_vcf(m) : 0;
+    return ring_affine(m) ? 0 : ensure_vcf(m);
 }
 
 // the effective force's launches (bielak_prepare and ring_ready first):
@@ -3340,7 +3343,8 @@ extern "C" int f25_gn_fv(f25_mesh *m, int ntrip, const double *omega, const doub
     TRY(upload(&d_l, dl.data(), n, m->st));
     TRY(upload(&d_m, dm.data(), n, m->st));
     // the perturbation's records, and its blocks for elements of general shape
-    const bool aff = affine_product(m), blocks = !aff || m->ngen;
+    const bool aff = affine_product(m) && (!m->ngen || affine_batch(m, ntrip, F25_APPLY_F64));
+    const bool blocks = !aff || m->ngen;
     int r = 0;
     if (aff) {
         if (!m->d_drec) r = dalloc(&m->d_drec, (size_t)m->d.nelem * AFR);
@@ -3481,6 +3485,12 @@ extern "C" int f25_gn_diag(f25_mesh *m, int ntrip, const double *omega, const do
     }
     dfree(du); dfree(dcols); dfree(dd);
     return r;
+}
+
+extern "C" int f25_selftest_route(int nord, int64_t nin, int64_t npar, int64_t npair, int mode) {
+    if (nord < 2 || nord > 6 || npar < 0 || npar > nin || npair <= 0 || (mode != F25_APPLY_F64 && mode != F25_APPLY_F32))
+        return -1;
+    return sum_factorised(nord, nin, npar, npair, mode == F25_APPLY_F32) ? 1 : 0;
 }
 
 // Workgroup residency: the most workgroups of nt threads, holding vgprs

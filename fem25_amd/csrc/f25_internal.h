@@ -29,6 +29,9 @@ void gll_nodes(int n, double *x, double *w);
 // (2 nl <= 14 values), at 14 and 15 w h0 and w h1; after the rows h0, h1 and
 // w at the points (h0 = (1 - s)/2, h1 = (1 + s)/2)
 std::vector<double> af_table(const Tables &t);
+// whether a batched product of npair pairs takes its parallelograms by sum
+// factorisation: nin elements outside the PML, npar of them parallelograms
+bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npair, bool fp32);
 
 // Host-side mesh graph (GEN_GRAPH25 numbering, graph25_driver.f90:30-86).
 struct Graph {

@@ -222,6 +222,27 @@ std::vector<double> af_table(const Tables &t) {
     return o;
 }
 
+// On a mesh that holds other elements too, both kinds are launched for every
+// colour, one after the other: worth it where the mesh is large enough that
+// the blocks of a colour are more than one launch's latency, and the
+// parallelograms are at least half of the elements.  Measured on MI355X, all
+// on blocks / both kinds, a tenth of the elements general, 8 pairs: FP64
+// 64x32 p5 221 / 176 us, 97x61 p3 160 / 126, p4 310 / 204, p6 985 / 332, but
+// 40x20 p4 122 / 158, 97x61 p2 84 / 98; FP32 97x61 p5 391 / 254, 200x100 p4
+// 422 / 284, but 97x61 p3 68 / 103, p4 153 / 174.  Larger batches of low order
+// gain nothing: 97x61, 45 pairs, FP64 p3 214 / 240, p4 380 / 402.
+bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npair, bool fp32) {
+    if (npar != nin) {
+        struct Least { int64_t nelem, most; };   // elements, pairs
+        constexpr int64_t never = INT64_MAX, any = INT64_MAX;
+        constexpr Least f64[5] = {{16384, 16}, {4096, 16}, {4096, 24}, {4096, any}, {2048, any}};
+        constexpr Least f32[5] = {{never, 0}, {never, 0}, {16384, any}, {4096, any}, {4096, any}};
+        const Least l = (fp32 ? f32 : f64)[nord - 2];
+        return 2 * npar >= nin && nin >= l.nelem && npair <= l.most;
+    }
+    return nord >= (fp32 ? 4 : 3) || nin * npair < (1 << 18);
+}
+
 // ---------------------------------------------------------------------------
 // Bilinear position of GLL point (xi, eta) in element e (CSF2DND, csf2d.f:135).
 void gll_xz(const f25_mesh_desc &d, int e, double xi, double eta, double &x, double &z) {

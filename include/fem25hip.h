@@ -447,6 +447,11 @@ const char *f25_last_error(void);
  * the operand/result lane layout the batched product relies on; *maxerr is
  * the largest deviation (0 when the layout holds). */
 int f25_selftest_mfma(double *maxerr);
+/* Which way a batched product takes its parallelogram elements: 1 by sum
+ * factorisation, 0 on element blocks as the others, -1 for arguments out of
+ * range.  nin elements outside the PML, npar of them parallelograms, mode
+ * F25_APPLY_F64 or F25_APPLY_F32. */
+int f25_selftest_route(int nord, int64_t nin, int64_t npar, int64_t npair, int mode);
 /* Workgroup residency on the current device: *groups_per_cu = the most
  * workgroups of nt threads (192, 256, 320, 384 or 512) holding vgprs
  * registers per lane (128 or 168) and lds bytes of LDS that are resident

@@ -1,0 +1,124 @@
+"""Which elements of a batched product run by sum factorisation and which on
+their blocks: the rule at the sizes where both were timed, and the products of
+meshes that hold both kinds on the two routes."""
+from __future__ import annotations
+
+import functools
+
+import numpy as np
+import pytest
+
+from fem25_amd import _lib
+from fem25_amd import configs as cf
+
+F64, F32 = _lib.F25_APPLY_F64, _lib.F25_APPLY_F32
+
+
+def pw(p: int) -> int:
+    """Complex vectors of one wave: half of the even number of (p + 1)-lane groups in 64."""
+    return (64 // (p + 1)) // 2
+
+
+def row_tiles(p: int) -> int:
+    """The order's own row tiles: asked for, every element runs on its blocks."""
+    return 1 if p <= 4 else 2
+
+
+def general(m) -> np.ndarray:
+    """Elements that are no parallelograms (coordinates exact in FP64)."""
+    x, z = m.xlocs[m.ieng - 1], m.zlocs[m.ieng - 1]
+    return sum(np.abs(v[:, 0] - v[:, 1] + v[:, 2] - v[:, 3]) for v in (x, z)) > 0
+
+
+def mixed_mesh(nx, nz, p, every=37, shear=0.25, **kw):
+    """A sheared mesh with every 37th anchor off the outer sides displaced."""
+    m = cf.structured_mesh(nx, nz, p, width=1e3 * nx, depth=1e3 * nz, **kw)
+    m.xlocs += shear * m.zlocs
+    cn = np.frombuffer(m.cnnpg, "S2")
+    ix, iz = np.arange(m.nnpg) % (nx + 1), np.arange(m.nnpg) // (nx + 1)
+    a = np.flatnonzero((cn != b"AA") & (ix > 0) & (ix < nx) & (iz > 0) & (iz < nz))[::every]
+    m.xlocs[a] += 155.0
+    m.zlocs[a] -= 85.0
+    return m
+
+
+@functools.lru_cache(maxsize=1)
+def handle(nx, nz, p, every):
+    from fem25_amd.api import MeshInfo
+    m = mixed_mesh(nx, nz, p, every) if every else cf.structured_mesh(nx, nz, p, width=1e3 * nx, depth=1e3 * nz)
+    mi = MeshInfo(m)
+    mi.set_model(cf.layered_model(m, seed=11, n_anom=4, amp=0.1))
+    return mi
+
+
+def batch(n: int):
+    om, ky, _, _ = cf.freq_ky_batch(3, (n + 2) // 3, 0.02, 0.1, 3500.0)
+    return om[:n], ky[:n]
+
+
+def vectors(mi, n, seed=5):
+    import torch
+    return torch.randn(mi.ndof, n, dtype=torch.complex128, device="cuda",
+                       generator=torch.Generator(device="cuda").manual_seed(seed))
+
+
+def product(mi, om, ky, x, mode=F64, tiles=0):
+    import torch
+    y = torch.full_like(x, complex(float("nan"), float("nan")))
+    mi.set_apply_tiles(tiles)
+    mi.apply_batch_dev(om, ky, x, y, mode)
+    mi.set_apply_tiles(0)
+    return y
+
+
+def err(a, b):
+    """The largest normwise error of a column."""
+    import torch
+    return float((torch.linalg.norm(a - b, dim=0) / torch.linalg.norm(b, dim=0)).max())
+
+
+# (order, elements, pairs, mode, sum factorisation faster) as timed, a tenth to half of the elements general
+@pytest.mark.parametrize("p,nin,n,mode,sf", [
+    (2, 800, 8, F64, False), (2, 5917, 8, F64, False), (2, 20000, 8, F64, True), (2, 20000, 40, F64, False),
+    (3, 2048, 8, F64, False), (3, 5917, 8, F64, True), (3, 5917, 45, F64, False),
+    (4, 800, 1, F64, False), (4, 5917, 24, F64, True), (4, 5917, 45, F64, False), (5, 5917, 128, F64, True),
+    (6, 800, 75, F64, False), (6, 2048, 75, F64, True),
+    (2, 20000, 1, F32, False), (3, 20000, 40, F32, False), (4, 5917, 8, F32, False), (4, 20000, 40, F32, True),
+    (5, 2048, 24, F32, False), (5, 5917, 45, F32, True), (6, 800, 8, F32, False), (6, 5917, 1, F32, True)])
+def test_rule_of_mixed_meshes(p, nin, n, mode, sf):
+    route = _lib.load().f25_selftest_route
+    assert route(p, nin, nin * 3 // 4, n, mode) == sf
+    assert route(p, nin, nin // 10, n, mode) == 0       # few parallelograms: one launch a colour
+    assert route(p, nin, 0, n, mode) == 0               # none but the PML elements
+
+
+def test_rule_refuses_what_there_is_not():
+    route = _lib.load().f25_selftest_route
+    for a in ((1, 10, 10, 1, F64), (7, 10, 10, 1, F64), (4, 10, 11, 1, F64), (4, 10, 10, 0, F64), (4, 10, 10, 1, 99)):
+        assert route(*a) == -1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p,nx,nz,n,mode", [
+    (2, 130, 128, 3, F64), (3, 68, 61, 9, F64), (4, 68, 61, 24, F64), (5, 68, 61, 41, F64), (6, 64, 32, 65, F64),
+    (4, 130, 128, 7, F32), (5, 68, 61, 6, F32), (6, 68, 61, 5, F32)])
+def test_product_of_both_kinds(p, nx, nz, n, mode):
+    """Meshes large enough that each colour launches both kernels, some waves
+    with a second chunk of pairs: the product on blocks alone (FP64, other
+    points and sums: within a few hundred roundings), and in FP32 the FP64
+    product (whose blocks' FP32 sums are known to 2e-6)."""
+    import torch
+    mi = handle(nx, nz, p, 37)
+    g = general(mi.mesh)
+    assert 0 < np.count_nonzero(g) < g.size // 2
+    assert _lib.load().f25_selftest_route(p, g.size, int(g.size - np.count_nonzero(g)), n, mode) == 1
+    om, ky = batch(n)
+    x = vectors(mi, n)
+    if mode == F32:
+        x32 = x.to(torch.complex64)
+        got, x = product(mi, om, ky, x32, F32).to(torch.complex128), x32.to(torch.complex128)
+    else:
+        got = product(mi, om, ky, x)
+    e = err(got, product(mi, om, ky, x, tiles=row_tiles(p)))
+    print(f"p{p} {nx}x{nz} {n} pairs mode {mode}: {e:.2e}", flush=True)
+    assert e < (2e-6 if mode == F32 else 1e-13)

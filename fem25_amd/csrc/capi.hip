@@ -1168,18 +1168,7 @@ static int affine_colour(f25_mesh *m, const int *order, int n, const int *lm_in,
 // (f25_set_apply_tiles) means the block kernel
 static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt && m->g.ndof < (1 << 27); }
 
-// Whether a batch of the operator product takes them there (mode F64 or F32).
-// FP64 arithmetic runs at the rate of FP32 arithmetic without packed
-// instructions, so k_apply_af beats the blocks in both modes (FP32: their
-// matrix units) where the blocks are large (45 pairs, FP32: 200x100 p4 920 ->
-// 700 us, 97x61 p5 696 -> 380, 120x60 p6 1765 -> 669) or the batch is too
-// small to fill the chip with a workgroup or a few waves per element (FP32,
-// 40x20, 320 pairs: p2 178 -> 104 us, p3 212 -> 145; 200x100, 8 pairs: 108 ->
-// 85, 133 -> 112).  Blocks of p2 (and of p3 in FP32) cost little and lose less
-// on large batches: FP32, blocks / k_apply_af: 97x61, 45 pairs p3 141 / 163,
-// 128 pairs p2 193 / 221, p3 254 / 360, 200x100, 128 pairs 519 / 570, 695 /
-// 966; FP64 p2, 97x61: 45 pairs 117 / 123, 128 pairs 228 / 250.  The line lies
-// between 256,000 and 266,000 products of one element and one pair.
+// whether a batch of the operator product takes them there (mode F64 or F32)
 static bool affine_batch(const f25_mesh *m, int npair, int mode) {
     return affine_product(m) && sum_factorised(m->tab.nord, m->nin, m->npar, npair, mode == F25_APPLY_F32);
 }

@@ -222,6 +222,24 @@ std::vector<double> af_table(const Tables &t) {
     return o;
 }
 
+// Where parallelograms run by sum factorisation.  FP64 arithmetic runs at the
+// rate of FP32 arithmetic without packed instructions, so it beats the blocks
+// in both types (FP32: their matrix units) where the blocks are large (FP32,
+// 24 pairs, 200x100 p4 592 -> 426 us; p3 and up in FP64, p4 and up in FP32).
+// Blocks of p2, and of p3 in FP32, cost little, and one read of them serves up
+// to 64 pairs: they win on large batches.  Measured on MI355X, blocks / sum
+// factorisation, us:
+//   FP64 p2  97x61: 40 pairs 98 / 98, 44 101 / 114, 64 112 / 131; 140x80: 24
+//            133 / 120; 200x100: 24 234 / 173, 48 295 / 318; 64x32: 48 65 / 65,
+//            64 68 / 81; 40x20: 100 64 / 60, 160 67 / 79
+//   FP32 p2  97x61: 20 pairs 72 / 64, 24 72 / 83; 140x80: 20 103 / 88, 23 104 /
+//            113; 200x100: 16 125 / 120, 24 146 / 160; with a workgroup per
+//            element the blocks of a small mesh leave the chip idle: 40x20:
+//            240 141 / 82, 64x32: 128 105 / 99
+//   FP32 p3  97x61: 8 pairs 68 / 61, 16 80 / 83, 20 87 / 106, 44 121 / 166;
+//            140x80: 16 109 / 119, 20 123 / 154; 200x100: 16 178 / 169, 24 212 /
+//            224, 48 321 / 457; 64x32: 48 86 / 83, 64 87 / 93; 40x20: 320 197 / 144
+//
 // On a mesh that holds other elements too, both kinds are launched for every
 // colour, one after the other: worth it where the mesh is large enough that
 // the blocks of a colour are more than one launch's latency, and the
@@ -240,7 +258,9 @@ bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npair, bool fp3
         const Least l = (fp32 ? f32 : f64)[nord - 2];
         return 2 * npar >= nin && nin >= l.nelem && npair <= l.most;
     }
-    return nord >= (fp32 ? 4 : 3) || nin * npair < (1 << 18);
+    if (nord >= (fp32 ? 4 : 3)) return true;
+    if (fp32 && nin <= (nord == 2 ? 2048 : 1024)) return true;
+    return npair <= (fp32 ? (nord == 2 ? 20 : 16) : 40) || nin * npair <= 3 << 15;
 }
 
 // ---------------------------------------------------------------------------

@@ -92,6 +92,19 @@ def test_rule_of_mixed_meshes(p, nin, n, mode, sf):
     assert route(p, nin, 0, n, mode) == 0               # none but the PML elements
 
 
+# parallelograms alone: (order, elements, pairs, mode, sum factorisation faster) as timed
+@pytest.mark.parametrize("p,nin,n,mode,sf", [
+    (2, 800, 160, F64, False), (2, 2048, 48, F64, True), (2, 2048, 64, F64, False), (2, 5917, 40, F64, True),
+    (2, 5917, 44, F64, False), (2, 11200, 24, F64, True), (2, 20000, 24, F64, True), (2, 20000, 48, F64, False),
+    (3, 20000, 128, F64, True), (2, 800, 640, F32, True), (2, 2048, 128, F32, True), (2, 5917, 20, F32, True),
+    (2, 5917, 24, F32, False), (2, 11200, 23, F32, False), (2, 20000, 24, F32, False), (3, 800, 640, F32, True),
+    (3, 2048, 48, F32, True), (3, 2048, 64, F32, False), (3, 5917, 8, F32, True), (3, 5917, 20, F32, False),
+    (3, 5917, 44, F32, False), (3, 11200, 23, F32, False), (3, 20000, 16, F32, True), (3, 20000, 24, F32, False),
+    (4, 20000, 128, F32, True)])
+def test_rule_of_parallelograms(p, nin, n, mode, sf):
+    assert _lib.load().f25_selftest_route(p, nin, nin, n, mode) == sf
+
+
 def test_rule_refuses_what_there_is_not():
     route = _lib.load().f25_selftest_route
     for a in ((1, 10, 10, 1, F64), (7, 10, 10, 1, F64), (4, 10, 11, 1, F64), (4, 10, 10, 0, F64), (4, 10, 10, 1, 99)):
@@ -122,3 +135,28 @@ def test_product_of_both_kinds(p, nx, nz, n, mode):
     e = err(got, product(mi, om, ky, x, tiles=row_tiles(p)))
     print(f"p{p} {nx}x{nz} {n} pairs mode {mode}: {e:.2e}", flush=True)
     assert e < (2e-6 if mode == F32 else 1e-13)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p,nx,nz,n,mode", [
+    (2, 97, 61, 40, F64), (2, 97, 61, 41, F64), (2, 97, 61, 20, F32), (2, 97, 61, 21, F32),
+    (3, 97, 61, 16, F32), (3, 97, 61, 17, F32), (2, 64, 32, 170, F32), (3, 40, 20, 300, F32)])
+def test_product_both_sides_of_the_pair_rule(p, nx, nz, n, mode):
+    """Parallelograms alone, on either side of the number of pairs, and batches
+    whose waves take a second chunk of pairs, against blocks in FP64.  In FP32
+    a value is rounded when stored, up to four times (a corner node's
+    elements), each within 2^-24 of the partial sum; the blocks' sums in FP32
+    are known to 2e-6."""
+    import torch
+    mi = handle(nx, nz, p, 0)
+    sf = _lib.load().f25_selftest_route(p, nx * nz, nx * nz, n, mode)
+    om, ky = batch(n)
+    x = vectors(mi, n)
+    if mode == F32:
+        x32 = x.to(torch.complex64)
+        got, x = product(mi, om, ky, x32, F32).to(torch.complex128), x32.to(torch.complex128)
+    else:
+        got = product(mi, om, ky, x)
+    e = err(got, product(mi, om, ky, x, tiles=row_tiles(p)))
+    print(f"p{p} {nx}x{nz} {n} pairs mode {mode} route {sf}: {e:.2e}", flush=True)
+    assert e < (1e-13 if mode == F64 else 2.4e-7 if sf else 2e-6)

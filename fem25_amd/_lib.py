@@ -26,6 +26,7 @@ class MeshDesc(C.Structure):
 
 F25_C64, F25_C128 = 0, 1
 F25_APPLY_F64, F25_APPLY_F32, F25_APPLY_F32_REFINED = 0, 1, 2
+F25_ROUTE_GRADIENT = 64   # f25_selftest_route: the FP64 gradient
 F25_APPLY_GRAPH = 16   # or'ed with F25_APPLY_F64: replay a captured HIP graph
 F25_ERR_ARG, F25_ERR_HIP, F25_ERR_STATE = 1, 4, 8    # status codes of fem25hip.h
 

@@ -1927,6 +1927,8 @@ static int grad_launch(f25_mesh *m, int ntrip, const double *d_om, const double 
                        bool fp32) {
     HIPCHK(hipEventRecord(m->ev0, m->st));
     if (fp32) return grad_general<float>(m, nullptr, m->d.nelem, ntrip, d_om, d_ky, u, l);
+    if (!grad_sum_factorised(m->nin, m->npar, ntrip))
+        return grad_general<double>(m, nullptr, m->d.nelem, ntrip, d_om, d_ky, u, l);
     const double2 *ud = (const double2 *)u, *ld = (const double2 *)l;
     if (m->naff) switch (m->tab.nl) {
         case 3: TRY(grad_affine<3>(m, ntrip, d_om, d_ky, ud, ld)); break;
@@ -3477,8 +3479,10 @@ extern "C" int f25_gn_diag(f25_mesh *m, int ntrip, const double *omega, const do
 }
 
 extern "C" int f25_selftest_route(int nord, int64_t nin, int64_t npar, int64_t npair, int mode) {
-    if (nord < 2 || nord > 6 || npar < 0 || npar > nin || npair <= 0 || (mode != F25_APPLY_F64 && mode != F25_APPLY_F32))
+    if (nord < 2 || nord > 6 || npar < 0 || npar > nin || npair <= 0 ||
+        (mode != F25_APPLY_F64 && mode != F25_APPLY_F32 && mode != F25_ROUTE_GRADIENT))
         return -1;
+    if (mode == F25_ROUTE_GRADIENT) return grad_sum_factorised(nin, npar, npair) ? 1 : 0;
     return sum_factorised(nord, nin, npar, npair, mode == F25_APPLY_F32) ? 1 : 0;
 }
 

@@ -32,6 +32,8 @@ std::vector<double> af_table(const Tables &t);
 // whether a batched product of npair pairs takes its parallelograms by sum
 // factorisation: nin elements outside the PML, npar of them parallelograms
 bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npair, bool fp32);
+// the same for the FP64 gradient of ntrip triples
+bool grad_sum_factorised(int64_t nin, int64_t npar, int64_t ntrip);
 
 // Host-side mesh graph (GEN_GRAPH25 numbering, graph25_driver.f90:30-86).
 struct Graph {

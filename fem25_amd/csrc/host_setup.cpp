@@ -263,6 +263,18 @@ bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npair, bool fp3
     return npair <= (fp32 ? (nord == 2 ? 20 : 16) : 40) || nin * npair <= 3 << 15;
 }
 
+// The gradient of a mesh that holds both kinds is one launch of each: on the
+// general points alone where the parallelograms are hardly any (or only the
+// PML elements, which both kernels skip), or few triples of a small mesh leave
+// each launch at its latency.  Measured on MI355X, general points / both
+// kinds: half of 40x20 elements general, p6, one triple 63.0 / 69.8 us, 3 81.6 /
+// 84.2, 4 92.5 / 92.0, 8 132 / 125; p4 one 60.9 / 63.1, 4 72.9 / 69.4; half of 97x61,
+// p6, one 138 / 123; nine tenths of 97x61, p4, 4 triples 168 / 163, 45 970 / 893, of
+// 40x20, p6, 4 93 / 99, p4, 45 218 / 198; all of 40x20 but two PML rings, p6, 45 triples 434 / 461.
+bool grad_sum_factorised(int64_t nin, int64_t npar, int64_t ntrip) {
+    return npar == nin || npar * ntrip >= 2048 || (ntrip >= 4 && 4 * npar >= nin);
+}
+
 // ---------------------------------------------------------------------------
 // Bilinear position of GLL point (xi, eta) in element e (CSF2DND, csf2d.f:135).
 void gll_xz(const f25_mesh_desc &d, int e, double xi, double eta, double &x, double &z) {

@@ -105,6 +105,15 @@ def test_rule_of_parallelograms(p, nin, n, mode, sf):
     assert _lib.load().f25_selftest_route(p, nin, nin, n, mode) == sf
 
 
+@pytest.mark.parametrize("nin,npar,n,sf", [
+    (800, 800, 1, True), (800, 400, 1, False), (800, 400, 4, True), (5917, 3000, 1, True), (5917, 600, 1, False),
+    (5917, 600, 4, True), (5917, 100, 8, False), (800, 80, 4, False),
+    (800, 80, 45, True), (480, 0, 45, False)])
+def test_rule_of_the_gradient(nin, npar, n, sf):
+    for p in (2, 4, 6):
+        assert _lib.load().f25_selftest_route(p, nin, npar, n, _lib.F25_ROUTE_GRADIENT) == sf
+
+
 def test_rule_refuses_what_there_is_not():
     route = _lib.load().f25_selftest_route
     for a in ((1, 10, 10, 1, F64), (7, 10, 10, 1, F64), (4, 10, 11, 1, F64), (4, 10, 10, 0, F64), (4, 10, 10, 1, 99)):
@@ -160,3 +169,23 @@ def test_product_both_sides_of_the_pair_rule(p, nx, nz, n, mode):
     e = err(got, product(mi, om, ky, x, tiles=row_tiles(p)))
     print(f"p{p} {nx}x{nz} {n} pairs mode {mode} route {sf}: {e:.2e}", flush=True)
     assert e < (1e-13 if mode == F64 else 2.4e-7 if sf else 2e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p", [2, 4, 6])
+def test_gradient_of_both_kinds_with_pml(p):
+    """PML elements, parallelograms and elements of general shape in one mesh:
+    one triple on the general points alone, more on both, against the oracle."""
+    import oracle
+    from tests import test_affine as ta
+    m, mod, pml, g = ta.case(p, 2)
+    mi = ta.handle(p, 2)
+    n = pw(p) + 1
+    om, ky, f, py = ta.batch(n)
+    u, lam = cf.seeded_complex(g.ndof, batch=n, seed=1), cf.seeded_complex(g.ndof, batch=n, seed=2)
+    each = [oracle.grad_exact(m, mod, g, f[b], py[b], u[b], lam[b], pml)[1] for b in range(n)]
+    for k in (1, n):
+        assert _lib.load().f25_selftest_route(p, 16, 12, k, _lib.F25_ROUTE_GRADIENT) == (k > 1)
+        ref, got = sum(each[:k]), mi.gradient(om[:k], ky[:k], u[:k], lam[:k])
+        for c in range(3):
+            assert ta.err(got[:, c], ref[:, c]) < 1e-12, (k, c)

@@ -123,6 +123,8 @@ struct f25_mesh_s {
     // element blocks and coefficients that hold the current model: built by the
     // first call that reads them (the parallelograms' products do not)
     bool blk_ok = false, blk32_ok = false, vcf_ok = false;
+    // the FP32 copies were read for the current model, and for the one before
+    bool blk32_read = false, blk32_want = false;
     double *d_dblk = nullptr;   // blocks of a model perturbation (GN products)
     double *d_drec = nullptr;   // element records of a model perturbation
     double *d_vcf = nullptr;    // d_blk in the coefficient layout of the FP64 product (k_apply_v)
@@ -648,7 +650,12 @@ static int vcoef(f25_mesh *m, const double *blk, double **vcf);
 // blocks were most of its time (k_blocks and k_vcoef, 1.6 ms of 1.9 per model
 // and 16 products at 120x61 p4).
 static int ensure_blocks(f25_mesh *m, bool fp32) {
+    m->blk32_read |= fp32;
     if (m->blk_ok && (m->blk32_ok || !fp32)) return 0;
+    // one pass for all of them where the last model needed the FP32 copies
+    // too: a second one for a program that runs both products (40x20 p6, one
+    // pair in FP64 and FP32 per model 1.86 -> 2.92 ms)
+    fp32 = fp32 || m->blk32_want;
     const size_t nb = (size_t)m->d.nelem * NBLK * m->tab.nen * m->tab.nen;
     if (!m->d_blk) TRY(dalloc(&m->d_blk, nb));
     if (fp32) {
@@ -710,6 +717,8 @@ extern "C" int f25_set_model(f25_mesh *m, const double *dens, const double *ecoe
     HIPCHK(hipGetLastError());
     TRY(check_err(m));
     m->blk_ok = m->blk32_ok = m->vcf_ok = false;
+    m->blk32_want = m->blk32_read;
+    m->blk32_read = false;
     m->have_model = true;
     m->basis_ok = false;
     m->pa.valid = false;

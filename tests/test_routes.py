@@ -189,3 +189,48 @@ def test_gradient_of_both_kinds_with_pml(p):
         ref, got = sum(each[:k]), mi.gradient(om[:k], ky[:k], u[:k], lam[:k])
         for c in range(3):
             assert ta.err(got[:, c], ref[:, c]) < 1e-12, (k, c)
+
+
+@pytest.mark.gpu
+def test_blocks_of_both_types_in_one_pass():
+    """Elements of general shape under one new model after another, each applied
+    in FP64 and FP32: results of a handle that knows this model only, and the
+    blocks built once a model, not once a type (their pass is most of the time:
+    both products cost well under one product of each kind with a model of its
+    own)."""
+    import time
+
+    import torch
+    from fem25_amd.api import MeshInfo
+    p = 6
+    m = mixed_mesh(40, 20, p, every=2)
+    assert np.count_nonzero(general(m)) == m.nelem
+    models = [cf.layered_model(m, seed=s, n_anom=4, amp=0.1) for s in range(8)]
+    mi = MeshInfo(m)
+    om, ky = batch(2)
+
+    def run(model, x, x32):
+        mi.set_model(model)
+        return [product(mi, om, ky, v, k) for v, k in ((x, F64), (x32, F32)) if v is not None]
+
+    def best(x, x32):
+        t = []
+        for model in models:
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            run(model, x, x32)
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    x = vectors(mi, 2)
+    x32 = x.to(torch.complex64)
+    for k in (3, 5, 3):
+        fresh = MeshInfo(m)
+        fresh.set_model(models[k])
+        want = [product(fresh, om, ky, x), product(fresh, om, ky, x32, F32)]
+        assert all(torch.equal(a, b) for a, b in zip(run(models[k], x, x32), want))
+        fresh.close()
+    both, f64, f32 = best(x, x32), best(x, None), best(None, x32)
+    print(f"per model: FP64 {f64 * 1e3:.3f} ms, FP32 {f32 * 1e3:.3f}, both {both * 1e3:.3f}", flush=True)
+    assert both < 0.8 * (f64 + f32)
+    mi.close()

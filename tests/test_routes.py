@@ -234,3 +234,24 @@ def test_blocks_of_both_types_in_one_pass():
     print(f"per model: FP64 {f64 * 1e3:.3f} ms, FP32 {f32 * 1e3:.3f}, both {both * 1e3:.3f}", flush=True)
     assert both < 0.8 * (f64 + f32)
     mi.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["folded", "clockwise", "flat"])
+def test_bad_elements_are_refused_by_every_model(kind):
+    """The Jacobians are checked once a mesh: a mesh that fails is refused by
+    every new model, not only the first (F25_ERR_JACOBIAN)."""
+    from fem25_amd.api import MeshInfo
+    m = cf.structured_mesh(6, 4, 3, width=6e3, depth=4e3)
+    if kind == "folded":
+        m.xlocs[9] += 2.5e3
+    elif kind == "clockwise":
+        m.ieng[5] = m.ieng[5][[0, 3, 2, 1]]
+    else:                                # no height: a parallelogram without area
+        m.zlocs[m.ieng[0, 2:] - 1] = m.zlocs[m.ieng[0, 0] - 1]
+    mi = MeshInfo(m)
+    for seed in (1, 2, 2):
+        with pytest.raises(_lib.Fem25Error) as e:
+            mi.set_model(cf.layered_model(m, seed=seed))
+        assert e.value.code == 2
+    mi.close()

@@ -1181,24 +1181,30 @@ static int affine_colour(f25_mesh *m, const int *order, int n, const int *lm_in,
 // (f25_set_apply_tiles) means the block kernel
 static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt && m->g.ndof < (1 << 27); }
 
+// The kernels of affine.hip load complex128 values into LDS 16 bytes at a
+// time; vectors that start between such pieces (8 bytes off, from a caller's
+// own allocation) go to the kernels that load them into registers.
+static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 // whether a batch of the operator product takes them there (mode F64 or F32)
-static bool affine_batch(const f25_mesh *m, int npair, int mode) {
-    return affine_product(m) && sum_factorised(m->tab.nord, m->nin, m->npar, npair, mode == F25_APPLY_F32);
+static bool affine_batch(const f25_mesh *m, int npair, int mode, const void *x) {
+    const bool fp32 = mode == F25_APPLY_F32;
+    return affine_product(m) && (fp32 || aligned16(x)) && sum_factorised(m->tab.nord, m->nin, m->npar, npair, fp32);
 }
 
 // what the product's launches read: zero rows and sink, and the element
 // blocks of the elements that are not parallelograms
-static int product_ready(f25_mesh *m, int npair, int mode) {
+static int product_ready(f25_mesh *m, int npair, int mode, const void *x) {
     TRY(ensure_vpad(m, npair));
     if (m->disp) return 0;   // every element per omega
     if (mode == F25_APPLY_F32_REFINED) return ensure_blocks(m, true);
-    if (affine_batch(m, npair, mode) && !m->ngen) return 0;
+    if (affine_batch(m, npair, mode, x) && !m->ngen) return 0;
     return mode == F25_APPLY_F32 ? ensure_blocks(m, true) : ensure_vcf(m);
 }
 
 // the records launch_f64 takes for the operator product
-static const double *product_rec(const f25_mesh *m, int npair) {
-    return affine_batch(m, npair, F25_APPLY_F64) ? m->d_rec : nullptr;
+static const double *product_rec(const f25_mesh *m, int npair, const void *x) {
+    return affine_batch(m, npair, F25_APPLY_F64, x) ? m->d_rec : nullptr;
 }
 
 // the launches of the FP64 product (product_ready first), one or two per
@@ -1221,7 +1227,7 @@ static int launch_f64(f25_mesh *m, const double *om, const double *kv, int npair
 // The FP32 products (product_ready first).  The refined product keeps its
 // blocks for every element.
 static int launch_f32(f25_mesh *m, const double *om, const double *kv, int npair, const float2 *x, float2 *y) {
-    const bool aff = affine_batch(m, npair, F25_APPLY_F32);
+    const bool aff = affine_batch(m, npair, F25_APPLY_F32, x);
     for (size_t c = 0; c + 1 < m->cptr.size(); ++c) {
         const std::vector<int> &gp = aff ? m->gcptr : m->cptr;
         if (aff && m->acptr[c + 1] > m->acptr[c])
@@ -1494,8 +1500,8 @@ extern "C" int f25_apply_batch_dev(f25_mesh *m, int npair, const double *omega, 
     if (!m->have_model) FAIL(F25_ERR_STATE, "f25_set_model has not been called");
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
-    TRY(product_ready(m, npair, mode & ~F25_APPLY_GRAPH));
-    return apply_core(m, npair, m->d_omky, m->d_omky + npair, mode, x, y, product_rec(m, npair), m->d_vcf, omega);
+    TRY(product_ready(m, npair, mode & ~F25_APPLY_GRAPH, x));
+    return apply_core(m, npair, m->d_omky, m->d_omky + npair, mode, x, y, product_rec(m, npair, x), m->d_vcf, omega);
 }
 
 extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omega, const double *ky,
@@ -1505,8 +1511,8 @@ extern "C" int f25_residual_batch_dev(f25_mesh *m, int npair, const double *omeg
     if (!m->have_model) FAIL(F25_ERR_STATE, "f25_set_model has not been called");
     HIPCHK(hipSetDevice(m->dev));
     TRY(stage_omky(m, npair, omega, ky));
-    TRY(product_ready(m, npair, F25_APPLY_F64));
-    TRY(apply_core(m, npair, m->d_omky, m->d_omky + npair, F25_APPLY_F64, u, r, product_rec(m, npair), m->d_vcf,
+    TRY(product_ready(m, npair, F25_APPLY_F64, u));
+    TRY(apply_core(m, npair, m->d_omky, m->d_omky + npair, F25_APPLY_F64, u, r, product_rec(m, npair, u), m->d_vcf,
                    omega));
     const int gy = (int)std::min<int64_t>(256, std::max<int64_t>(1, m->g.ndof / 256));
     double *part = nullptr, *sums = nullptr;
@@ -1622,7 +1628,7 @@ static int ring_blocks(f25_mesh *m, int pass, const int *order, int n, const dou
 
 // The ring's elements are too few for a launch of each kind per colour to pay
 // (sum_factorised): on blocks unless all are parallelograms.
-static bool ring_affine(const f25_mesh *m) { return affine_product(m) && m->br.affine; }
+static bool ring_affine(const f25_mesh *m, const void *x) { return affine_product(m) && m->br.affine && aligned16(x); }
 
 static int ring_pass(f25_mesh *m, int pass, const double *om, const double *kv, int npair, const double2 *x,
                      double2 *y) {
@@ -1630,7 +1636,7 @@ static int ring_pass(f25_mesh *m, int pass, const double *om, const double *kv, 
     for (size_t c = 0; c + 1 < B.cptr.size(); ++c) {
         const int n = B.cptr[c + 1] - B.cptr[c], *order = B.d_order + B.cptr[c];
         if (!n) continue;
-        if (ring_affine(m))
+        if (ring_affine(m, x))
             TRY(affine_colour(m, order, n, B.d_lm[2 * pass], B.d_lm[2 * pass + 1], B.d_first0, m->d_rec, om, kv, npair, x,
                               y));
         else
@@ -1640,9 +1646,9 @@ static int ring_pass(f25_mesh *m, int pass, const double *om, const double *kv, 
 }
 
 // what the ring's launches read (bielak_prepare first)
-static int ring_ready(f25_mesh *m, int npair) {
+static int ring_ready(f25_mesh *m, int npair, const void *x) {
     TRY(ensure_vpad(m, npair));
-    return ring_affine(m) ? 0 : ensure_vcf(m);
+    return ring_affine(m, x) ? 0 : ensure_vcf(m);
 }
 
 // the effective force's launches (bielak_prepare and ring_ready first):
@@ -1674,7 +1680,7 @@ extern "C" int f25_peff_batch_dev(f25_mesh *m, int npair, const double *omega, c
     HIPCHK(hipSetDevice(m->dev));
     TRY(bielak_prepare(m));
     TRY(stage_omky(m, npair, omega, ky));
-    TRY(ring_ready(m, npair));
+    TRY(ring_ready(m, npair, ue_dev));
     const double *om = m->d_omky, *kv = m->d_omky + npair;
     HIPCHK(hipEventRecord(m->ev0, m->st));
     TRY(peff_launches(m, npair, om, kv, (const double2 *)ue_dev, (double2 *)peff_dev));
@@ -1794,7 +1800,7 @@ extern "C" int f25_bielak_rhs_dev(f25_mesh *m, int npair, const double *omega, c
         B.exec = nullptr;
     }
     TRY(stage_omky(m, npair, omega, ky));
-    TRY(ring_ready(m, npair));
+    TRY(ring_ready(m, npair, ue_dev));
     TRY(uwave_params(m, npair, kappax, kappaz, baz, aoi));
     const double *om = m->d_omky, *kv = m->d_omky + npair;
     // staging buffers may have moved since the capture
@@ -1940,7 +1946,7 @@ static int grad_launch(f25_mesh *m, int ntrip, const double *d_om, const double 
                        bool fp32) {
     HIPCHK(hipEventRecord(m->ev0, m->st));
     if (fp32) return grad_general<float>(m, nullptr, m->d.nelem, ntrip, d_om, d_ky, u, l);
-    if (!grad_sum_factorised(m->nin, m->npar, ntrip))
+    if (!grad_sum_factorised(m->nin, m->npar, ntrip) || !aligned16(u) || !aligned16(l))
         return grad_general<double>(m, nullptr, m->d.nelem, ntrip, d_om, d_ky, u, l);
     const double2 *ud = (const double2 *)u, *ld = (const double2 *)l;
     if (m->naff) switch (m->tab.nl) {
@@ -3347,7 +3353,7 @@ extern "C" int f25_gn_fv(f25_mesh *m, int ntrip, const double *omega, const doub
     TRY(upload(&d_l, dl.data(), n, m->st));
     TRY(upload(&d_m, dm.data(), n, m->st));
     // the perturbation's records, and its blocks for elements of general shape
-    const bool aff = affine_product(m) && (!m->ngen || affine_batch(m, ntrip, F25_APPLY_F64));
+    const bool aff = affine_product(m) && (!m->ngen || affine_batch(m, ntrip, F25_APPLY_F64, nullptr));
     const bool blocks = !aff || m->ngen;
     int r = 0;
     if (aff) {

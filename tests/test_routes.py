@@ -255,3 +255,57 @@ def test_bad_elements_are_refused_by_every_model(kind):
             mi.set_model(cf.layered_model(m, seed=seed))
         assert e.value.code == 2
     mi.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("npml", [0, 2])
+def test_vectors_eight_bytes_off(npml):
+    """complex128 vectors that start 8 bytes past a multiple of 16 (a caller's
+    own allocation, through the C entry points): the product and the effective
+    force on blocks, bit for bit, the gradient on the general points."""
+    import ctypes as C
+
+    import torch
+    from fem25_amd.api import MeshInfo
+    p, n = 4, 7
+    m = cf.structured_mesh(10, 6, p, width=20e3, depth=12e3, npml=npml, nbielak=1 if npml else 0)
+    mi = MeshInfo(m, cf.PML(rcoeff=1e-3, kappa=1.0, fcent=0.05) if npml else cf.PML())
+    mi.set_model(cf.layered_model(m, seed=3, n_anom=3))
+    om, ky = batch(n)
+    dev = lambda t: C.c_void_p(t.data_ptr())
+
+    def off(t):
+        v = torch.empty(2 * t.numel() + 1, dtype=torch.float64, device="cuda")[1:]
+        v.copy_(torch.view_as_real(t).reshape(-1))
+        assert v.data_ptr() % 16 == 8
+        return v
+
+    def call(name, *a):
+        _lib.check(getattr(_lib.load(), name)(mi.h, n, om.ctypes.data_as(_lib.dp), ky.ctypes.data_as(_lib.dp), *a), name)
+
+    x = vectors(mi, n)
+    xo, yo = off(x), off(x)
+    torch.cuda.synchronize()
+    names = ("f25_apply_batch_dev",) + (("f25_peff_batch_dev",) if npml else ())
+    for name in names:
+        mode = (F64,) if "apply" in name else ()
+        a = (dev(xo), dev(yo))
+        call(name, *mode, *a)
+        got = yo.clone()
+        y = torch.empty_like(x)
+        for tiles in (0, row_tiles(p)):
+            mi.set_apply_tiles(tiles)
+            call(name, *mode, dev(x), dev(y))
+            want = torch.view_as_real(y).reshape(-1)
+            e = float(torch.linalg.norm(got - want) / torch.linalg.norm(want))
+            assert e < 1e-13 and (tiles == 0 or e == 0.0), (name, tiles, e)
+        mi.set_apply_tiles(0)
+    u, lam = x.T.contiguous(), vectors(mi, n, seed=9).T.contiguous()
+    g = [torch.zeros(m.nnpg, 3, dtype=torch.float64, device="cuda") for _ in range(3)]
+    uo, lo = off(u), off(lam)
+    torch.cuda.synchronize()
+    for k, (a, b) in enumerate(((u, lam), (uo, lam), (u, lo))):
+        call("f25_gradient_dev", dev(a), dev(b), dev(g[k]))
+    assert torch.equal(g[1], g[2])
+    assert float(torch.linalg.norm(g[1] - g[0]) / torch.linalg.norm(g[0])) < 1e-12
+    mi.close()

@@ -244,30 +244,6 @@ static int check_err(f25_mesh *m) {
     return 0;
 }
 
-// Elements the kernels of affine.hip take: those whose bilinear map is affine
-// in FP64 (x1 - x2 + x3 - x4 zero to the rounding of the differences, as on
-// any structured rectangular or sheared mesh: the twist then changes the
-// Jacobian by less than its own rounding) with det J > 0 as geo_at requires;
-// and the PML elements, which those kernels skip as the others do.  Anything
-// else keeps the reference's quadrature.
-static bool is_affine(const f25_mesh *m, int e) {
-    double x[4], z[4];
-    for (int k = 0; k < 4; ++k) {
-        x[k] = m->xl[m->ieng[4 * e + k] - 1];
-        z[k] = m->zl[m->ieng[4 * e + k] - 1];
-    }
-    double h = 0.0;
-    for (int k = 0; k < 4; ++k) {
-        const int n = (k + 1) % 4;
-        h = std::max(h, std::max(std::fabs(x[n] - x[k]), std::fabs(z[n] - z[k])));
-    }
-    const double bx = (x[0] - x[1]) + (x[2] - x[3]), bz = (z[0] - z[1]) + (z[2] - z[3]);
-    const double tol = 4e-16 * h;
-    const double det = 0.0625 * (((x[1] - x[0]) + (x[2] - x[3])) * ((z[3] - z[0]) + (z[2] - z[1])) -
-                                 ((x[3] - x[0]) + (x[2] - x[1])) * ((z[1] - z[0]) + (z[2] - z[3])));
-    return std::fabs(bx) <= tol && std::fabs(bz) <= tol && det > 2.22e-16;
-}
-
 // a colour order's elements by kind (m->affine), each in colour order
 static void split_order(const f25_mesh *m, const std::vector<int> &order, const std::vector<int> &cptr,
                         std::vector<int> &ao, std::vector<int> &ap, std::vector<int> &go, std::vector<int> &gp) {
@@ -350,7 +326,12 @@ static int upload_mesh(f25_mesh *m) {
     m->affine.assign(d.nelem, 0);
     std::vector<int> ael, gel;
     for (int e = 0; e < d.nelem; ++e) {
-        m->affine[e] = m->cdom[e] == 'A' || is_affine(m, e);
+        double x[4], z[4];
+        for (int k = 0; k < 4; ++k) {
+            x[k] = m->xl[m->ieng[4 * e + k] - 1];
+            z[k] = m->zl[m->ieng[4 * e + k] - 1];
+        }
+        m->affine[e] = m->cdom[e] == 'A' || parallelogram(x, z);   // the kernels of affine.hip skip 'A' as the others do
         (m->affine[e] ? ael : gel).push_back(e);
         if (!m->affine[e] || m->cdom[e] == 'A') continue;
         const int *a = &m->ieng[4 * e];
@@ -3495,6 +3476,10 @@ extern "C" int f25_gn_diag(f25_mesh *m, int ntrip, const double *omega, const do
     }
     dfree(du); dfree(dcols); dfree(dd);
     return r;
+}
+
+extern "C" int f25_selftest_parallelogram(const double *x, const double *z) {
+    return x && z ? (parallelogram(x, z) ? 1 : 0) : -1;
 }
 
 extern "C" int f25_selftest_route(int nord, int64_t nin, int64_t npar, int64_t npair, int mode) {

@@ -29,6 +29,8 @@ void gll_nodes(int n, double *x, double *w);
 // (2 nl <= 14 values), at 14 and 15 w h0 and w h1; after the rows h0, h1 and
 // w at the points (h0 = (1 - s)/2, h1 = (1 + s)/2)
 std::vector<double> af_table(const Tables &t);
+// whether the element of corners x, z (counter-clockwise) runs as a parallelogram
+bool parallelogram(const double *x, const double *z);
 // whether a batched product of npair pairs takes its parallelograms by sum
 // factorisation: nin elements outside the PML, npar of them parallelograms
 bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npair, bool fp32);

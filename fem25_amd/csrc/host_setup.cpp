@@ -222,6 +222,25 @@ std::vector<double> af_table(const Tables &t) {
     return o;
 }
 
+// The bilinear map of the corners is x(xi, eta) = x_c + J (xi, eta) + b xi eta,
+// b a quarter of x1 - x2 + x3 - x4.  An element runs at the (p + 1)-point rule
+// if J^-1 b, the twist in its own coordinates, is within the rounding of one:
+// no Jacobian at a quadrature point then differs from J by more than its own
+// rounding, whatever the element's shape (a tolerance in metres would let a
+// flat element's short side be off by its aspect ratio); and det J > 0 as
+// geo_at requires.  That holds for every element of a mesh whose lines run along
+// x and z, or whose coordinates are exact in FP64.  Coordinates rounded at
+// their own magnitude (a sheared or rotated mesh far from the origin) leave
+// twists of 1e-14 of the element, which the reference's quadrature resolves:
+// such elements keep it (97x61 elements over 80 km, x + z/4: 18% of them).
+bool parallelogram(const double *x, const double *z) {
+    const double xx = 0.25 * ((x[1] - x[0]) + (x[2] - x[3])), xe = 0.25 * ((x[3] - x[0]) + (x[2] - x[1]));
+    const double zx = 0.25 * ((z[1] - z[0]) + (z[2] - z[3])), ze = 0.25 * ((z[3] - z[0]) + (z[2] - z[1]));
+    const double bx = 0.25 * ((x[0] - x[1]) + (x[2] - x[3])), bz = 0.25 * ((z[0] - z[1]) + (z[2] - z[3]));
+    const double det = xx * ze - xe * zx, tol = 2.2204e-16 * det;
+    return det > 2.22e-16 && std::fabs(ze * bx - xe * bz) <= tol && std::fabs(xx * bz - zx * bx) <= tol;
+}
+
 // Where parallelograms run by sum factorisation.  FP64 arithmetic runs at the
 // rate of FP32 arithmetic without packed instructions, so it beats the blocks
 // in both types (FP32: their matrix units) where the blocks are large (FP32,

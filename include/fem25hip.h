@@ -447,6 +447,9 @@ const char *f25_last_error(void);
  * the operand/result lane layout the batched product relies on; *maxerr is
  * the largest deviation (0 when the layout holds). */
 int f25_selftest_mfma(double *maxerr);
+/* 1 if the element of corners x[4], z[4] (counter-clockwise) counts as a
+ * parallelogram: its twist is within the rounding of its sides, det J > 0. */
+int f25_selftest_parallelogram(const double *x, const double *z);
 /* Which way a batched product takes its parallelogram elements: 1 by sum
  * factorisation, 0 on element blocks as the others, -1 for arguments out of
  * range.  nin elements outside the PML, npar of them parallelograms, mode

@@ -4,6 +4,7 @@ meshes that hold both kinds on the two routes."""
 from __future__ import annotations
 
 import functools
+from fractions import Fraction
 
 import numpy as np
 import pytest
@@ -75,6 +76,58 @@ def err(a, b):
     """The largest normwise error of a column."""
     import torch
     return float((torch.linalg.norm(a - b, dim=0) / torch.linalg.norm(b, dim=0)).max())
+
+
+def parallelogram(x, z) -> bool:
+    x, z = np.ascontiguousarray(x, np.float64), np.ascontiguousarray(z, np.float64)
+    return _lib.load().f25_selftest_parallelogram(x.ctypes.data_as(_lib.dp), z.ctypes.data_as(_lib.dp)) == 1
+
+
+def share(m) -> float:
+    return float(np.mean([parallelogram(m.xlocs[a - 1], m.zlocs[a - 1]) for a in m.ieng]))
+
+
+def twist(x, z) -> float:
+    """max |J^-1 b| of the bilinear map, in rational arithmetic."""
+    x, z = [Fraction(float(v)) for v in x], [Fraction(float(v)) for v in z]
+    xx, xe, b1 = x[1] - x[0] + x[2] - x[3], x[3] - x[0] + x[2] - x[1], x[0] - x[1] + x[2] - x[3]
+    zx, ze, b2 = z[1] - z[0] + z[2] - z[3], z[3] - z[0] + z[2] - z[1], z[0] - z[1] + z[2] - z[3]
+    det = xx * ze - xe * zx
+    return float(max(abs((ze * b1 - xe * b2) / det), abs((xx * b2 - zx * b1) / det)))
+
+
+def test_parallelograms_of_meshes():
+    """Structured meshes are all parallelograms, exact shears too; rounded
+    shears in part, and what is accepted there has no twist to speak of."""
+    for nx, nz in ((200, 100), (97, 61)):
+        m = cf.structured_mesh(nx, nz, 2)
+        assert share(m) == 1.0
+        m.xlocs += 0.25 * m.zlocs
+        assert 0.5 < share(m) <= 1.0
+        for a in m.ieng[:: 7]:
+            if parallelogram(m.xlocs[a - 1], m.zlocs[a - 1]):
+                assert twist(m.xlocs[a - 1], m.zlocs[a - 1]) < 1e-15
+    m = mixed_mesh(20, 14, 2)
+    assert share(m) == 1.0 - np.mean(general(m))
+
+
+@pytest.mark.parametrize("lx,lz", [(1e4, 10.0), (10.0, 1e4), (400.0, 400.0), (1e5, 1.0)])
+def test_twist_is_measured_in_the_elements_own_shape(lx, lz):
+    """A twist of the short side, far below the rounding of the long one, is
+    refused at any aspect ratio; one within the rounding of the side it moves
+    is accepted."""
+    x, z = np.array([0.0, lx, lx, 0.0]), np.array([0.0, 0.0, lz, lz])
+    assert parallelogram(x, z)
+    for v, h in ((x, lx), (z, lz)):
+        w = v.copy()
+        w[2] += 1e-14 * h
+        e = (w, z) if v is x else (x, w)
+        assert twist(*e) > 1e-15 and not parallelogram(*e)
+    w = z.copy()
+    w[2] = np.nextafter(lz, 2 * lz)
+    assert parallelogram(x, w) and twist(x, w) < 2.3e-16
+    assert not parallelogram(x[[0, 3, 2, 1]], z[[0, 3, 2, 1]])      # clockwise
+    assert not parallelogram(x, 0 * z)                              # no area
 
 
 # (order, elements, pairs, mode, sum factorisation faster) as timed, a tenth to half of the elements general

@@ -158,7 +158,8 @@ struct f25_mesh_s {
         int grp_cap = 0, gpair_cap = 0, ngrp = 0;
     } pa;
     // CSR positions of the values of the elements integrated per call
-    // (k_pml_pos): the PML elements', and every element's (dispersive medium)
+    // (k_pml_pos): the PML elements', and every element's while the medium is
+    // dispersive; 4 (3 NEN)^2 bytes an element (22.5 KB at p4, 86 KB at p6)
     int *d_pos[2] = {};
     int apply_nrt = 0;          // row tiles of k_apply_v (0: the order's default)
     double *d_vpad = nullptr;   // k_apply_v: vpad_cap zero double2, then vpad_cap double2 of store sink
@@ -716,6 +717,7 @@ extern "C" int f25_set_attenuation(f25_mesh *m, const double *qp, const double *
     if (!qp || !qs) {
         if (m->disp) m->pa.valid = false;
         m->disp = false;
+        dfree(m->d_pos[1]);   // read by a dispersive medium's assembly only
         return 0;
     }
     const int n = m->d.nnpg;
@@ -819,7 +821,7 @@ static int ensure_basis(f25_mesh *m) {
 }
 
 // CSR positions for the elements integrated per call, built once per mesh
-// (and again for every element when a medium first is dispersive)
+// (and for every element when the medium becomes dispersive)
 static int ensure_pml_pos(f25_mesh *m) {
     const int k = m->disp ? 1 : 0;
     const size_t n = m->disp ? m->order.size() : m->pml_order.size(), nee = 3 * m->tab.nen;

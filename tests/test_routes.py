@@ -362,3 +362,27 @@ def test_vectors_eight_bytes_off(npml):
     assert torch.equal(g[1], g[2])
     assert float(torch.linalg.norm(g[1] - g[0]) / torch.linalg.norm(g[0])) < 1e-12
     mi.close()
+
+
+@pytest.mark.gpu
+def test_dispersive_table_is_given_back():
+    """Elastic, dispersive and elastic again: the assembled values of either
+    medium repeat bit for bit, and the table of every element's positions (4 (3
+    NEN)^2 bytes each, 47.5 MB here) is released with the attenuation."""
+    import torch
+    from fem25_amd.api import MeshInfo
+    m = cf.structured_mesh(64, 33, 4, npml=2, nbielak=1)
+    mi = MeshInfo(m, cf.PML(rcoeff=1e-3, kappa=1.0, fcent=0.05))
+    elastic = cf.layered_model(m, seed=2)
+    media = [elastic, cf.with_attenuation(elastic, 300.0, 150.0, 1.0)]
+    out = [None, None]
+    for k in (0, 1, 0, 1, 0):
+        before = torch.cuda.mem_get_info()[0]
+        mi.set_model(media[k])
+        if k == 0 and out[1] is not None:
+            assert torch.cuda.mem_get_info()[0] - before > 40e6
+        v = torch.empty(mi.nz, dtype=torch.complex128, device="cuda")
+        mi.asmble_dev(b"B", 0.05, 5e-5, v)
+        assert out[k] is None or torch.equal(v, out[k])
+        out[k] = v
+    mi.close()

@@ -1160,9 +1160,10 @@ static int affine_colour(f25_mesh *m, const int *order, int n, const int *lm_in,
 }
 
 // whether k_apply_af can take the product's parallelograms: it packs a DOF
-// and a pair into one register, and a row-tile count asked for
+// and a pair into one register.  FP64: a row-tile count asked for
 // (f25_set_apply_tiles) means the block kernel
-static bool affine_product(const f25_mesh *m) { return m->naff && !m->apply_nrt && m->g.ndof < (1 << 27); }
+static bool affine_fits(const f25_mesh *m) { return m->naff && m->g.ndof < (1 << 27); }
+static bool affine_product(const f25_mesh *m) { return affine_fits(m) && !m->apply_nrt; }
 
 // The kernels of affine.hip load complex128 values into LDS 16 bytes at a
 // time; vectors that start between such pieces (8 bytes off, from a caller's
@@ -1172,7 +1173,8 @@ static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 // whether a batch of the operator product takes them there (mode F64 or F32)
 static bool affine_batch(const f25_mesh *m, int npair, int mode, const void *x) {
     const bool fp32 = mode == F25_APPLY_F32;
-    return affine_product(m) && (fp32 || aligned16(x)) && sum_factorised(m->tab.nord, m->nin, m->npar, npair, fp32);
+    return (fp32 ? affine_fits(m) : affine_product(m) && aligned16(x)) &&
+           sum_factorised(m->tab.nord, m->nin, m->npar, npair, fp32);
 }
 
 // what the product's launches read: zero rows and sink, and the element

@@ -191,8 +191,10 @@ int f25_apply_batch(f25_mesh *m, int npair, const double *omega, const double *k
  * has no batched product): number of row tiles per output component of the
  * product on element blocks, 0 = the order's default (and parallelograms by
  * sum factorisation).  Compiled candidates: p2, p3: 1, 2; p4: 1..3; p5, p6:
- * 2..4.  Any other value than 0 sends every element through its blocks; their
- * coefficient layout is written by the next product.
+ * 2..4.  Any other value than 0 sends every element of the FP64 products (the
+ * batch, the residual, the effective force, f25_gn_fv) through its blocks;
+ * their coefficient layout is written by the next product.  The FP32 modes are
+ * not affected.
  * fem25_amd/tune_apply.py times the candidates. */
 int f25_set_apply_tiles(f25_mesh *m, int nrt);
 

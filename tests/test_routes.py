@@ -386,3 +386,16 @@ def test_dispersive_table_is_given_back():
         assert out[k] is None or torch.equal(v, out[k])
         out[k] = v
     mi.close()
+
+
+@pytest.mark.gpu
+def test_row_tiles_leave_the_fp32_product_alone():
+    """Row tiles are the FP64 block product's: the FP32 product of
+    parallelograms keeps its route, bit for bit, whatever they are."""
+    import torch
+    mi = handle(40, 20, 4, 0)
+    om, ky = batch(9)
+    x = vectors(mi, 9).to(torch.complex64)
+    want = product(mi, om, ky, x, F32)
+    for tiles in (1, 2, 3):
+        assert torch.equal(product(mi, om, ky, x, F32, tiles), want), tiles

@@ -5,12 +5,15 @@ on the GPU and reports the fastest.
                                    [--nfreq 6] [--nky 32] [--reps 5]
 
 Every candidate runs on the same mesh, model and vectors; the time is the
-library's HIP-event figure for the product's launches (one per element
-colour).  The results of the candidates are compared with each other (they
-differ only in the order of floating-point sums), and all run the product on
-element blocks (row tiles asked for switch sum factorisation off).  The per-order defaults
-compiled into the library (apply_nrt_default in csrc/capi.hip) come from
-this script; f25_set_apply_tiles selects another candidate at run time.
+library's HIP-event figure for the product's launches.  Counts other than 0
+run every element on its blocks (one launch per element colour); 0 is the
+library's own choice (parallelograms by sum factorisation where that is
+faster), so what is best here is never slower than leaving the hook alone.
+The results of the candidates are compared with each other (they differ by
+the order of floating-point sums, and for 0 the quadrature rule).  The
+per-order defaults compiled into the library (apply_nrt_default in
+csrc/capi.hip) come from this script; f25_set_apply_tiles selects another
+candidate at run time.
 One JSON line per (order, candidate), then one per order with the fastest.
 """
 from __future__ import annotations
@@ -20,8 +23,8 @@ import json
 import math
 import sys
 
-# row-tile counts compiled into the library, by element order p
-CANDIDATES = {2: (1, 2), 3: (1, 2), 4: (1, 2, 3), 5: (2, 3, 4), 6: (2, 3, 4)}
+# 0, the library's own choice, and the row-tile counts compiled into it, by element order p
+CANDIDATES = {2: (0, 1, 2), 3: (0, 1, 2), 4: (0, 1, 2, 3), 5: (0, 2, 3, 4), 6: (0, 2, 3, 4)}
 
 
 def main(argv=None) -> int:
@@ -73,11 +76,11 @@ def main(argv=None) -> int:
             else:
                 diff = float(torch.linalg.norm(y - yref) / torch.linalg.norm(yref))
             t = float(np.median(ms))
-            rec = {"order": nord, "row_tiles": nrt, "rows_per_tile": -(-(nord + 1) ** 2 // nrt),
+            rec = {"order": nord, "row_tiles": nrt, "rows_per_tile": -(-(nord + 1) ** 2 // nrt) if nrt else None,
                    "kernel_ms_per_step": round(t, 4),
                    "gdof_per_s": round(mi.ndof * npair / (t * 1e-3) / 1e9, 3), "rel_diff_vs_first": diff}
             print(json.dumps(rec), flush=True)
-            if best is None or t < best[1]:
+            if best is None or t < best[1]:   # 0 first: only a faster count replaces it
                 best = (nrt, t)
         print(json.dumps({"order": nord, "best_row_tiles": best[0], "kernel_ms_per_step": round(best[1], 4),
                           "mesh": f"{args.nx}x{args.nz}", "npair": npair}), flush=True)

@@ -399,3 +399,21 @@ def test_row_tiles_leave_the_fp32_product_alone():
     want = product(mi, om, ky, x, F32)
     for tiles in (1, 2, 3):
         assert torch.equal(product(mi, om, ky, x, F32, tiles), want), tiles
+
+
+@pytest.mark.gpu
+def test_tuner_times_the_librarys_own_choice(capsys):
+    """The tuner's candidates hold 0 (no row tiles asked for), so what it calls
+    best is no slower than leaving the hook alone."""
+    import json
+
+    from fem25_amd import tune_apply
+    assert tune_apply.main(["--orders", "4", "6", "--nx", "40", "--nz", "20", "--nfreq", "1", "--nky", "4",
+                            "--reps", "5"]) == 0
+    lines = [json.loads(ln) for ln in capsys.readouterr().out.splitlines() if ln.startswith("{")]
+    for order in (4, 6):
+        ms = {d["row_tiles"]: d["kernel_ms_per_step"] for d in lines if d["order"] == order and "row_tiles" in d}
+        best = [d for d in lines if d["order"] == order and "best_row_tiles" in d]
+        assert 0 in ms and len(best) == 1
+        assert best[0]["kernel_ms_per_step"] == min(ms.values()) == ms[best[0]["best_row_tiles"]]
+        assert all(d["rel_diff_vs_first"] < 1e-13 for d in lines if "rel_diff_vs_first" in d)

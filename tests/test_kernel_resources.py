@@ -4,14 +4,20 @@ only).  A register array indexed by a run-time value, or a change that
 pushes a kernel over its register budget, shows up as scratch memory
 (spills) or as a lower occupancy long before it shows up as a slower run;
 this test keeps those budgets fixed:
-  * the batched product (k_apply_v), the pseudo-Hessian element columns
-    (k_fcols_sf) and the element derivative products (k_dab_sf) use no
-    scratch at any order or tiling;
+  * the batched product on element blocks (k_apply_v), the pseudo-Hessian
+    element columns (k_fcols_sf) and the element derivative products (k_dab_sf)
+    use no scratch at any order or tiling;
+  * the product and the gradient of parallelograms (k_apply_af, the
+    benchmark's kernel, and k_grad_af) use none up to p5 and keep two waves per
+    SIMD at every order (three at p2); at p6, where 256 registers are all there
+    are, they spill 36 and 16 bytes per lane;
+  * the matrices of elements integrated per omega (k_pml_sf) use none, their
+    product (k_apply_pml) at most 12 bytes at four waves per SIMD;
   * the FP64 gradient (k_grad_sf) spills at most a few registers (the
     addresses of the prefetch and the point's inverse Jacobian, which it
     keeps in registers to save LDS), at most 64 bytes per lane, and the FP32
     gradient none;
-  * the product for p4 with one row tile (the benchmark's kernel) keeps
+  * the block product for p4 with one row tile keeps
     three waves per SIMD and at most 168 registers, and the gradient and
     pseudo-Hessian kernels for p2..p5 keep four.
 """
@@ -95,6 +101,20 @@ def test_occupancy_budgets(usage):
         for name, v in kernels(usage, base).items():
             if nl_of(name) <= 5:
                 assert v["occupancy"] >= 4, (name, v)
+
+
+def test_sum_factorised_kernels(usage):
+    for base, spill in (("k_apply_af", 36), ("k_grad_af", 16)):
+        for name, v in kernels(usage, base).items():
+            assert v["scratch"] <= (spill if nl_of(name) == 7 else 0), (name, v)
+            assert v["occupancy"] >= (3 if nl_of(name) == 3 else 2), (name, v)
+
+
+def test_kernels_of_elements_per_omega(usage):
+    for name, v in kernels(usage, "k_pml_sf").items():
+        assert v["scratch"] == 0 and v["occupancy"] >= 3, (name, v)
+    for name, v in kernels(usage, "k_apply_pml").items():
+        assert v["scratch"] <= 12 and v["occupancy"] >= 4, (name, v)
 
 
 def test_parser_reads_remarks():

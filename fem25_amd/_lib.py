@@ -108,7 +108,7 @@ EXPORTS = {
     "f25_last_kernel_ms": (C.c_double, [C.c_char_p]),
     "f25_selftest_mfma": (C.c_int, [dp]),
     "f25_selftest_parallelogram": (C.c_int, [dp, dp]),
-    "f25_selftest_route": (C.c_int, [C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int]),
+    "f25_selftest_route": (C.c_int, [C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int]),
     "f25_selftest_residency": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]),
 }
 

@@ -1174,7 +1174,7 @@ static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 static bool affine_batch(const f25_mesh *m, int npair, int mode, const void *x) {
     const bool fp32 = mode == F25_APPLY_F32;
     return (fp32 ? affine_fits(m) : affine_product(m) && aligned16(x)) &&
-           sum_factorised(m->tab.nord, m->nin, m->npar, npair, fp32);
+           sum_factorised(m->tab.nord, m->nin, m->npar, (int64_t)m->pml_order.size(), npair, fp32);
 }
 
 // what the product's launches read: zero rows and sink, and the element
@@ -3486,12 +3486,12 @@ extern "C" int f25_selftest_parallelogram(const double *x, const double *z) {
     return x && z ? (parallelogram(x, z) ? 1 : 0) : -1;
 }
 
-extern "C" int f25_selftest_route(int nord, int64_t nin, int64_t npar, int64_t npair, int mode) {
-    if (nord < 2 || nord > 6 || npar < 0 || npar > nin || npair <= 0 ||
+extern "C" int f25_selftest_route(int nord, int64_t nin, int64_t npar, int64_t npml, int64_t npair, int mode) {
+    if (nord < 2 || nord > 6 || npar < 0 || npar > nin || npml < 0 || npair <= 0 ||
         (mode != F25_APPLY_F64 && mode != F25_APPLY_F32 && mode != F25_ROUTE_GRADIENT))
         return -1;
     if (mode == F25_ROUTE_GRADIENT) return grad_sum_factorised(nin, npar, npair) ? 1 : 0;
-    return sum_factorised(nord, nin, npar, npair, mode == F25_APPLY_F32) ? 1 : 0;
+    return sum_factorised(nord, nin, npar, npml, npair, mode == F25_APPLY_F32) ? 1 : 0;
 }
 
 // Workgroup residency: the most workgroups of nt threads, holding vgprs

@@ -32,8 +32,9 @@ std::vector<double> af_table(const Tables &t);
 // whether the element of corners x, z (counter-clockwise) runs as a parallelogram
 bool parallelogram(const double *x, const double *z);
 // whether a batched product of npair pairs takes its parallelograms by sum
-// factorisation: nin elements outside the PML, npar of them parallelograms
-bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npair, bool fp32);
+// factorisation: nin elements outside the PML, npar of them parallelograms,
+// npml PML elements
+bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npml, int64_t npair, bool fp32);
 // the same for the FP64 gradient of ntrip triples
 bool grad_sum_factorised(int64_t nin, int64_t npar, int64_t ntrip);
 

@@ -260,22 +260,24 @@ bool parallelogram(const double *x, const double *z) {
 //            224, 48 321 / 457; 64x32: 48 86 / 83, 64 87 / 93; 40x20: 320 197 / 144
 //
 // On a mesh that holds other elements too, both kinds are launched for every
-// colour, one after the other: worth it where the mesh is large enough that
-// the blocks of a colour are more than one launch's latency, and the
-// parallelograms are at least half of the elements.  Measured on MI355X, all
-// on blocks / both kinds, a tenth of the elements general, 8 pairs: FP64
-// 64x32 p5 221 / 176 us, 97x61 p3 160 / 126, p4 310 / 204, p6 985 / 332, but
-// 40x20 p4 122 / 158, 97x61 p2 84 / 98; FP32 97x61 p5 391 / 254, 200x100 p4
-// 422 / 284, but 97x61 p3 68 / 103, p4 153 / 174.  Larger batches of low order
-// gain nothing: 97x61, 45 pairs, FP64 p3 214 / 240, p4 380 / 402.
-bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npair, bool fp32) {
+// colour, one after the other: worth it where the parallelograms are so many
+// that their blocks take longer than another launch does.  Measured on
+// MI355X, all on blocks / both kinds, 8 pairs, us: FP64, a tenth of the elements
+// general: 200x100 p2 200 / 131, 97x61 p2 84 / 98, p3 160 / 126, p4 310 / 204, 40x20
+// p4 122 / 158, 64x32 p5 221 / 176, 40x20 p5 162 / 165, p6 255 / 238; half of them:
+// 97x61 p3 158 / 152, p4 310 / 264, 64x32 p5 221 / 220; FP32, a tenth: 200x100
+// p4 422 / 284, 97x61 p4 153 / 174, p5 391 / 254, 64x32 p5 169 / 203, p6 341 / 246.
+// Larger batches of low order run at the rate of the vectors' traffic: 97x61, 45
+// pairs, FP64 p3 214 / 240, p4 380 / 402.  In FP64 p5 and p6 a launch that only
+// stores the zeros of PML elements costs less than their blocks (40x20 p6, two
+// rings, the rest general, one pair 380 / 307).
+bool sum_factorised(int nord, int64_t nin, int64_t npar, int64_t npml, int64_t npair, bool fp32) {
     if (npar != nin) {
-        struct Least { int64_t nelem, most; };   // elements, pairs
-        constexpr int64_t never = INT64_MAX, any = INT64_MAX;
-        constexpr Least f64[5] = {{16384, 16}, {4096, 16}, {4096, 24}, {4096, any}, {2048, any}};
-        constexpr Least f32[5] = {{never, 0}, {never, 0}, {16384, any}, {4096, any}, {4096, any}};
-        const Least l = (fp32 ? f32 : f64)[nord - 2];
-        return 2 * npar >= nin && nin >= l.nelem && npair <= l.most;
+        constexpr int64_t never = INT64_MAX;
+        // parallelograms from which on: up to 24 pairs, more pairs
+        constexpr int64_t f64[5][2] = {{8000, never}, {3000, never}, {2500, 8000}, {1400, 1400}, {400, 400}};
+        constexpr int64_t f32[5][2] = {{never, never}, {never, never}, {8000, 8000}, {2500, 2500}, {1000, 2500}};
+        return npar >= (fp32 ? f32 : f64)[nord - 2][npair <= 24 ? 0 : 1] || (!fp32 && nord >= 5 && npml >= 128);
     }
     if (nord >= (fp32 ? 4 : 3)) return true;
     if (fp32 && nin <= (nord == 2 ? 2048 : 1024)) return true;

@@ -457,11 +457,11 @@ int f25_selftest_mfma(double *maxerr);
 int f25_selftest_parallelogram(const double *x, const double *z);
 /* Which way a batched product takes its parallelogram elements: 1 by sum
  * factorisation, 0 on element blocks as the others, -1 for arguments out of
- * range.  nin elements outside the PML, npar of them parallelograms, mode
+ * range.  nin elements outside the PML, npar of them parallelograms, npml PML elements, mode
  * F25_APPLY_F64, F25_APPLY_F32, or F25_ROUTE_GRADIENT for the FP64 gradient of
  * npair triples (0: at the general quadrature points as the others). */
 enum { F25_ROUTE_GRADIENT = 64 };
-int f25_selftest_route(int nord, int64_t nin, int64_t npar, int64_t npair, int mode);
+int f25_selftest_route(int nord, int64_t nin, int64_t npar, int64_t npml, int64_t npair, int mode);
 /* Workgroup residency on the current device: *groups_per_cu = the most
  * workgroups of nt threads (192, 256, 320, 384 or 512) holding vgprs
  * registers per lane (128 or 168) and lds bytes of LDS that are resident

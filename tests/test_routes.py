@@ -130,19 +130,22 @@ def test_twist_is_measured_in_the_elements_own_shape(lx, lz):
     assert not parallelogram(x, 0 * z)                              # no area
 
 
-# (order, elements, pairs, mode, sum factorisation faster) as timed, a tenth to half of the elements general
-@pytest.mark.parametrize("p,nin,n,mode,sf", [
-    (2, 800, 8, F64, False), (2, 5917, 8, F64, False), (2, 20000, 8, F64, True), (2, 20000, 40, F64, False),
-    (3, 2048, 8, F64, False), (3, 5917, 8, F64, True), (3, 5917, 45, F64, False),
-    (4, 800, 1, F64, False), (4, 5917, 24, F64, True), (4, 5917, 45, F64, False), (5, 5917, 128, F64, True),
-    (6, 800, 75, F64, False), (6, 2048, 75, F64, True),
-    (2, 20000, 1, F32, False), (3, 20000, 40, F32, False), (4, 5917, 8, F32, False), (4, 20000, 40, F32, True),
-    (5, 2048, 24, F32, False), (5, 5917, 45, F32, True), (6, 800, 8, F32, False), (6, 5917, 1, F32, True)])
-def test_rule_of_mixed_meshes(p, nin, n, mode, sf):
-    route = _lib.load().f25_selftest_route
-    assert route(p, nin, nin * 3 // 4, n, mode) == sf
-    assert route(p, nin, nin // 10, n, mode) == 0       # few parallelograms: one launch a colour
-    assert route(p, nin, 0, n, mode) == 0               # none but the PML elements
+# (order, elements, parallelograms, PML elements, pairs, mode, sum factorisation faster) as timed
+@pytest.mark.parametrize("p,nin,npar,npml,n,mode,sf", [
+    (2, 800, 700, 0, 8, F64, False), (2, 5917, 5680, 0, 8, F64, False), (2, 20000, 10600, 0, 8, F64, True),
+    (2, 20000, 19000, 0, 40, F64, False), (3, 2048, 1960, 0, 8, F64, False), (3, 5917, 3136, 0, 8, F64, True),
+    (3, 5917, 5200, 0, 45, F64, False), (4, 800, 770, 0, 1, F64, False), (4, 5917, 3136, 0, 24, F64, True),
+    (4, 5917, 5200, 0, 45, F64, False), (4, 5917, 590, 0, 8, F64, False), (4, 20000, 10600, 0, 40, F64, True),
+    (5, 800, 770, 0, 8, F64, False), (5, 2048, 1065, 0, 24, F64, False), (5, 2048, 1536, 0, 75, F64, True),
+    (5, 5917, 2958, 0, 128, F64, True), (6, 800, 80, 0, 8, F64, False), (6, 800, 600, 0, 8, F64, True),
+    (6, 5917, 590, 0, 8, F64, True), (5, 648, 0, 152, 75, F64, True), (6, 648, 0, 152, 1, F64, True),
+    (4, 648, 0, 152, 1, F64, False), (2, 5487, 0, 430, 8, F64, False), (6, 648, 0, 152, 1, F32, False),
+    (2, 20000, 19000, 0, 1, F32, False), (3, 20000, 19000, 0, 40, F32, False), (4, 5917, 5680, 0, 8, F32, False),
+    (4, 20000, 10600, 0, 40, F32, True), (5, 2048, 1960, 0, 24, F32, False), (5, 5917, 2958, 0, 45, F32, True),
+    (6, 800, 770, 0, 8, F32, False), (6, 2048, 1065, 0, 24, F32, True), (6, 2048, 1960, 0, 75, F32, False),
+    (6, 5917, 3136, 0, 128, F32, True)])
+def test_rule_of_mixed_meshes(p, nin, npar, npml, n, mode, sf):
+    assert _lib.load().f25_selftest_route(p, nin, npar, npml, n, mode) == sf
 
 
 # parallelograms alone: (order, elements, pairs, mode, sum factorisation faster) as timed
@@ -155,7 +158,7 @@ def test_rule_of_mixed_meshes(p, nin, n, mode, sf):
     (3, 5917, 44, F32, False), (3, 11200, 23, F32, False), (3, 20000, 16, F32, True), (3, 20000, 24, F32, False),
     (4, 20000, 128, F32, True)])
 def test_rule_of_parallelograms(p, nin, n, mode, sf):
-    assert _lib.load().f25_selftest_route(p, nin, nin, n, mode) == sf
+    assert _lib.load().f25_selftest_route(p, nin, nin, 0, n, mode) == sf
 
 
 @pytest.mark.parametrize("nin,npar,n,sf", [
@@ -164,12 +167,13 @@ def test_rule_of_parallelograms(p, nin, n, mode, sf):
     (800, 80, 45, True), (480, 0, 45, False)])
 def test_rule_of_the_gradient(nin, npar, n, sf):
     for p in (2, 4, 6):
-        assert _lib.load().f25_selftest_route(p, nin, npar, n, _lib.F25_ROUTE_GRADIENT) == sf
+        assert _lib.load().f25_selftest_route(p, nin, npar, 0, n, _lib.F25_ROUTE_GRADIENT) == sf
 
 
 def test_rule_refuses_what_there_is_not():
     route = _lib.load().f25_selftest_route
-    for a in ((1, 10, 10, 1, F64), (7, 10, 10, 1, F64), (4, 10, 11, 1, F64), (4, 10, 10, 0, F64), (4, 10, 10, 1, 99)):
+    for a in ((1, 10, 10, 0, 1, F64), (7, 10, 10, 0, 1, F64), (4, 10, 11, 0, 1, F64), (4, 10, 10, -1, 1, F64),
+              (4, 10, 10, 0, 0, F64), (4, 10, 10, 0, 1, 99)):
         assert route(*a) == -1
 
 
@@ -186,7 +190,7 @@ def test_product_of_both_kinds(p, nx, nz, n, mode):
     mi = handle(nx, nz, p, 37)
     g = general(mi.mesh)
     assert 0 < np.count_nonzero(g) < g.size // 2
-    assert _lib.load().f25_selftest_route(p, g.size, int(g.size - np.count_nonzero(g)), n, mode) == 1
+    assert _lib.load().f25_selftest_route(p, g.size, int(g.size - np.count_nonzero(g)), 0, n, mode) == 1
     om, ky = batch(n)
     x = vectors(mi, n)
     if mode == F32:
@@ -211,7 +215,7 @@ def test_product_both_sides_of_the_pair_rule(p, nx, nz, n, mode):
     are known to 2e-6."""
     import torch
     mi = handle(nx, nz, p, 0)
-    sf = _lib.load().f25_selftest_route(p, nx * nz, nx * nz, n, mode)
+    sf = _lib.load().f25_selftest_route(p, nx * nz, nx * nz, 0, n, mode)
     om, ky = batch(n)
     x = vectors(mi, n)
     if mode == F32:
@@ -238,7 +242,7 @@ def test_gradient_of_both_kinds_with_pml(p):
     u, lam = cf.seeded_complex(g.ndof, batch=n, seed=1), cf.seeded_complex(g.ndof, batch=n, seed=2)
     each = [oracle.grad_exact(m, mod, g, f[b], py[b], u[b], lam[b], pml)[1] for b in range(n)]
     for k in (1, n):
-        assert _lib.load().f25_selftest_route(p, 16, 12, k, _lib.F25_ROUTE_GRADIENT) == (k > 1)
+        assert _lib.load().f25_selftest_route(p, 16, 12, 32, k, _lib.F25_ROUTE_GRADIENT) == (k > 1)
         ref, got = sum(each[:k]), mi.gradient(om[:k], ky[:k], u[:k], lam[:k])
         for c in range(3):
             assert ta.err(got[:, c], ref[:, c]) < 1e-12, (k, c)

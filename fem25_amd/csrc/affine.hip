@@ -157,8 +157,9 @@ __device__ __forceinline__ void af_first(const R *a, const R *an, const double *
 }
 
 // acc += (value J of the row of 16 lanes in cq) * op, in program order: the
-// statement order below keeps the live values within the registers, which the
-// compiler's own order of an unrolled point loop does not
+// statement order below keeps the live values within the registers up to p5
+// (at p6 all but 36 bytes a lane of them), which the compiler's own order of an
+// unrolled point loop does not
 template <int J>
 __device__ __forceinline__ void fb(double &acc, double cq, double op) {
     asm volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
@@ -436,7 +437,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // sides lie along x and z (sx = rz = 0), and T2 carries sz.
 //
 // Bound by latency at two waves per SIMD (T1, T2 of both fields are 12 NL doubles
-// a lane, 168 of the 256 registers at p6).  Measured on MI355X: 200x100 p4, 128 triples
+// a lane, 168 of the 256 registers at p6, where 12 to 16 bytes a lane spill), at
+// p6 and many triples by memory too (400x200, 192 triples: 101 GB read, each
+// value 1.9 times, 2 GB written by the spills, 22.8 ms).  Measured on MI355X: 200x100 p4, 128 triples
 // 9.30 -> 1.62 ms (FP64 pipe about half busy, 4.5 GB from HBM of 3.9 GB read
 // once); 121x59 p6, 45 triples 2.99 -> 0.56 ms.  On the way: slots numbered
 // across vectors (index arithmetic per load) 2.03 ms at p4, one column at a

@@ -672,7 +672,7 @@ extern "C" int f25_set_model(f25_mesh *m, const double *dens, const double *ecoe
     if (!m || !dens || !ecoeff) FAIL(F25_ERR_ARG, "null argument");
     HIPCHK(hipSetDevice(m->dev));
     const int n = m->d.nnpg;
-    // unchanged model: the element blocks on the device are current
+    // unchanged model: the records on the device are current, and blocks if built
     if (m->have_model && std::equal(dens, dens + n, m->rho.begin()) &&
         std::equal(ecoeff, ecoeff + n, m->lam.begin()) && std::equal(ecoeff + n, ecoeff + 2 * n, m->mu.begin()))
         return 0;
@@ -1134,9 +1134,9 @@ static int launch_apply_af(f25_mesh *m, const int *order, int n, const int *lm_i
     // lines of neighbouring chunks, and about 8,192 waves a launch, four times
     // what the chip holds, as each wave starts with the element's addresses;
     // one per chunk where there are fewer.
-    // (At least 16,384 waves, any count: 97x61, 75 pairs, p5 FP32 593 -> 521
-    // us, p4 500 -> 433, p3 304 -> 266; 48 sizes of p3..p6 1.026 times faster
-    // in the mean, 60x40, 75 pairs, p4 FP32 196 -> 212.)
+    // (Against at least 16,384 waves, any count: 97x61, 75 pairs, p5 FP32 594 ->
+    // 507 us, p4 500 -> 433, p3 304 -> 266; 112 products of p3..p6 1.026 times
+    // faster in the mean, 60x40, 75 pairs, p4 FP32 196 -> 212.)
     const int nsplit = std::min(nch, S::NW * std::max(1, (8192 / n + S::NW / 2) / S::NW));
     const int64_t nwg = ((int64_t)n * nsplit + S::NW - 1) / S::NW;
     if (nwg > 0x7fffffff) FAIL(F25_ERR_ARG, "too many pairs for one launch");

@@ -1127,7 +1127,7 @@ __global__ __launch_bounds__(256) void k_spmv(int ndof, const int64_t *__restric
 #pragma unroll
             for (int i = 0; i < 4; ++i) add(v[i], w[i]);
         }
-        // the last up to four entries of the lane, clamped loads past the end
+        // the last up to three entries of the lane, clamped loads past the end
         // (the row holds an entry if any lane gets here with one)
         if (k < e) {
             int c[3];

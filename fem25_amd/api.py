@@ -261,7 +261,8 @@ class MeshInfo:
         return rn
 
     def set_apply_tiles(self, nrt: int = 0) -> None:
-        """Row tiles per output component of the FP64 product (0: the order's default)."""
+        """Row tiles per output component of the FP64 product on element blocks, every
+        element sent there (0: the library's own choice of kernel and tiles)."""
         check(_lib.load().f25_set_apply_tiles(self.h, int(nrt)), "f25_set_apply_tiles")
 
     def apply_batch(self, omega, ky, x: np.ndarray, mode: int = _lib.F25_APPLY_F64) -> np.ndarray:
